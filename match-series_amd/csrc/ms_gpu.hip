@@ -1815,11 +1815,6 @@ int stats_impl(const void *stack, int nimg, int n, double fill, void *mean, void
 template <typename S>
 int normalize_impl(void *img, int n, int nimg, double pct, int min_to_zero, hipStream_t s) {
   const int nn = n * n;
-  void *sorted, *tmp;
-  CHK(scratch_get(81, sizeof(S) * nn, &sorted));
-  size_t tbytes = 0;
-  HIPCHK(hipcub::DeviceRadixSort::SortKeys(nullptr, tbytes, (const S *)img, (S *)sorted, nn, 0, sizeof(S) * 8, s));
-  CHK(scratch_get(82, tbytes, &tmp));
   const int m1 = nn - 1;
   int i0 = 0, i1 = m1;
   if (pct >= 0) {
@@ -1828,11 +1823,24 @@ int normalize_impl(void *img, int n, int nimg, double pct, int min_to_zero, hipS
     i0 = std::min(std::max(i0, 0), m1);
     i1 = std::min(std::max(i1, 0), m1);
   }
-  for (int k = 0; k < nimg; ++k) {
-    S *im = (S *)img + (size_t)k * nn;
-    HIPCHK(hipcub::DeviceRadixSort::SortKeys(tmp, tbytes, (const S *)im, (S *)sorted, nn, 0, sizeof(S) * 8, s));
-    hipLaunchKernelGGL((msg::k_normalize<S>), dim3(cdiv(nn, 256)), dim3(256), 0, s, im, nn, (const S *)sorted, i0, i1,
-                       pct >= 0 ? 1 : 0, min_to_zero);
+  constexpr int P = msg::SelKey<S>::PASSES;
+  const int per = std::min(nimg, 1024);  // images per sweep: bounds the counts (16 KiB per image and digit)
+  const size_t words = (size_t)P * per * 2 * msg::SEL_BINS;
+  void *hist, *st;
+  CHK(scratch_get(81, sizeof(unsigned) * words, &hist));
+  CHK(scratch_get(82, sizeof(msg::SelState) * (P + 1) * per * 2, &st));
+  for (int k0 = 0; k0 < nimg; k0 += per) {
+    const int m = std::min(per, nimg - k0);
+    S *im = (S *)img + (size_t)k0 * nn;
+    const dim3 g(cdiv(nn, msg::SEL_CHUNK), m), b(msg::SEL_THREADS);
+    const size_t w = (size_t)P * m * 2 * msg::SEL_BINS;
+    hipLaunchKernelGGL(msg::k_fill_u32, dim3((unsigned)std::min<size_t>((w + 255) / 256, 4096)), b, 0, s,
+                       (unsigned *)hist, w, 0u);
+    for (int p = 0; p < P; ++p)
+      hipLaunchKernelGGL((msg::k_sel_count<S>), g, b, 0, s, (const S *)im, nn, m, p, (unsigned)i0, (unsigned)i1,
+                         (unsigned *)hist, (msg::SelState *)st);
+    hipLaunchKernelGGL((msg::k_normalize<S>), g, b, 0, s, im, nn, m, (unsigned)i0, (unsigned)i1,
+                       (const unsigned *)hist, (const msg::SelState *)st, pct >= 0 ? 1 : 0, min_to_zero);
     HIPCHK(hipGetLastError());
   }
   return MSG_OK;

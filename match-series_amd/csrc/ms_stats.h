@@ -93,31 +93,216 @@ k_series_stats(const S *__restrict__ stack, int nimg, int nn, double fill, S *__
   }
 }
 
-// prepareMultilevelArray (registration.h:331-347) given the sorted copy of the image:
-// pct >= 0: clamp to [lo, hi], subtract the minimum (lo) and divide by the maximum (hi - lo);
-// pct < 0: subtract the minimum if negative or min_to_zero, divide by the (shifted) maximum.
+// ------------------------------------------------------------------------------------------------
+// Order statistics of images by radix selection: the two ranks prepareMultilevelArray needs of every
+// image (its percentile bounds, or its minimum and maximum), found digit by digit from histograms
+// instead of sorting the image. Keys are the values' bit patterns in increasing order (negative values
+// complemented, positive ones with the sign bit set), so the result is the element a sort would put
+// there. Pass p counts digit p of the elements that share the digits found so far, once per rank (one
+// histogram serves both ranks while their prefixes agree); the next pass, and the normalisation after the
+// last, find their rank's digit from those counts, every workgroup for itself (2048 counts from L2).
+// Bound by one read of the images per digit (3 for FP32, 6 for FP64) and, for one image, by its 5 small
+// launches. 24 frames of 1024^2 in FP32: 160 us with the copy of the frames, where one library sort
+// after another took 3.71 ms (21 launches and about 150 us per frame).
+// ------------------------------------------------------------------------------------------------
+constexpr int SEL_BITS = 11, SEL_BINS = 1 << SEL_BITS;
+constexpr int SEL_THREADS = 256, SEL_PER_THREAD = 32, SEL_CHUNK = SEL_THREADS * SEL_PER_THREAD;
+
 template <typename S>
-__global__ void k_normalize(S *__restrict__ img, int nn, const S *__restrict__ sorted, int i0, int i1, int saturate,
-                            int min_to_zero) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= nn) return;
-  double v = ld(img, j);
-  if (saturate) {
-    const double lo = ld(sorted, i0), hi = ld(sorted, i1);
-    v = v < lo ? lo : (v > hi ? hi : v);
-    v += -1 * lo;                 // addToAll(-1 * getMinValue()), the minimum being lo
-    const double mx = hi + -1 * lo;  // getMaxValue() of the shifted image
-    if (mx != 0) v /= mx;
-  } else {
-    const double mn = ld(sorted, 0), mxo = ld(sorted, nn - 1);
-    double mx = mxo;
-    if (mn < 0. || min_to_zero) {
-      v += -mn;
-      mx = mxo + -mn;
-    }
-    if (mx != 0.) v /= mx;
+struct SelKey;
+template <>
+struct SelKey<float> {
+  typedef unsigned type;
+  static constexpr int PASSES = 3;
+  __device__ static type key(float v) {
+    const unsigned u = __float_as_uint(v);
+    return u & 0x80000000u ? ~u : u | 0x80000000u;
   }
-  img[j] = static_cast<S>(v);
+  __device__ static float value(type k) { return __uint_as_float(k & 0x80000000u ? k & 0x7fffffffu : ~k); }
+};
+template <>
+struct SelKey<double> {
+  typedef unsigned long long type;
+  static constexpr int PASSES = 6;
+  __device__ static type key(double v) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    return u >> 63 ? ~u : u | (1ull << 63);
+  }
+  __device__ static double value(type k) {
+    return __longlong_as_double((long long)(k >> 63 ? k & ~(1ull << 63) : ~k));
+  }
+};
+// right shift of digit p (the last digit holds the bits left over)
+template <typename S>
+__device__ __forceinline__ int sel_shift(int p) {
+  const int s = (int)sizeof(S) * 8 - SEL_BITS * (p + 1);
+  return s > 0 ? s : 0;
+}
+
+// What is known of a rank before a pass: the digits found so far and the rank among the elements that
+// share them.
+struct SelState {
+  unsigned long long prefix;
+  unsigned rank, pad;
+};
+
+// The digit that holds `rank` in counts h[SEL_BINS] and the rank within it, for every thread of the
+// workgroup. tmp: 4 + 2 words of LDS.
+__device__ __forceinline__ void sel_digit(const unsigned *__restrict__ h, unsigned rank, unsigned *tmp,
+                                          unsigned &digit, unsigned &rest) {
+  constexpr int PER = SEL_BINS / SEL_THREADS;
+  unsigned c[PER], mine = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    c[k] = h[threadIdx.x * PER + k];
+    mine += c[k];
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  unsigned inc = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned v = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += v;
+  }
+  __syncthreads();  // earlier reads of tmp are done
+  if (lane == 63) tmp[wid] = inc;
+  __syncthreads();
+  unsigned below = inc - mine;
+  for (int w = 0; w < wid; ++w) below += tmp[w];
+  if (rank >= below && rank - below < mine) {  // exactly one thread: the counts add up to more than rank
+    unsigned r = rank - below;
+    int k = 0;
+#pragma unroll
+    for (int j = 0; j < PER - 1; ++j)
+      if (k == j && r >= c[j]) {
+        r -= c[j];
+        ++k;
+      }
+    tmp[4] = threadIdx.x * PER + k;
+    tmp[5] = r;
+  }
+  __syncthreads();
+  digit = tmp[4];
+  rest = tmp[5];
+}
+
+// State of both ranks of image `img` before digit p, from the state before digit p - 1 and that digit's
+// counts (layout [pass][image][rank][SEL_BINS], rank 1's unused where the prefixes agreed).
+template <typename S>
+__device__ __forceinline__ void sel_advance(const unsigned *__restrict__ hist, const SelState *__restrict__ st, int img,
+                                            int nimg, int p, unsigned rank0, unsigned rank1, unsigned *tmp,
+                                            SelState (&s)[2]) {
+  if (p == 0) {
+    s[0] = {0, rank0, 0};
+    s[1] = {0, rank1, 0};
+    return;
+  }
+  SelState q[2];
+  if (p == 1) {
+    q[0] = {0, rank0, 0};
+    q[1] = {0, rank1, 0};
+  } else {
+    q[0] = st[((size_t)(p - 1) * nimg + img) * 2];
+    q[1] = st[((size_t)(p - 1) * nimg + img) * 2 + 1];
+  }
+  const int bits = sel_shift<S>(p - 2) - sel_shift<S>(p - 1);  // width of digit p - 1 (p == 1: see below)
+  const int w = p == 1 ? SEL_BITS : bits;
+  const bool same = q[0].prefix == q[1].prefix;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const unsigned *h = hist + (((size_t)(p - 1) * nimg + img) * 2 + (same ? 0 : r)) * SEL_BINS;
+    unsigned d, rest;
+    sel_digit(h, q[r].rank, tmp, d, rest);
+    s[r] = {(q[r].prefix << w) | d, rest, 0};
+  }
+}
+
+// Counts of digit p. Grid (chunks of SEL_CHUNK elements, images).
+template <typename S>
+__global__ void __launch_bounds__(SEL_THREADS)
+k_sel_count(const S *__restrict__ imgs, int nn, int nimg, int p, unsigned rank0, unsigned rank1,
+            unsigned *__restrict__ hist, SelState *__restrict__ st) {
+  typedef typename SelKey<S>::type K;
+  __shared__ unsigned h[2][SEL_BINS];
+  __shared__ unsigned tmp[6];
+  const int img = blockIdx.y;
+  const S *im = imgs + (size_t)img * nn;
+  SelState s[2];
+  sel_advance<S>(hist, st, img, nimg, p, rank0, rank1, tmp, s);
+  if (p > 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+    st[((size_t)p * nimg + img) * 2] = s[0];
+    st[((size_t)p * nimg + img) * 2 + 1] = s[1];
+  }
+  const bool two = s[0].prefix != s[1].prefix;
+  for (int i = threadIdx.x; i < SEL_BINS; i += SEL_THREADS) h[0][i] = h[1][i] = 0;
+  __syncthreads();
+  const int shift = sel_shift<S>(p);
+  const int top = p == 0 ? 0 : sel_shift<S>(p - 1);  // bits below the prefix
+  const unsigned mask = p == 0 ? SEL_BINS - 1 : (unsigned)((1u << (top - shift)) - 1u);
+  const K p0 = (K)s[0].prefix, p1 = (K)s[1].prefix;
+  const int i0 = blockIdx.x * SEL_CHUNK + threadIdx.x;
+  constexpr int RUN = 8;  // loads in flight per thread
+  for (int k = 0; k < SEL_PER_THREAD; k += RUN) {
+    S v[RUN];
+#pragma unroll
+    for (int r = 0; r < RUN; ++r) {
+      const int i = i0 + (k + r) * SEL_THREADS;
+      v[r] = im[i < nn ? i : nn - 1];
+    }
+#pragma unroll
+    for (int r = 0; r < RUN; ++r) {
+      if (i0 + (k + r) * SEL_THREADS < nn) {
+        const K key = SelKey<S>::key(v[r]);
+        const unsigned d = (unsigned)(key >> shift) & mask;
+        if (p == 0 || (key >> top) == p0) atomicAdd(&h[0][d], 1u);
+        if (two && (key >> top) == p1) atomicAdd(&h[1][d], 1u);
+      }
+    }
+  }
+  __syncthreads();
+  unsigned *g = hist + ((size_t)p * nimg + img) * 2 * SEL_BINS;
+  for (int i = threadIdx.x; i < SEL_BINS; i += SEL_THREADS) {
+    if (h[0][i]) atomicAdd(g + i, h[0][i]);
+    if (two && h[1][i]) atomicAdd(g + SEL_BINS + i, h[1][i]);
+  }
+}
+
+// prepareMultilevelArray (registration.h:331-347) with the image's elements of rank0 and rank1:
+// saturate: clamp to [lo, hi], subtract the minimum (lo) and divide by the maximum (hi - lo);
+// otherwise lo, hi are the extrema: subtract the minimum if negative or min_to_zero, divide by the
+// (shifted) maximum. Grid as k_sel_count.
+template <typename S>
+__global__ void __launch_bounds__(SEL_THREADS)
+k_normalize(S *__restrict__ imgs, int nn, int nimg, unsigned rank0, unsigned rank1, const unsigned *__restrict__ hist,
+            const SelState *__restrict__ st, int saturate, int min_to_zero) {
+  typedef typename SelKey<S>::type K;
+  __shared__ unsigned tmp[6];
+  const int img = blockIdx.y;
+  SelState s[2];
+  sel_advance<S>(hist, st, img, nimg, SelKey<S>::PASSES, rank0, rank1, tmp, s);
+  const double lo = (double)SelKey<S>::value((K)s[0].prefix), hi = (double)SelKey<S>::value((K)s[1].prefix);
+  const bool shifted = saturate || lo < 0. || min_to_zero;
+  const double mx = shifted ? hi + -1 * lo : hi;  // getMaxValue() of the shifted image
+  S *im = imgs + (size_t)img * nn;
+  const int i0 = blockIdx.x * SEL_CHUNK + threadIdx.x;
+  constexpr int RUN = 8;
+  for (int k = 0; k < SEL_PER_THREAD; k += RUN) {
+    S in[RUN];
+#pragma unroll
+    for (int r = 0; r < RUN; ++r) {
+      const int i = i0 + (k + r) * SEL_THREADS;
+      in[r] = im[i < nn ? i : nn - 1];
+    }
+#pragma unroll
+    for (int r = 0; r < RUN; ++r) {
+      const int i = i0 + (k + r) * SEL_THREADS;
+      double v = (double)in[r];
+      if (saturate) v = v < lo ? lo : (v > hi ? hi : v);
+      if (shifted) v += -1 * lo;  // addToAll(-1 * getMinValue())
+      if (mx != 0) v /= mx;
+      if (i < nn) im[i] = static_cast<S>(v);
+    }
+  }
 }
 
 }  // namespace msg
