@@ -1799,6 +1799,17 @@ int compose_impl(const void *phi1, const void *phi2, void *result, int n, hipStr
 template <typename S>
 int stats_impl(const void *stack, int nimg, int n, double fill, void *mean, void *count, void *median, hipStream_t s) {
   const int nn = n * n;
+  // up to 64 frames: samples sorted in registers, padded to 8, 16, 32 or 64
+  if (nimg <= msg::ST_SORT_MAX) {
+    const dim3 g(cdiv(nn, 256)), b(256);
+    const S *st = (const S *)stack;
+    if (nimg <= 8) hipLaunchKernelGGL((msg::k_series_stats_sort<S, 8>), g, b, 0, s, st, nimg, nn, fill, (S *)mean, (S *)count, (S *)median);
+    else if (nimg <= 16) hipLaunchKernelGGL((msg::k_series_stats_sort<S, 16>), g, b, 0, s, st, nimg, nn, fill, (S *)mean, (S *)count, (S *)median);
+    else if (nimg <= 32) hipLaunchKernelGGL((msg::k_series_stats_sort<S, 32>), g, b, 0, s, st, nimg, nn, fill, (S *)mean, (S *)count, (S *)median);
+    else hipLaunchKernelGGL((msg::k_series_stats_sort<S, 64>), g, b, 0, s, st, nimg, nn, fill, (S *)mean, (S *)count, (S *)median);
+    HIPCHK(hipGetLastError());
+    return MSG_OK;
+  }
   const int P = msg::stats_pixels_per_wave(nimg);
   if (P == 0) return fail(MSG_ERR_ARG, "series longer than 8192 frames are not supported by the median kernel");
   const size_t lds = sizeof(double) * P * std::max(nimg, 1);

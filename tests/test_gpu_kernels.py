@@ -58,3 +58,36 @@ def test_normalize_ranks(gpu, n, frames, code):
                         v, top = v - lo, top - lo
                 want = (v / top if top != 0 else v).astype(np_dt)
             assert np.array_equal(out[k], want, equal_nan=True), (k, pct, zero)
+
+
+@pytest.mark.parametrize("frames", [1, 7, 8, 9, 16, 17, 31, 32, 33, 63, 64, 65])
+@pytest.mark.parametrize("code", [0, 1])
+def test_series_stats_networks(gpu, frames, code):
+    """Every length around the sorting networks' sizes and the counting kernel beyond them, on a pixel
+    count that is no multiple of a workgroup: ties, missing samples, -Inf; the statistics are selections
+    and one FP64 sum in frame order, so count and median are exact."""
+    n = 16 if frames != 33 else 8
+    rng = np.random.default_rng(100 + frames)
+    dt = gpu.torch_dtype(code)
+    st = rng.normal(size=(frames, n, n))
+    st = np.round(st * 4) / 4 if frames % 3 == 0 else st
+    st[rng.random(st.shape) < 0.25] = np.inf
+    st[:, 0, 0] = np.inf
+    st[frames // 2, 1, 1] = -np.inf
+    st = st.astype(np.float64 if code else np.float32)
+    t = torch.tensor(st, device="cuda")
+    mean, count, med = (host(x) for x in gpu.series_stats(t, 0.375))
+    have = st != np.inf
+    c = have.sum(0)
+    assert np.array_equal(count, c)
+    s = np.sort(st.astype(np.float64), axis=0)
+    for y in range(n):
+        for x in range(n):
+            k = c[y, x]
+            want = 0.375 if k == 0 else (s[k // 2, y, x] if k % 2 else (s[k // 2 - 1, y, x] + s[k // 2, y, x]) / 2)
+            assert med[y, x] == (want if code else np.float64(np.float32(want)))
+            acc = 0.0
+            for f in range(frames):
+                acc += float(st[f, y, x]) if have[f, y, x] else 0.0
+            want = acc / k if k else 0.375
+            assert mean[y, x] == (want if code else np.float64(np.float32(want)))
