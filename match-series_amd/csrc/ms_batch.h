@@ -273,15 +273,11 @@ int batch_group(const std::vector<const msg_series_job *> &jobs, int slot) {
       for (int i = 0; i < n; ++i) {
         double ext = 0;
         CHK(mean_value<S>(t + (size_t)i * nn, (int)nn, &ext, s));
-        hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, t + (size_t)i * nn,
-                           defs + (size_t)i * 2 * nn, (S *)stack.p + (size_t)i * nn, N, 1, 0, 0, ext, nearest);
-        HIPCHK(hipGetLastError());
+        CHK(launch_warp<S>(t + (size_t)i * nn, defs + (size_t)i * 2 * nn, (S *)stack.p + (size_t)i * nn, N, 1, 0, 0,
+                           ext, nearest, s));
       }
     } else {
-      const size_t cnt = nn * n;
-      hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, t, defs,
-                         (S *)stack.p, N, n, 0, 0, (double)INFINITY, nearest);
-      HIPCHK(hipGetLastError());
+      CHK(launch_warp<S>(t, defs, (S *)stack.p, N, n, 0, 0, (double)INFINITY, nearest, s));
     }
     double fill = 0;
     CHK(mean_value<S>(t + (size_t)(n - 1) * nn, (int)nn, &fill, s));

@@ -185,6 +185,15 @@ __device__ __forceinline__ double interp_wh(const S *__restrict__ img, int w, in
   return (1 - X) * (1 - Y) * v0 + X * (1 - Y) * v1 + (1 - X) * Y * v2 + X * Y * v3;
 }
 
+// One axis of interp_wh: lower node (in [0, w-2]) and the coordinate relative to it.
+__device__ __forceinline__ void interp_cell(double X, int w, int &lo, double &rel) {
+  if (X != X) X = 0.;
+  lo = (int)X;
+  if (X >= (double)(w - 1)) lo = w - 2;
+  if (X < 0.) lo = 0;
+  rel = X - lo;
+}
+
 template <typename S>
 __device__ __forceinline__ double interp(const S *__restrict__ img, int n, double X, double Y) {
   return interp_wh(img, n, n, X, Y);

@@ -491,6 +491,23 @@ int launch_prolong(const S *coarse, S *fine, int nc, int nfields, hipStream_t s)
   return MSG_OK;
 }
 
+// Warps of nimg n x n images (n a power of two); see k_warp.
+template <typename S>
+int launch_warp(const S *img, const S *phi, S *out, int n, int nimg, int phi_shared, int mode, double ext, int nearest,
+                hipStream_t s) {
+  const int nblk = cdiv(n * n, 256 * msg::WARP_RUN);
+  const size_t nn = (size_t)n * n;
+  const int per = std::max(1, (1 << 23) / nblk);  // images a launch: a grid of at most 2^31 threads
+  for (int i = 0; i < nimg; i += per) {
+    const int m = std::min(per, nimg - i);
+    hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)nblk * m), dim3(256), 0, s, img + i * nn,
+                       phi + (phi_shared ? 0 : i * 2 * nn), out + i * nn, n, log2i(n), nblk, phi_shared, mode, ext,
+                       nearest);
+    HIPCHK(hipGetLastError());
+  }
+  return MSG_OK;
+}
+
 // Sampling positions k * (nc-1)/(n-1) of ResampleCopier (scalarArray.h:311-330): the step divided in
 // double and held in long double, each product rounded to double.
 int resample_coords(int nc, int n, double **dcoord, hipStream_t s) {
@@ -1650,15 +1667,12 @@ int msg_warp(int dtype, const void *img, const void *phi, void *out, int n, int 
   CHK(check_dtype(dtype));
   CHK(check_n(n));
   if (!img || !phi || !out || nimg < 1 || mode < 0 || mode > 2) return fail(MSG_ERR_ARG, "invalid argument");
-  const size_t cnt = (size_t)n * n * nimg;
-  const dim3 grid((unsigned)((cnt + 255) / 256));
   if (dtype == MSG_F64)
-    hipLaunchKernelGGL((msg::k_warp<double>), grid, dim3(256), 0, strm(stream), (const double *)img,
-                       (const double *)phi, (double *)out, n, nimg, phi_shared, mode, ext, nearest);
+    CHK(launch_warp<double>((const double *)img, (const double *)phi, (double *)out, n, nimg, phi_shared, mode, ext,
+                            nearest, strm(stream)));
   else
-    hipLaunchKernelGGL((msg::k_warp<float>), grid, dim3(256), 0, strm(stream), (const float *)img, (const float *)phi,
-                       (float *)out, n, nimg, phi_shared, mode, ext, nearest);
-  HIPCHK(hipGetLastError());
+    CHK(launch_warp<float>((const float *)img, (const float *)phi, (float *)out, n, nimg, phi_shared, mode, ext,
+                           nearest, strm(stream)));
   HIPCHK(hipStreamSynchronize(strm(stream)));
   return MSG_OK;
 }
@@ -2266,9 +2280,7 @@ int pairwise_batch(const msg_series_params *p, const msg_solve_params &sp, const
       DevBuf w;
       HIPCHK(hipMalloc(&w.p, sizeof(S) * nn * nb));
       const size_t c = nn * nb;
-      hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)((c + 255) / 256)), dim3(256), 0, s, (const S *)pc->T[L],
-                         (const S *)pc->phi[L], (S *)w.p, N, nb, 0, 0, (double)INFINITY, 0);
-      HIPCHK(hipGetLastError());
+      CHK(launch_warp<S>((const S *)pc->T[L], (const S *)pc->phi[L], (S *)w.p, N, nb, 0, 0, (double)INFINITY, 0, s));
       std::vector<S> h(c);
       HIPCHK(hipMemcpyAsync(h.data(), w.p, sizeof(S) * c, hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));
@@ -2571,10 +2583,7 @@ int match_series_impl(const msg_series_params *p, const void *templates, int n, 
     HIPCHK(hipStreamSynchronize(s));
     CHK(reduce_impl<S>(defs, n, L, p->reduce_max_iter, p->reduce_stop_eps, rp, nullptr, nullptr));
     HIPCHK(hipMalloc(&pre.p, sizeof(S) * nn * n));
-    const size_t cnt = nn * n;
-    hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, raw, (const S *)rp,
-                       (S *)pre.p, N, n, 1, 0, (double)INFINITY, 0);
-    HIPCHK(hipGetLastError());
+    CHK(launch_warp<S>(raw, (const S *)rp, (S *)pre.p, N, n, 1, 0, (double)INFINITY, 0, s));
     src = (const S *)pre.p;
   }
   // averageSeries (matchSeries.h:353-451): DeformImage of each template, +Inf (no sample) or the
@@ -2584,15 +2593,11 @@ int match_series_impl(const msg_series_params *p, const void *templates, int n, 
     for (int i = 0; i < n; ++i) {
       double ext = 0;
       CHK(mean_value<S>(src + (size_t)i * nn, (int)nn, &ext, s));
-      hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, src + (size_t)i * nn,
-                         (const S *)defs + (size_t)i * 2 * nn, (S *)stack.p + (size_t)i * nn, N, 1, 0, 0, ext, nearest);
-      HIPCHK(hipGetLastError());
+      CHK(launch_warp<S>(src + (size_t)i * nn, (const S *)defs + (size_t)i * 2 * nn, (S *)stack.p + (size_t)i * nn, N,
+                         1, 0, 0, ext, nearest, s));
     }
   } else {
-    const size_t cnt = nn * n;
-    hipLaunchKernelGGL((msg::k_warp<S>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, src, (const S *)defs,
-                       (S *)stack.p, N, n, 0, 0, (double)INFINITY, nearest);
-    HIPCHK(hipGetLastError());
+    CHK(launch_warp<S>(src, (const S *)defs, (S *)stack.p, N, n, 0, 0, (double)INFINITY, nearest, s));
   }
   double fill = 0;
   CHK(mean_value<S>(raw + (size_t)(n - 1) * nn, (int)nn, &fill, s));

@@ -1491,38 +1491,71 @@ __global__ void k_resample_rect(const S *__restrict__ src, int w, int h, S *__re
 
 // DeformImage (deformations.h:62-101; ExtendWithConstant, optional nearest-neighbour rounding),
 // FastDeformImage (L140-162; clamp) and the NaN-extended variant of L226-256 (mode 2).
-// img: nimg images; phi: one field per image (or one shared field if phi_shared).
+// img: nimg images; phi: one field per image (or one shared field if phi_shared). n is a power of two,
+// logn its logarithm. Bound by HBM (phi, the image and the result once, 16 B per FP32 pixel). A workgroup
+// takes WARP_RUN x 256 pixels of one image: coordinates by shifts, and a thread's WARP_RUN pixels step by
+// step together, displacements, then the 4 neighbours each, so a wave waits for two memory round trips in
+// WARP_RUN pixels. Pixels outside gather from clamped nodes and are replaced by a select (no branches).
+// 31 frames of 1024^2 in FP32: 192 -> 118 us (4.5 TB/s) against one pixel per thread with 64-bit index
+// divisions.
+constexpr int WARP_RUN = 4;
+
 template <typename S>
-__global__ void k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out, int n, int nimg,
-                       int phi_shared, int mode, double ext, int nearest) {
-  const size_t cnt = (size_t)n * n;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= cnt * nimg) return;
-  const int f = (int)(i / cnt);
-  const int j = (int)(i - (size_t)f * cnt);
-  const int x = j % n, y = j / n;
+__global__ void __launch_bounds__(256)
+k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out, int n, int logn, int nblk,
+       int phi_shared, int mode, double ext, int nearest) {
+  const int f = blockIdx.x / nblk;
+  const int cnt = n * n;
+  const int j0 = (blockIdx.x - f * nblk) * (256 * WARP_RUN) + threadIdx.x;
   const double h = 1.0 / (double)(n - 1);
   const S *ph = phi + (phi_shared ? 0 : (size_t)f * 2 * cnt);
-  double dx = x + ld(ph, j) / h, dy = y + ld(ph, cnt + j) / h;
   const S *im = img + (size_t)f * cnt;
-  double v;
-  if (mode == 1) {  // clamp
-    const double hi = (double)(n - 1);
-    dx = dx < 0 ? 0 : (dx > hi ? hi : dx);
-    dy = dy < 0 ? 0 : (dy > hi ? hi : dy);
-    v = interp(im, n, dx, dy);
-  } else {
-    bool inside = true;
-    const double hi = (double)(n - 1);
-    if (dx < 0.0 || dx > hi || (mode == 0 && isnan(dx))) inside = false;
-    if (dy < 0.0 || dy > hi || (mode == 0 && isnan(dy))) inside = false;
-    if (nearest && mode == 0) {
-      dx = floor(dx + 0.5);
-      dy = floor(dy + 0.5);
-    }
-    v = inside ? interp(im, n, dx, dy) : (mode == 2 ? __builtin_nan("") : ext);
+  S *o = out + (size_t)f * cnt;
+  const double hi = (double)(n - 1);
+  S p0[WARP_RUN], p1[WARP_RUN];
+#pragma unroll
+  for (int k = 0; k < WARP_RUN; ++k) {
+    const int j = min(j0 + 256 * k, cnt - 1);
+    p0[k] = ph[j];
+    p1[k] = ph[(size_t)cnt + j];
   }
-  out[i] = static_cast<S>(v);
+  double X[WARP_RUN], Y[WARP_RUN];
+  S v[WARP_RUN][4];
+  bool inside[WARP_RUN];
+#pragma unroll
+  for (int k = 0; k < WARP_RUN; ++k) {
+    const int j = min(j0 + 256 * k, cnt - 1);
+    const int x = j & (n - 1), y = j >> logn;
+    double dx = x + (double)p0[k] / h, dy = y + (double)p1[k] / h;
+    inside[k] = true;
+    if (mode == 1) {  // clamp
+      dx = dx < 0 ? 0 : (dx > hi ? hi : dx);
+      dy = dy < 0 ? 0 : (dy > hi ? hi : dy);
+    } else {
+      if (dx < 0.0 || dx > hi || (mode == 0 && isnan(dx))) inside[k] = false;
+      if (dy < 0.0 || dy > hi || (mode == 0 && isnan(dy))) inside[k] = false;
+      if (nearest && mode == 0) {
+        dx = floor(dx + 0.5);
+        dy = floor(dy + 0.5);
+      }
+    }
+    int xL, yL;  // ScalarArray<QC_2D>::interpolate as interp(), inside the image for every input
+    interp_cell(dx, n, xL, X[k]);
+    interp_cell(dy, n, yL, Y[k]);
+    const S *c = im + xL + (size_t)yL * n;
+    v[k][0] = c[0];
+    v[k][1] = c[1];
+    v[k][2] = c[n];
+    v[k][3] = c[n + 1];
+  }
+#pragma unroll
+  for (int k = 0; k < WARP_RUN; ++k) {
+    const double v0 = v[k][0], v1 = v[k][1], v2 = v[k][2], v3 = v[k][3];
+    const double r0 = (1 - X[k]) * v0 + X[k] * v1;
+    const double r1 = (1 - X[k]) * (1 - Y[k]) * v0 + X[k] * (1 - Y[k]) * v1 + (1 - X[k]) * Y[k] * v2 + X[k] * Y[k] * v3;
+    const double r = inside[k] ? (Y[k] == 0 ? r0 : r1) : (mode == 2 ? __builtin_nan("") : ext);
+    if (j0 + 256 * k < cnt) o[j0 + 256 * k] = static_cast<S>(r);
+  }
 }
 
 }  // namespace msg

@@ -91,3 +91,45 @@ def test_series_stats_networks(gpu, frames, code):
                 acc += float(st[f, y, x]) if have[f, y, x] else 0.0
             want = acc / k if k else 0.375
             assert mean[y, x] == (want if code else np.float64(np.float32(want)))
+
+
+@pytest.mark.parametrize("n,count", [(2, 3), (16, 2), (32, 1), (64, 3)])
+@pytest.mark.parametrize("code", [0, 1])
+def test_warp_modes(gpu, n, count, code):
+    """Images below, at and above one workgroup's pixels, every mode, one field per image and one
+    shared, displacements that leave the grid, land on its border and are not finite. The kernel's FP64
+    operations are repeated in their order: exact up to the rounding to the storage type."""
+    rng = np.random.default_rng(n)
+    np_dt = np.float64 if code else np.float32
+    dt = gpu.torch_dtype(code)
+    img = rng.normal(size=(count, n, n)).astype(np_dt)
+    phi = (rng.normal(size=(count, 2, n, n)) * 3 / (n - 1)).astype(np_dt)
+    phi[:, :, 0, :] = 0
+    phi[0, 0, 1, 0], phi[0, 1, 1, 1], phi[0, 0, 0, 1] = np.inf, -np.inf, np.nan
+    h, hi = 1.0 / (n - 1), float(n - 1)
+    yy, xx = np.mgrid[0:n, 0:n]
+    for shared in (False, True):
+        p = phi[0] if shared else phi
+        for mode, nearest in ((0, False), (0, True), (1, False), (2, False)):
+            got = gpu.warp(dev(img, dt), dev(p, dt), mode, 0.75, nearest).cpu().numpy()
+            for k in range(count):
+                f = (p if shared else p[k]).astype(np.float64)
+                with np.errstate(invalid="ignore"):
+                    X, Y = xx + f[0] / h, yy + f[1] / h
+                    if mode == 1:
+                        X, Y = (np.where(c < 0, 0, np.where(c > hi, hi, c)) for c in (X, Y))
+                        inside = np.ones((n, n), bool)
+                    else:
+                        inside = ~((X < 0) | (X > hi) | (Y < 0) | (Y > hi))
+                        if mode == 0:
+                            inside &= ~(np.isnan(X) | np.isnan(Y))
+                        if nearest:
+                            X, Y = np.floor(X + 0.5), np.floor(Y + 0.5)
+                    X, Y = np.where(np.isnan(X), 0, X), np.where(np.isnan(Y), 0, Y)
+                    i, j = (np.clip(np.trunc(np.clip(c, -1, n)), 0, n - 2).astype(int) for c in (X, Y))
+                    X, Y = X - i, Y - j
+                    v = [img[k][b, a].astype(np.float64) for b in (j, j + 1) for a in (i, i + 1)]
+                    r0 = (1 - X) * v[0] + X * v[1]
+                    r1 = (1 - X) * (1 - Y) * v[0] + X * (1 - Y) * v[1] + (1 - X) * Y * v[2] + X * Y * v[3]
+                    want = np.where(inside, np.where(Y == 0, r0, r1), np.nan if mode == 2 else 0.75).astype(np_dt)
+                assert np.array_equal(got[k], want, equal_nan=True), (shared, mode, nearest, k)
