@@ -310,8 +310,10 @@ k_energy_exact_f32(const float *__restrict__ R, const float *__restrict__ T, con
                    const float *__restrict__ z, const float *__restrict__ dold, int n, double h, int width,
                    const PairState *st, double *__restrict__ part, int ntx, int nty, int npairs) {
   const int tiles = ntx * nty;
+  constexpr int NC = 2;  // plan_exact: the step, and 0 for the current position
   const size_t nn = (size_t)n * n;
   const int run = en32_run(n);
+  const Div hd = make_div(h);
   for (int pair = 0; pair < npairs; ++pair) {
     if (!st[pair].exact || st[pair].ncand == 0) continue;  // uniform across the workgroup
     const float *Rp = R + pair * nn, *Tp = T + pair * nn;
@@ -320,14 +322,14 @@ k_energy_exact_f32(const float *__restrict__ R, const float *__restrict__ T, con
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
       const int ex = (tile % ntx) * EN_TX + (threadIdx.x % EN_TX);
       const int ey0 = (tile / ntx) * (4 * run) + (threadIdx.x / EN_TX) * run;
-      double accS[MAX_CAND], accR[MAX_CAND];
+      double acc[2 * NC];
 #pragma unroll
-      for (int k = 0; k < MAX_CAND; ++k) accS[k] = accR[k] = 0.0;
+      for (int k = 0; k < 2 * NC; ++k) acc[k] = 0.0;
       if (ex < n - 1)
         for (int j = 0; j < run; ++j)
           if (ey0 + j < n - 1)
-            energy_elem<float>(Rp, Tp, px, py, zx, zy, ox_, oy_, n, h, width, st[pair], ex, ey0 + j, accS, accR);
-      energy_write_partials(accS, accR, st[pair].ncand, part, pair, tile, tiles);
+            energy_elem<float, NC>(Rp, Tp, px, py, zx, zy, ox_, oy_, n, hd, width, st[pair], ex, ey0 + j, acc);
+      energy_write_partials<NC>(acc, st[pair].ncand, part, pair, tile, tiles);
     }
   }
 }
@@ -346,8 +348,9 @@ k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float
   if (st && !participates(st[pair])) return;
   const double lambda6 = (st ? st[pair].lambda : lambda_default) * (1.0 / 6.0);
 
-  __shared__ float cf[GR_EY * GR_EX][4][2];  // force contribution per element, dof, component
-  __shared__ float ck[GR_EY * GR_EX][4][2];  // stiffness contribution
+  // per dof, component and element (consecutive lanes, consecutive elements: no bank conflicts)
+  __shared__ float cf[4][2][GR_NE];  // force contribution
+  __shared__ float ck[4][2][GR_NE];  // stiffness contribution
 
   const size_t nn = (size_t)n * n;
   const float *Rp = R + pair * nn, *Tp = T + pair * nn;
@@ -393,8 +396,8 @@ k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float
         a0 += bqf(dof, q) * nl[q][0];
         a1 += bqf(dof, q) * nl[q][1];
       }
-      cf[e][dof][0] = wv * a0;
-      cf[e][dof][1] = wv * a1;
+      cf[dof][0][e] = wv * a0;
+      cf[dof][1][e] = wv * a1;
     }
     // 6 K_loc = [4 -1 -1 -2; -1 4 -2 -1; -1 -2 4 -1; -2 -1 -1 4] applied to the element's dofs. Its
     // rows sum to zero, so row i is sum over j != i of K_ij (f_j - f_i): differences of close values
@@ -411,8 +414,8 @@ k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float
         s0 += kl[i][j] * (f0[j] - f0[i]);
         s1 += kl[i][j] * (f1[j] - f1[i]);
       }
-      ck[e][i][0] = s0;
-      ck[e][i][1] = s1;
+      ck[i][0][e] = s0;
+      ck[i][1][e] = s1;
     }
   }
   __syncthreads();
@@ -426,10 +429,10 @@ k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float
       if (ex < 0 || ey < 0 || ex >= n - 1 || ey >= n - 1) continue;
       const int e = (ex - (x0 - 1)) + (ey - (y0 - 1)) * GR_EX;
       const int dof = (x - ex) + 2 * (y - ey);
-      F0 += cf[e][dof][0];
-      F1 += cf[e][dof][1];
-      K0 += ck[e][dof][0];
-      K1 += ck[e][dof][1];
+      F0 += cf[dof][0][e];
+      F1 += cf[dof][1][e];
+      K0 += ck[dof][0][e];
+      K1 += ck[dof][1][e];
     }
   float *o = DE + pair * 2 * nn;
   const int i = x + y * n;
@@ -670,6 +673,15 @@ k_mg_coarse_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x
   const double tau = 0.5 * (sigma * sigma);
   __shared__ float X[MGC_OFF[MGC_MAXL_F32 + 1]], B[MGC_OFF[MGC_MAXL_F32 + 1]], Y[1 << (2 * MGC_MAXL_F32)];
   __shared__ double red[(MGC_THREADS / 64) * NORM_TERMS];
+  // the levels' constants, formed once while the right-hand side loads (a division in FP64 on the chain
+  // of every level and leg otherwise)
+  __shared__ float lhs[MGC_MAXL_F32 + 1], lidg[MGC_MAXL_F32 + 1];
+  if ((int)threadIdx.x <= L) {
+    const int m = 1 << threadIdx.x;
+    const double s = (double)((m - 1) * (m - 1));
+    lhs[threadIdx.x] = (float)(tau * s);
+    lidg[threadIdx.x] = (float)(1.0 / (1 + 4 * tau * s));
+  }
   const int n = 1 << L;
   const size_t nn = (size_t)n * n;
   const float *rp = rhs + field * nn;
@@ -688,10 +700,8 @@ k_mg_coarse_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x
   __syncthreads();
 
   auto consts = [&](int l, float &hs, float &idg) {
-    const int m = 1 << l;
-    const double s = (double)((m - 1) * (m - 1));
-    hs = (float)(tau * s);
-    idg = (float)(1.0 / (1 + 4 * tau * s));
+    hs = lhs[l];
+    idg = lidg[l];
   };
 
   // Down leg of level l with nthr threads (thread tid): two Jacobi sweeps from zero, the second kept
