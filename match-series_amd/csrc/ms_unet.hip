@@ -9,7 +9,7 @@
 //
 // Layout: activations NHWC in BF16 (channels innermost, so a convolution's reduction dimension is
 // contiguous); gradients of activations NHWC in FP32; weights FP32 masters [9][Cout][Cin] with BF16
-// copies in the forward layout [tap][Cout][Cin] and the data-gradient layout [tap][Cin][Cout].
+// copies packed for the forward and for the data gradient (k_weights_bf16).
 // A 3x3 convolution is an implicit GEMM on MFMA (v_mfma_f32_32x32x16_bf16): rows = output channels
 // (weights), columns = 32 consecutive pixels, reduction = 9 taps x input channels in steps of 16;
 // FP32 accumulation, bias and ReLU fused into the epilogue. The upsampling and the concatenation are
@@ -51,6 +51,8 @@ typedef unsigned short bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // FP32 -> BF16, round to nearest even (NaN stays NaN)
 __host__ __device__ inline bf16 f2bf(float f) {
@@ -70,6 +72,13 @@ __device__ inline bf16x8 as_bf16x8(u16x8 v) { return __builtin_bit_cast(bf16x8, 
 
 inline int cdivu(long a, long b) { return (int)((a + b - 1) / b); }
 
+// Workgroup ids in an order that gives each of the 8 XCDs a contiguous range (ids are dispatched
+// round-robin over them): neighbouring tiles and the channel blocks of one tile share an L2.
+__device__ inline int xcd_order(int wg, int total) {
+  const int xcd = wg % 8, base = total / 8, extra = total % 8;
+  return xcd * base + (xcd < extra ? xcd : extra) + wg / 8;
+}
+
 // The input of a convolution at H x W: channels [0, c1) from x1 (H/2 x W/2 and upsampled when up1),
 // channels [c1, c1 + c2) from x2 (H x W). c1 and c2 are multiples of 16 (c2 may be 0).
 struct ConvIn {
@@ -79,27 +88,70 @@ struct ConvIn {
 };
 
 // ------------------------------------------------------------------------------------------------
-// 3x3 convolution, forward (or data gradient with flip = 1 and the transposed weights):
-// y[p][co] = act(bias[co] + sum_tap sum_ci w[tap'][co][ci] in[p + off(tap)][ci]), tap' = tap or 8 - tap.
-// One wave: 32 output channels x NT times and 32 x NP consecutive pixels of one image row (W % (32 NP)
-// == 0); four waves per workgroup along the pixels. A weight operand loaded for an MFMA serves the NP
-// pixel tiles, an input operand the NT channel tiles. Output FP32 or BF16, NHWC with `cout` channels.
+// 3x3 convolution, forward (or data gradient, with its own packed weights):
+// y[p][co] = act(bias[co] + sum_tap sum_ci w[tap][co][ci] in[p + off(tap)][ci]).
+//
+// A workgroup of four waves computes 32 columns x 4 NP rows of one image and 32 NT output channels; a wave
+// NP rows of them, NT x NP MFMA tiles (rows: channels, columns: the 32 pixels of one row). Per chunk of KC
+// input channels the tile's pixels with a 1-pixel halo and the chunk's weights of all 9 taps go to LDS
+// once; the input fragment of a row then serves the three taps of its column offset and every channel
+// tile, a weight fragment all NP rows: (NP + 2) + 3 NT KB from LDS per 3 NT NP instructions, 12 KB per 24
+// at NT = 2, NP = 4 (half of the LDS bandwidth at full MFMA rate). Operands read from the caches
+// instead, 4 KB per 4 instructions, bound the kernel at 150 TFLOP/s. The 14 convolutions of a forward pass
+// of 8 pairs of 256^2 (4 scales, 32 channels): 1049 -> 321 us, 530 TFLOP/s; the small batches and 32
+// channels at full size are bound by the staging's latency and by HBM.
+//
+// LDS slots of 16 bytes (8 channels) are permuted within a pixel (or weight row) by bits of its column, so
+// that 8 or 16 lanes reading the same channels of consecutive columns hit distinct banks.
 // ------------------------------------------------------------------------------------------------
-template <int NT, int NP, typename OutT>
-__global__ void __launch_bounds__(256)
+template <int KC>
+__device__ __forceinline__ int conv_slot(int col, int seg) {
+  if constexpr (KC == 32)
+    return seg ^ (((col >> 2) & 1) | ((((col >> 1) ^ (col >> 3)) & 1) << 1));
+  else
+    return seg ^ (((col >> 2) ^ (col >> 3)) & 1);
+}
+
+// Packed weights: per block of 32 output channels and chunk of KC input channels, [tap][channel row][KC]
+// with the rows' slots permuted, in the order the kernel copies them to LDS.
+__host__ __device__ inline int conv_kc(int cin) { return cin % 32 == 0 ? 32 : 16; }
+
+template <int NT, int NP, int KC, typename OutT>
+__global__ void __launch_bounds__(256, 2)
 k_conv3x3(ConvIn in, const bf16 *__restrict__ w, const float *__restrict__ bias, OutT *__restrict__ y, int B, int H,
-          int W, int cout, int relu, int flip) {
+          int W, int cout, int relu) {
+  constexpr int SEG = KC / 8, HR = 4 * NP + 2, HC = 34, NLD = HR * HC * SEG, NIN = (NLD + 255) / 256;
+  constexpr int WB = 9 * 32 * KC;  // values of one packed weight block
+  __shared__ bf16 sx[HR * HC * KC];
+  __shared__ bf16 sw[NT * WB];
   const int cin = in.c1 + in.c2;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long M = (long)B * H * W;
-  const long m0 = ((long)blockIdx.x * 4 + wave) * 32 * NP;
-  if (m0 >= M) return;  // whole waves only (M % (32 NP) == 0)
-  const int n0 = blockIdx.y * 32 * NT;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tilesx = W / 32, tilesy = H / (4 * NP), ncb = cout / (32 * NT);
+  int t0 = xcd_order(blockIdx.x, gridDim.x);
+  const int cb = t0 % ncb;
+  t0 /= ncb;
+  const int x0 = (t0 % tilesx) * 32;
+  t0 /= tilesx;
+  const int y0 = (t0 % tilesy) * (4 * NP), b = t0 / tilesy;
   const int px = lane & 31, kh = lane >> 5;
-  // the NP tiles lie in one image row: same row and batch, x advancing by 32
-  const int x0 = (int)((m0 + px) % W);
-  const long t0 = (m0 + px) / W;
-  const int yy = (int)(t0 % H), b = (int)(t0 / H);
+  const int nchunk = cin / KC;
+  const int Hh = H >> 1, Wh = W >> 1;
+
+  // the pixels this thread stages: index in the first source (at half size when upsampled) and in the
+  // second; -1 outside the image (zeros)
+  int p1[NIN], p2[NIN];
+  unsigned slots = 0;  // the LDS slots within the pixels, 2 bits each
+#pragma unroll
+  for (int k = 0; k < NIN; ++k) {
+    const int i = tid + 256 * k, pix = i / SEG, seg = i % SEG;
+    const int row = pix / HC, col = pix % HC;
+    const int gy = y0 + row - 1, gx = x0 + col - 1;
+    const bool ok = i < NLD && gy >= 0 && gy < H && gx >= 0 && gx < W;
+    p2[k] = ok ? (b * H + gy) * W + gx : -1;
+    p1[k] = ok ? (in.up1 ? (b * Hh + (gy >> 1)) * Wh + (gx >> 1) : p2[k]) : -1;
+    slots |= (unsigned)conv_slot<KC>(col, seg) << (2 * k);
+  }
+
   f32x16 acc[NT][NP];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -107,62 +159,90 @@ k_conv3x3(ConvIn in, const bf16 *__restrict__ w, const float *__restrict__ bias,
     for (int q = 0; q < NP; ++q)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[t][q][r] = 0.f;
-  const int Hh = H >> 1, Wh = W >> 1;
-  for (int tap = 0; tap < 9; ++tap) {
-    const int sy = yy + tap / 3 - 1;
-    const int wt = flip ? 8 - tap : tap;
-    const bf16 *p1[NP], *p2[NP];
-    bool inb[NP];
+
+  for (int ch = 0; ch < nchunk; ++ch) {
+    const int c0 = ch * KC;
+    const bool first = c0 < in.c1;  // a chunk lies in one source
+    const bf16 *src = first ? in.x1 + c0 : in.x2 + (c0 - in.c1);
+    const int cs = first ? in.c1 : in.c2;
+    u16x8 v[NIN];
 #pragma unroll
-    for (int q = 0; q < NP; ++q) {
-      const int sx = x0 + 32 * q + tap % 3 - 1;
-      inb[q] = sy >= 0 && sy < H && sx >= 0 && sx < W;
-      p1[q] = in.x1;
-      p2[q] = in.x2;
-      if (inb[q]) {
-        p1[q] += (in.up1 ? (((long)b * Hh + (sy >> 1)) * Wh + (sx >> 1)) : (((long)b * H + sy) * W + sx)) * in.c1;
-        if (in.c2) p2[q] += (((long)b * H + sy) * W + sx) * in.c2;
+    for (int k = 0; k < NIN; ++k) {
+      const int p = first ? p1[k] : p2[k];
+      v[k] = (u16x8)0;
+      if (p >= 0) v[k] = *(const u16x8 *)(src + (long)p * cs + (tid % SEG) * 8);
+    }
+    constexpr int NW = WB / 8;  // 16-byte pieces of a weight block
+    u16x8 wv[NT][(NW + 255) / 256];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const bf16 *wb = w + ((long)(cb * NT + t) * nchunk + ch) * WB;
+#pragma unroll
+      for (int k = 0; k < (NW + 255) / 256; ++k) {
+        const int i = tid + 256 * k;
+        if (i < NW) wv[t][k] = *(const u16x8 *)(wb + i * 8);
       }
     }
-    const bf16 *wrow = w + ((long)wt * cout + n0 + px) * cin + 8 * kh;
-    for (int c0 = 0; c0 < cin; c0 += 16) {
-      const int c = c0 + 8 * kh;
-      u16x8 bv[NP];
+    if (ch) __syncthreads();  // the previous chunk's reads are done
 #pragma unroll
-      for (int q = 0; q < NP; ++q) {
-        bv[q] = (u16x8)0;
-        if (inb[q]) bv[q] = *(const u16x8 *)(c < in.c1 ? p1[q] + c : p2[q] + (c - in.c1));
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const u16x8 av = *(const u16x8 *)(wrow + (long)t * 32 * cin + c0);
-#pragma unroll
-        for (int q = 0; q < NP; ++q)
-          acc[t][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(av), as_bf16x8(bv[q]), acc[t][q], 0, 0, 0);
-      }
-    }
-  }
-  // lane: pixel m0 + 32 q + px (column px of tile q); rows = output channels (r/4)*8 + kh*4 + r%4
-#pragma unroll
-  for (int q = 0; q < NP; ++q) {
-    const long m = m0 + 32 * q + px;
+    for (int k = 0; k < NIN; ++k)
+      if (tid + 256 * k < NLD)
+        *(u16x8 *)(sx + (tid / SEG + 256 / SEG * k) * KC + ((slots >> (2 * k)) & 3) * 8) = v[k];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int co = n0 + t * 32 + j * 8 + kh * 4;
-        OutT *dst = y + m * cout + co;
+      for (int k = 0; k < (NW + 255) / 256; ++k) {
+        const int i = tid + 256 * k;
+        if (i < NW) *(u16x8 *)(sw + t * WB + i * 8) = wv[t][k];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < KC / 16; ++ks) {
+      const bf16 *wr = sw + (px * SEG + conv_slot<KC>(px, 2 * ks + kh)) * 8;
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        const bf16 *xr = sx + ((wave * NP * HC + px + dx) * SEG + conv_slot<KC>(px + dx, 2 * ks + kh)) * 8;
+        u16x8 bv[NP + 2];
+#pragma unroll
+        for (int r = 0; r < NP + 2; ++r) bv[r] = *(const u16x8 *)(xr + r * HC * KC);
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const u16x8 av = *(const u16x8 *)(wr + t * WB + (dy * 3 + dx) * 32 * KC);
+#pragma unroll
+            for (int q = 0; q < NP; ++q)
+              acc[t][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(av), as_bf16x8(bv[q + dy]), acc[t][q], 0, 0, 0);
+          }
+      }
+    }
+  }
+  // lane: pixel px of row q; rows of the tile = output channels (r/4)*8 + kh*4 + r%4
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int co = (cb * NT + t) * 32 + j * 8 + kh * 4;
+      float bs[4] = {0.f, 0.f, 0.f, 0.f};
+      if (bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bs[e] = bias[co + e];
+      }
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        OutT *dst = y + ((long)(b * H + y0 + wave * NP + q) * W + x0 + px) * cout + co;
+        float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float v = acc[t][q][j * 4 + e] + (bias ? bias[co + e] : 0.f);
-          if (relu) v = v > 0.f ? v : 0.f;
-          if constexpr (sizeof(OutT) == 2)
-            dst[e] = f2bf(v);
-          else
-            dst[e] = v;
+          v[e] = acc[t][q][j * 4 + e] + bs[e];
+          if (relu) v[e] = v[e] > 0.f ? v[e] : 0.f;
         }
+        if constexpr (sizeof(OutT) == 2)
+          *(u16x4 *)dst = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+        else
+          *(f32x4 *)dst = f32x4{v[0], v[1], v[2], v[3]};
       }
-  }
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -489,7 +569,8 @@ __global__ void k_adam(float *__restrict__ w, const float *__restrict__ g, float
   w[i] -= lr * (a / c1) / (sqrtf(v / c2) + eps);
 }
 
-// BF16 copies of a layer's weights: wf[tap][co][ci] (forward) and wd[tap][ci][co] (data gradient)
+// BF16 copies of a layer's weights packed for k_conv3x3: wf (rows: output channels) for the forward, wd
+// (rows: input channels, taps flipped) for the data gradient.
 __global__ void k_weights_bf16(const float *__restrict__ w, bf16 *__restrict__ wf, bf16 *__restrict__ wd, int cout,
                                int cin) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -499,8 +580,13 @@ __global__ void k_weights_bf16(const float *__restrict__ w, bf16 *__restrict__ w
   const long t = i / cin;
   const int co = (int)(t % cout), tap = (int)(t / cout);
   const bf16 v = f2bf(w[i]);
-  wf[i] = v;
-  if (wd) wd[((long)tap * cin + ci) * cout + co] = v;
+  auto at = [](int row, int k, int tap, int ktotal) {
+    const int kc = conv_kc(ktotal), r = row & 31, seg = (k % kc) >> 3;
+    const int slot = kc == 32 ? conv_slot<32>(r, seg) : conv_slot<16>(r, seg);
+    return ((((long)(row >> 5) * (ktotal / kc) + k / kc) * 9 + tap) * 32 + r) * kc + slot * 8 + (k & 7);
+  };
+  wf[at(co, ci, tap, cin)] = v;
+  if (wd) wd[at(ci, co, 8 - tap, cout)] = v;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -665,35 +751,34 @@ int ensure_acts(msg_unet *u, int B, int H, int W, bool grads) {
   return MSG_OK;
 }
 
-int launch_conv(msg_unet *u, const Conv &c, const bf16 *w, const float *bias, void *y, bool out_f32, int cout,
-                int relu, int flip, ConvIn in, int H, int W) {
-  const long M = (long)u->B * H * W;
-  const int nt = (cout % 64 == 0) ? 2 : 1;
-  const int np = (W % 64 == 0) ? 2 : 1;
-  dim3 grid(cdivu(M, 128 * np), cout / (32 * nt));
-  if (out_f32) {
-    float *yo = (float *)y;
-    if (nt == 2 && np == 2)
-      hipLaunchKernelGGL((k_conv3x3<2, 2, float>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-    else if (nt == 2)
-      hipLaunchKernelGGL((k_conv3x3<2, 1, float>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-    else if (np == 2)
-      hipLaunchKernelGGL((k_conv3x3<1, 2, float>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
+template <int NT, int NP, typename OutT>
+void launch_conv_tile(msg_unet *u, ConvIn in, const bf16 *w, const float *bias, OutT *y, int H, int W, int cout,
+                      int relu) {
+  const dim3 grid((unsigned)((long)u->B * (W / 32) * (H / (4 * NP)) * (cout / (32 * NT))));
+  if (conv_kc(in.c1 + in.c2) == 32)
+    hipLaunchKernelGGL((k_conv3x3<NT, NP, 32, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
+  else
+    hipLaunchKernelGGL((k_conv3x3<NT, NP, 16, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
+}
+
+// H and W are multiples of 32, cout of 32. The largest tile that still gives every compute unit two
+// workgroups (one waits at its staging while the other computes); failing that, one; else the smallest.
+template <typename OutT>
+int launch_conv(msg_unet *u, ConvIn in, const bf16 *w, const float *bias, OutT *y, int cout, int relu, int H, int W) {
+  const long rows = (long)u->B * (W / 32) * (H / 4) * (cout / 32);  // workgroups at NT = NP = 1
+  const bool two = cout % 64 == 0;
+  if (two && rows / 8 >= 512)
+    launch_conv_tile<2, 4>(u, in, w, bias, y, H, W, cout, relu);
+  else if (rows / 4 >= 512) {
+    if (two)
+      launch_conv_tile<2, 2>(u, in, w, bias, y, H, W, cout, relu);
     else
-      hipLaunchKernelGGL((k_conv3x3<1, 1, float>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-  } else {
-    bf16 *yo = (bf16 *)y;
-    if (nt == 2 && np == 2)
-      hipLaunchKernelGGL((k_conv3x3<2, 2, bf16>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-    else if (nt == 2)
-      hipLaunchKernelGGL((k_conv3x3<2, 1, bf16>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-    else if (np == 2)
-      hipLaunchKernelGGL((k_conv3x3<1, 2, bf16>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-    else
-      hipLaunchKernelGGL((k_conv3x3<1, 1, bf16>), grid, dim3(256), 0, u->s, in, w, bias, yo, u->B, H, W, cout, relu, flip);
-  }
+      launch_conv_tile<1, 4>(u, in, w, bias, y, H, W, cout, relu);
+  } else if (rows / 2 >= 256)
+    launch_conv_tile<1, 2>(u, in, w, bias, y, H, W, cout, relu);
+  else
+    launch_conv_tile<1, 1>(u, in, w, bias, y, H, W, cout, relu);
   UHIP(hipGetLastError());
-  (void)c;
   return MSG_OK;
 }
 
@@ -726,8 +811,8 @@ int forward(msg_unet *u, const float *input) {
       ++pi;
     }
     const int s = u->acts[c.out].scale;
-    UCHK(launch_conv(u, c, u->wf[k].as<bf16>(), u->w.as<float>() + c.boff, u->acts[c.out].y.p, false, c.cout, 1, 0,
-                     conv_input(u, c), H >> s, W >> s));
+    UCHK(launch_conv(u, conv_input(u, c), u->wf[k].as<bf16>(), u->w.as<float>() + c.boff, u->acts[c.out].y.as<bf16>(),
+                     c.cout, 1, H >> s, W >> s));
   }
   hipLaunchKernelGGL(k_head, dim3(cdivu(px0, 256)), dim3(256), 0, u->s, u->acts[u->head_in].y.as<bf16>(),
                      u->w.as<float>() + u->whoff, u->w.as<float>() + u->bhoff, u->out.as<float>(), B, H, W,
@@ -790,7 +875,7 @@ int backward(msg_unet *u, const float *target, double *loss) {
     din.c1 = c.cout;
     din.c2 = 0;
     din.up1 = 0;
-    UCHK(launch_conv(u, c, u->wd[k].as<bf16>(), nullptr, u->dv.p, true, cin, 0, 1, din, Hs, Ws));
+    UCHK(launch_conv(u, din, u->wd[k].as<bf16>(), (const float *)nullptr, u->dv.as<float>(), cin, 0, Hs, Ws));
     const Act &a1 = u->acts[c.in1];
     const long n1 = (long)B * (H >> a1.scale) * (W >> a1.scale) * c.cin1;
     hipLaunchKernelGGL(k_split_grad1, dim3(cdivu(n1, 256)), dim3(256), 0, u->s, u->dv.as<float>(), a1.dy.as<float>(),
