@@ -246,96 +246,165 @@ k_conv3x3(ConvIn in, const bf16 *__restrict__ w, const float *__restrict__ bias,
 }
 
 // ------------------------------------------------------------------------------------------------
-// Weight gradient of a 3x3 convolution over one chunk of pixels:
-// part[chunk][tap][co][ci] = sum_{p in chunk} dz[p][co] in[p + off(tap)][ci].
-// Grid: x = chunk, y = tap * (cout / 32) + co block, z = ci block of 32. Each wave reduces a quarter of
-// the chunk with MFMA (rows co, columns ci, reduction over 16 pixels per instruction). Both operands
-// are channel-innermost while the reduction runs over pixels, so a wave stages each step's 16 pixels
-// x 32 channels of dz and of the input through its own LDS block with one 16-byte load per lane and
-// operand, then reads them across pixels; the four waves are summed in LDS in a fixed order.
+// Weight gradient of a 3x3 convolution: part[split][tap][co][ci] = sum over the split's pixels of
+// dz[p][co] in[p + off(tap)][ci].
+//
+// A workgroup takes 32 WM output x 32 WN input channels, all 9 taps, and a range of spatial tiles of R rows
+// x 32 columns; its four waves are WM x WN channel blocks times KS = 4 / (WM WN) shares of a tile's rows,
+// summed at the end in a fixed order. Per tile, dz and the input with a 1-pixel halo go to LDS as
+// [channel block][pixel][32]. The reduction runs over pixels while both operands are channel-innermost:
+// the transposing LDS read (ds_read_b64_tr_b16) gives a lane 4 consecutive pixels of its channel. A wave
+// walks the input's rows: the three fragments of a row (one per column offset) meet the dz fragments of
+// the three rows around it, which stay in registers, so 9 instructions take 4 KB from LDS (44 % of its
+// bandwidth at full MFMA rate). The 14 layers of a training step of 8 pairs of 256^2: 1.22 ms (with each
+// wave staging and gathering 16-bit operands by itself, 143 TFLOP/s) -> 0.41 ms.
 // ------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+
+// 8 pixels (from p, 32 values apart) of one channel per lane: the MFMA operand of 16 pixels x 32 channels
+// whose lane addresses p holds (rows 4 apart for the second half)
+__device__ __forceinline__ bf16x8 read_transposed(const bf16 *p) {
+  typedef __attribute__((address_space(3))) s16x4 lds4;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)(p + 4 * 32));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// 16 bytes per lane from global memory straight to LDS, no registers in between: lane l's to dst + 16 l
+// (dst is the same for the whole wave; inactive lanes write nothing). Complete after lds_loads_done.
+__device__ __forceinline__ void load_to_lds(const bf16 *src, bf16 *dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                   (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+}
+__device__ __forceinline__ void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// what pixels outside the image read
+__device__ __align__(16) const bf16 conv_zeros[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+
+template <int WM, int WN, int R>
+__global__ void __launch_bounds__(256, 2)
 k_conv3x3_wgrad(ConvIn in, const bf16 *__restrict__ dz, float *__restrict__ part, int B, int H, int W, int cout,
-                int chunk) {
+                int nsplit) {
+  constexpr int KS = 4 / (WM * WN), RW = R / KS, HC = 34;
+  constexpr int ZPIX = R * 32, XPIX = (R + 2) * HC;
+  constexpr int NZ = ZPIX * WM * 4, NX = XPIX * WN * 4;  // 16-byte pieces
+  __shared__ bf16 lds[(ZPIX * WM + XPIX * WN) * 32];
+  static_assert(sizeof(lds) >= 3 * 16 * 64 * sizeof(float), "the final sum over the row shares reuses the tile");
+  bf16 *sz = lds, *sx = lds + ZPIX * WM * 32;
   const int cin = in.c1 + in.c2;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int cob = cout / 32;
-  const int tap = blockIdx.y / cob, co0 = (blockIdx.y % cob) * 32, ci0 = blockIdx.z * 32;
-  const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-  const long M = (long)B * H * W;
-  const long pbeg = (long)blockIdx.x * chunk, pend = pbeg + chunk < M ? pbeg + chunk : M;
-  const int px = lane & 31, kh = lane >> 5;
-  // staging: lane -> pixel q = lane / 4 of the step, channels 8 g .. 8 g + 7 of the 32-block
-  const int q = lane >> 2, grp = lane & 3;
-  const int cs = ci0 + 8 * grp;  // first input channel this lane stages
-  const bool cs_ok = cs < cin;
-  const bool cs1 = cs < in.c1;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wave0 = __builtin_amdgcn_readfirstlane(wave * 64);  // this wave's first piece
+  const int wm = wave % WM, wn = (wave / WM) % WN, ks = wave / (WM * WN);
+  const int ncob = cout / (32 * WM), ncib = (cin + 32 * WN - 1) / (32 * WN);
+  int id = xcd_order(blockIdx.x, gridDim.x);
+  const int co0 = (id % ncob) * 32 * WM;
+  id /= ncob;
+  const int ci0 = (id % ncib) * 32 * WN, split = id / ncib;
+  const int tilesx = W / 32, tilesy = H / R, ntile = B * tilesy * tilesx;
+  const int tbeg = (int)((long)ntile * split / nsplit), tend = (int)((long)ntile * (split + 1) / nsplit);
   const int Hh = H >> 1, Wh = W >> 1;
-  __shared__ bf16 sa[4][16 * 32], sb[4][16 * 32];  // [wave][pixel][channel]
-  bf16 *la = sa[wave], *lb = sb[wave];
-  f32x16 acc;
+  // transposing reads: 16 lanes take 4 pixels x 16 channels; the wave's four groups two channel halves and
+  // pixels 0..3 and 8..11 (read_transposed adds 4..7 and 12..15)
+  const int g = lane >> 4, sl = lane & 15;
+  const int loff = (8 * (g >> 1) + (sl >> 2)) * 32 + 16 * (g & 1) + 4 * (sl & 3);
+  const bf16 *az = sz + (wm * ZPIX + ks * RW * 32) * 32 + loff, *bx = sx + (wn * XPIX + ks * RW * HC) * 32 + loff;
+
+  f32x16 acc[9];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  const long quarter = (chunk / 4 + 15) / 16 * 16;
-  const long wbeg = pbeg + wave * quarter;
-  const long wend = wbeg + quarter < pend ? wbeg + quarter : pend;
-  auto wave_sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
-  for (long p0 = wbeg; p0 < wend; p0 += 16) {
-    // 16 consecutive pixels from a multiple of 16 lie in one image row (W % 32 == 0)
-    const int row = (int)(p0 / W), x0 = (int)(p0 - (long)row * W);
-    const int yy = row % H, b = row / H;
-    const int sy = yy + dy;
-    const bool pin = p0 + q < wend;
-    u16x8 av = (u16x8)0, bv = (u16x8)0;
-    if (pin) av = *(const u16x8 *)(dz + (p0 + q) * cout + co0 + 8 * grp);
-    const int sx = x0 + q + dx;
-    if (pin && cs_ok && sy >= 0 && sy < H && sx >= 0 && sx < W) {
-      const bf16 *src;
-      if (cs1)
-        src = in.x1 + (in.up1 ? (((long)b * Hh + (sy >> 1)) * Wh + (sx >> 1)) : (((long)b * H + sy) * W + sx)) * in.c1 + cs;
-      else
-        src = in.x2 + (((long)b * H + sy) * W + sx) * in.c2 + (cs - in.c1);
-      bv = *(const u16x8 *)src;
-    }
-    wave_sync();  // the previous step's reads are done
-    *(u16x8 *)(la + q * 32 + 8 * grp) = av;
-    *(u16x8 *)(lb + q * 32 + 8 * grp) = bv;
-    wave_sync();
-    u16x8 a, bb;
+  for (int t = 0; t < 9; ++t)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      a[k] = la[(8 * kh + k) * 32 + px];
-      bb[k] = lb[(8 * kh + k) * 32 + px];
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+
+  for (int tile = tbeg; tile < tend; ++tile) {
+    const int x0 = (tile % tilesx) * 32, y0 = (tile / tilesx % tilesy) * R, b = tile / tilesx / tilesy;
+    if (tile > tbeg) __syncthreads();  // the previous tile's reads are done
+#pragma unroll
+    for (int k = 0; k < (NZ + 255) / 256; ++k) {
+      const int i = tid + 256 * k, seg = i & 3, pix = (i >> 2) % ZPIX, cb = (i >> 2) / ZPIX;
+      const bf16 *src = dz + ((long)(b * H + y0 + pix / 32) * W + x0 + pix % 32) * cout + co0 + 32 * cb + 8 * seg;
+      if (i < NZ) load_to_lds(src, sz + (wave0 + 256 * k) * 8);
     }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(bb), acc, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < (NX + 255) / 256; ++k) {
+      const int i = tid + 256 * k, seg = i & 3, pix = (i >> 2) % XPIX, cb = (i >> 2) / XPIX;
+      const int gy = y0 + pix / HC - 1, gx = x0 + pix % HC - 1, c = ci0 + 32 * cb + 8 * seg;
+      const bf16 *src = conv_zeros;
+      if (gy >= 0 && gy < H && gx >= 0 && gx < W && c < cin) {
+        if (c < in.c1)
+          src = in.x1 + (long)(in.up1 ? (b * Hh + (gy >> 1)) * Wh + (gx >> 1) : (b * H + gy) * W + gx) * in.c1 + c;
+        else
+          src = in.x2 + (long)((b * H + gy) * W + gx) * in.c2 + (c - in.c1);
+      }
+      if (i < NX) load_to_lds(src, sx + (wave0 + 256 * k) * 8);
+    }
+    lds_loads_done();
+    __syncthreads();
+#pragma unroll
+    for (int xs = 0; xs < 2; ++xs) {  // 16 columns at a time
+      bf16x8 a[3];
+#pragma unroll
+      for (int r = 0; r < RW + 2; ++r) {  // the input's row r - 1 relative to this wave's rows of dz
+        if (r < RW) a[r % 3] = read_transposed(az + (r * 32 + 16 * xs) * 32);
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          const bf16x8 bv = read_transposed(bx + (r * HC + 16 * xs + dx) * 32);
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy)
+            if (r - dy >= 0 && r - dy < RW)
+              acc[dy * 3 + dx] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[(r - dy) % 3], bv, acc[dy * 3 + dx], 0, 0, 0);
+        }
+      }
+    }
   }
-  __shared__ float red[4][16][64];
+
+  const int px = lane & 31, kh = lane >> 5, ci = ci0 + wn * 32 + px;
+  float *red = (float *)lds;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) red[wave][r][lane] = acc[r];
-  __syncthreads();
-  if (wave == 0) {
-    const int ci = ci0 + px;
-    float *dst = part + (((long)blockIdx.x * 9 + tap) * cout) * cin;
+  for (int t = 0; t < 9; ++t) {
+    if constexpr (KS > 1) {
+      __syncthreads();
+      if (ks > 0) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float v = ((red[0][r][lane] + red[1][r][lane]) + red[2][r][lane]) + red[3][r][lane];
-      const int orow = co0 + (r >> 2) * 8 + kh * 4 + (r & 3);
-      if (ci < cin) dst[(long)orow * cin + ci] = v;
+        for (int r = 0; r < 16; ++r) red[((wave - WM * WN) * 16 + r) * 64 + lane] = acc[t][r];
+      }
+      __syncthreads();
+    }
+    if (ks == 0) {
+      float *dst = part + (((long)split * 9 + t) * cout + co0 + wm * 32) * cin;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float v = acc[t][r];
+#pragma unroll
+        for (int k = 1; k < KS; ++k) v += red[((wave + (k - 1) * WM * WN) * 16 + r) * 64 + lane];
+        const int orow = (r >> 2) * 8 + kh * 4 + (r & 3);
+        if (ci < cin) dst[(long)orow * cin + ci] = v;
+      }
     }
   }
 }
 
-// dw[i] (+)= sum over chunks in order of part[chunk][i]
-__global__ void k_sum_chunks(const float *__restrict__ part, int nchunks, long n, float *__restrict__ dw) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// dw[i] = sum over chunks of part[chunk][i]: a workgroup takes 64 elements, its 4 waves every fourth chunk
+// in order (8 loads in flight each), their sums added in order. (One thread per element over all chunks:
+// 188 us per training step of 8 pairs of 256^2; so: 111 us, of more partial sums.)
+__global__ void __launch_bounds__(256)
+k_sum_chunks(const float *__restrict__ part, int nchunks, long n, float *__restrict__ dw) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long i = (long)blockIdx.x * 64 + lane, j = i < n ? i : n - 1;
   float a = 0.f;
-  for (int c = 0; c < nchunks; ++c) a += part[(long)c * n + i];
-  dw[i] = a;
+  for (int c0 = wave; c0 < nchunks; c0 += 32) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int c = c0 + 4 * k;
+      v[k] = part[(long)(c < nchunks ? c : nchunks - 1) * n + j];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a += c0 + 4 * k < nchunks ? v[k] : 0.f;
+  }
+  __shared__ float s[4][64];
+  s[wave][lane] = a;
+  __syncthreads();
+  if (wave == 0 && i < n) dw[i] = ((s[0][lane] + s[1][lane]) + s[2][lane]) + s[3][lane];
 }
 
 // dz = bf16(dy * [y > 0]) and per-block partial sums of dz (in FP32) per channel for the bias gradient.
@@ -710,6 +779,25 @@ int refresh_bf16(msg_unet *u) {
   return MSG_OK;
 }
 
+// Launch shape of the weight gradient: channel blocks per workgroup (wm x wn), rows per spatial tile, and
+// the number of pixel ranges, each a partial sum. 64 x 64 channels where both are multiples (a staged
+// pixel then meets most operands), the rows shared among waves otherwise. About two workgroups per compute
+// unit, fewer where a range would fall below two tiles: every range costs a write and a read of its
+// partial sums.
+struct WgradGeom {
+  int wm, wn, rows, nblocks, nsplit;
+};
+WgradGeom wgrad_geom(int B, int H, int W, int cin, int cout) {
+  WgradGeom g;
+  g.wm = cout % 64 == 0 ? 2 : 1;
+  g.wn = cin % 64 == 0 ? 2 : 1;
+  g.rows = g.wm * g.wn == 1 ? 16 : 8;
+  g.nblocks = (cout / (32 * g.wm)) * cdivu(cin, 32 * g.wn);
+  const int ntile = B * (H / g.rows) * (W / 32);
+  g.nsplit = std::max(1, std::min(cdivu(512, g.nblocks), cdivu(ntile, 2)));
+  return g;
+}
+
 int ensure_acts(msg_unet *u, int B, int H, int W, bool grads) {
   if (H % (32 << (u->scales - 1)) != 0 || W % (32 << (u->scales - 1)) != 0)
     return ufail(MSG_ERR_ARG, "msg_unet: H and W must be multiples of 32 * 2^(scales-1)");
@@ -734,8 +822,7 @@ int ensure_acts(msg_unet *u, int B, int H, int W, bool grads) {
       const int cin = c.cin1 + c.cin2;
       dvmax = std::max(dvmax, px * cin * 4);
       dzmax = std::max(dzmax, px * c.cout * 2);
-      const size_t chunks = (px + 4095) / 4096;
-      partmax = std::max(partmax, chunks * 9 * c.cout * cin * 4);
+      partmax = std::max(partmax, (size_t)wgrad_geom(B, H >> s, W >> s, cin, c.cout).nsplit * 9 * c.cout * cin * 4);
       bpmax = std::max(bpmax, (px * c.cout + 255) / 256 * 256 * 4);
     }
     UCHK(u->dv.ensure(dvmax));
@@ -858,14 +945,21 @@ int backward(msg_unet *u, const float *target, double *loss) {
     UHIP(hipGetLastError());
     const ConvIn in = conv_input(u, c);
     const int cin = c.cin1 + c.cin2;
-    const int chunk = 4096;
-    const int nch = cdivu(px, chunk);
-    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(nch, 9 * (c.cout / 32), cdivu(cin, 32)), dim3(256), 0, u->s, in,
-                       u->dz.as<bf16>(), u->part.as<float>(), B, Hs, Ws, c.cout, chunk);
+    const WgradGeom wg = wgrad_geom(B, Hs, Ws, cin, c.cout);
+    const dim3 gw((unsigned)(wg.nblocks * wg.nsplit));
+    float *pt = u->part.as<float>();
+    const bf16 *zp = u->dz.as<bf16>();
+    if (wg.wm == 2 && wg.wn == 2)
+      hipLaunchKernelGGL((k_conv3x3_wgrad<2, 2, 8>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
+    else if (wg.wm == 2)
+      hipLaunchKernelGGL((k_conv3x3_wgrad<2, 1, 8>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
+    else if (wg.wn == 2)
+      hipLaunchKernelGGL((k_conv3x3_wgrad<1, 2, 8>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
+    else
+      hipLaunchKernelGGL((k_conv3x3_wgrad<1, 1, 16>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
     UHIP(hipGetLastError());
     const long nw = 9L * c.cout * cin;
-    hipLaunchKernelGGL(k_sum_chunks, dim3(cdivu(nw, 256)), dim3(256), 0, u->s, u->part.as<float>(), nch, nw,
-                       g + c.woff);
+    hipLaunchKernelGGL(k_sum_chunks, dim3(cdivu(nw, 64)), dim3(256), 0, u->s, pt, wg.nsplit, nw, g + c.woff);
     UHIP(hipGetLastError());
     if (k == 0) continue;  // no gradient for the input
     // data gradient of the virtual input (FP32), then to its sources
