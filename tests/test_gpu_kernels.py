@@ -133,3 +133,48 @@ def test_warp_modes(gpu, n, count, code):
                     r1 = (1 - X) * (1 - Y) * v[0] + X * (1 - Y) * v[1] + (1 - X) * Y * v[2] + X * Y * v[3]
                     want = np.where(inside, np.where(Y == 0, r0, r1), np.nan if mode == 2 else 0.75).astype(np_dt)
                 assert np.array_equal(got[k], want, equal_nan=True), (shared, mode, nearest, k)
+
+
+@pytest.mark.parametrize("scales,base,H,W", [(4, 32, 256, 256), (2, 64, 128, 256)])
+def test_unet_tile_choice(gpu, scales, base, H, W):
+    """The convolutions' tiles depend on the amount of work; their sums run in one order, so an image's
+    prediction is the same bits alone as inside a batch of eight."""
+    net = gpu.UNet(scales, base, seed=2)
+    x = torch.rand((8, 2, H, W), device="cuda")
+    whole = net.forward(x)
+    for k in (0, 7):
+        assert torch.equal(net.forward(x[k:k + 1].contiguous())[0], whole[k])
+    net.close()
+
+
+@pytest.mark.parametrize("scales,base,B,H,W", [(1, 32, 3, 32, 96), (2, 64, 1, 64, 128), (2, 128, 1, 64, 64),
+                                               (2, 256, 1, 64, 64)])
+def test_unet_widths(gpu, scales, base, B, H, W):
+    """Every source of an activation's gradient (no pooling at one scale), the convolutions' channel
+    counts up to those whose input tile fits LDS (384) and beyond (512, 768), on one tile of rows and
+    columns and on several: against the CPU network, within four times the difference between FP64 and
+    FP32 accumulation of the same BF16 operands."""
+    import unet_ref as U
+    rng = np.random.default_rng(base)
+    x = rng.random((B, 2, H, W)).astype(np.float32)
+    t = (2.0 * rng.standard_normal((B, 2, H, W))).astype(np.float32)
+    net = gpu.UNet(scales, base, seed=3)
+    p = net.get_params().astype(np.float64)
+    out = host(net.forward(dev(x, torch.float32)))
+    _, g = net.gradient(dev(x, torch.float32), dev(t, torch.float32), want_grad=True)
+    net.close()
+
+    def gap(a, b):
+        return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+    ref, _ = U.forward(p, x.astype(np.float64), scales, base)
+    alt, _ = U.forward(p, x.astype(np.float64), scales, base, acc32=True)
+    assert gap(out, ref) < max(1e-3, 4 * gap(alt, ref))
+    if base == 256:
+        return  # the CPU gradient of this width takes half a minute and its kernels are those above
+    _, ref_g, _ = U.loss_and_grad(p, x.astype(np.float64), t.astype(np.float64), scales, base)
+    _, alt_g, _ = U.loss_and_grad(p, x.astype(np.float64), t.astype(np.float64), scales, base, acc32=True)
+    for c in U.graph(scales, base)[1]:
+        for a, k in ((c["woff"], 9 * c["cout"] * (c["cin1"] + c["cin2"])), (c["boff"], c["cout"])):
+            s = slice(a, a + k)
+            assert gap(g[s], ref_g[s]) < max(1e-2, 4 * gap(alt_g[s], ref_g[s])), a
