@@ -311,6 +311,13 @@ k_energy_exact_f32(const float *__restrict__ R, const float *__restrict__ T, con
                    const PairState *st, double *__restrict__ part, int ntx, int nty, int npairs) {
   const int tiles = ntx * nty;
   constexpr int NC = 2;  // plan_exact: the step, and 0 for the current position
+  // usually no pair is flagged: 64 flags a look, their loads in flight together
+  bool any = false;
+  for (int p0 = 0; p0 < npairs; p0 += 64) {
+    const int q = p0 + (int)(threadIdx.x & 63);
+    any |= __any(q < npairs && st[min(q, npairs - 1)].exact && st[min(q, npairs - 1)].ncand);
+  }
+  if (!any) return;
   const size_t nn = (size_t)n * n;
   const int run = en32_run(n);
   const Div hd = make_div(h);

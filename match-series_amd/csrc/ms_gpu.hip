@@ -122,6 +122,30 @@ int flag_snap(FlagSnap **out) {
   return MSG_OK;
 }
 
+// Pinned host memory of a thread and device for small results that a kernel writes itself (grown, kept):
+// the caller reads them after the stream is synchronised, with no copy launched.
+struct PinnedBuf {
+  void *p = nullptr;
+  size_t n = 0;
+};
+thread_local PinnedBuf g_pinned[16];
+
+int pinned_get(size_t bytes, void **p) {
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  PinnedBuf &b = g_pinned[dev & 15];
+  if (b.n < bytes) {
+    if (b.p) HIPCHK(hipHostFree(b.p));
+    b.p = nullptr;
+    b.n = 0;
+    bytes = std::max<size_t>(bytes, 4096);
+    HIPCHK(hipHostMalloc(&b.p, bytes, hipHostMallocDefault));
+    b.n = bytes;
+  }
+  *p = b.p;
+  return MSG_OK;
+}
+
 // ------------------------------------------------------------------------------------------------
 // Kernel timing with HIP events on the stream each kernel is launched on (opt-in, per class mask).
 // ------------------------------------------------------------------------------------------------
@@ -340,6 +364,34 @@ int launch_grad(const S *R, const S *T, const S *phi, S *DE, int n, const PairSt
   return MSG_OK;
 }
 
+// One control phase for every pair (DT_SSD's kernels also serve DT_CONS, whose partials are laid out alike).
+int launch_control(int phase, int data_term, int npairs, PairState *st, const double *part_e, const double *part_n,
+                   const msg::CtrlArgs &a, int *flags, msg::IterTrace *tr, hipStream_t s) {
+#define CONTROL(PH, DT)                                                                                              \
+  hipLaunchKernelGGL((msg::k_control<PH, DT>), dim3(npairs), dim3(msg::CTRL_THREADS), 0, s, st, part_e, part_n, a, \
+                     flags, tr)
+#define CONTROL_DT(PH)                      \
+  do {                                      \
+    if (data_term == msg::DT_NCC)           \
+      CONTROL(PH, msg::DT_NCC);             \
+    else if (data_term == msg::DT_XSHIFT)   \
+      CONTROL(PH, msg::DT_XSHIFT);          \
+    else                                    \
+      CONTROL(PH, msg::DT_SSD);             \
+  } while (0)
+  switch (phase) {
+    case msg::PH_LEVEL_INIT: CONTROL_DT(msg::PH_LEVEL_INIT); break;
+    case msg::PH_ARMIJO_STEP: CONTROL_DT(msg::PH_ARMIJO_STEP); break;
+    case msg::PH_ARMIJO_INIT: CONTROL(msg::PH_ARMIJO_INIT, msg::DT_SSD); break;
+    case msg::PH_NCC_REF0: CONTROL(msg::PH_NCC_REF0, msg::DT_NCC); break;
+    default: CONTROL(msg::PH_NCC_REF1, msg::DT_NCC); break;
+  }
+#undef CONTROL_DT
+#undef CONTROL
+  HIPCHK(hipGetLastError());
+  return MSG_OK;
+}
+
 // The reference statistics of the NCC energy for every pair of a level (two passes with their
 // control phases); the first energy pass of the level follows.
 template <typename S>
@@ -350,11 +402,9 @@ int ncc_reference_stats(const S *R, int n, PairState *st, double *part, double *
   for (int pass = 0; pass < 2; ++pass) {
     hipLaunchKernelGGL((msg::k_ncc_ref<S>), dim3(g.nblk * B), dim3(256), 0, s, R, n, h, st, part, g.ntx, g.nty, B, pass);
     HIPCHK(hipGetLastError());
-    a.phase = pass ? msg::PH_NCC_REF1 : msg::PH_NCC_REF0;
     a.nblk_energy = g.nblk;
     a.npairs = B;
-    hipLaunchKernelGGL(msg::k_control, dim3(B), dim3(msg::CTRL_THREADS), 0, s, st, part, part_n, a, flags, tr);
-    HIPCHK(hipGetLastError());
+    CHK(launch_control(pass ? msg::PH_NCC_REF1 : msg::PH_NCC_REF0, msg::DT_NCC, B, st, part, part_n, a, flags, tr, s));
   }
   return MSG_OK;
 }
@@ -693,7 +743,6 @@ int solve_level_impl(msg_ctx *c, int l, double lambda, int max_iter, double stop
   a.max_iter = max_iter;
   a.spec = spec;
   a.trace_cap = tcap;
-  a.data_term = c->data_term;
   a.npairs = B;
   a.sigma_fixed = c->sigma_fixed;
   a.sigma0 = c->sigma0;
@@ -705,10 +754,8 @@ int solve_level_impl(msg_ctx *c, int l, double lambda, int max_iter, double stop
   if (c->data_term == msg::DT_NCC)
     CHK(ncc_reference_stats<S>(R, n, c->st, c->part_e, c->part_n, B, a, c->flags_d, tr, s));
   CHK(launch_energy<S>(R, T, phi, z, d, n, c->st, c->part_e, B, s, c->data_term, 0.0, npsi, true, c->yreg));
-  a.phase = msg::PH_LEVEL_INIT;
   a.slot = 0;
-  hipLaunchKernelGGL(msg::k_control, dim3(B), dim3(msg::CTRL_THREADS), 0, s, c->st, c->part_e, c->part_n, a, c->flags_d, tr);
-  HIPCHK(hipGetLastError());
+  CHK(launch_control(msg::PH_LEVEL_INIT, c->data_term, B, c->st, c->part_e, c->part_n, a, c->flags_d, tr, s));
 
   bool any_active = max_iter > 0;
   int nactive = max_iter > 0 ? B : 0;
@@ -716,18 +763,13 @@ int solve_level_impl(msg_ctx *c, int l, double lambda, int max_iter, double stop
     a.slot = it & 1;
     CHK(launch_grad<S>(R, T, phi, DE, n, c->st, lambda, B, s, c->data_term, npsi, c->yreg));
     CHK(launch_vcycle<S>(DE, 1, z, l, mg, c->st, 1.0, 2 * B, c->part_n, d, s));
-    a.phase = msg::PH_ARMIJO_INIT;
-    hipLaunchKernelGGL(msg::k_control, dim3(B), dim3(msg::CTRL_THREADS), 0, s, c->st, c->part_e, c->part_n, a, c->flags_d, tr);
-    HIPCHK(hipGetLastError());
+    CHK(launch_control(msg::PH_ARMIJO_INIT, c->data_term, B, c->st, c->part_e, c->part_n, a, c->flags_d, tr, s));
     bool searching = true;
     int rounds = 0;
     int nsearch = nactive;  // pairs evaluating in this round (upper bound for the first round)
     while (searching) {
       CHK(launch_energy<S>(R, T, phi, z, d, n, c->st, c->part_e, B, s, c->data_term, 0.0, npsi, true, c->yreg));
-      a.phase = msg::PH_ARMIJO_STEP;
-      hipLaunchKernelGGL(msg::k_control, dim3(B), dim3(msg::CTRL_THREADS), 0, s, c->st, c->part_e, c->part_n, a, c->flags_d,
-                         tr);
-      HIPCHK(hipGetLastError());
+      CHK(launch_control(msg::PH_ARMIJO_STEP, c->data_term, B, c->st, c->part_e, c->part_n, a, c->flags_d, tr, s));
       HIPCHK(hipMemcpyAsync(c->flags_h, c->flags_d, sizeof(int) * B, hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));
       searching = false;
@@ -827,7 +869,6 @@ int solve_level_dd(msg_ctx *c, int l, double lambda, int max_iter, double stop_e
   a.max_iter = max_iter;
   a.spec = spec;
   a.trace_cap = tcap;
-  a.data_term = c->data_term;
   a.npairs = B;
   a.sigma_fixed = c->sigma_fixed;
   a.sigma0 = c->sigma0;
@@ -840,13 +881,9 @@ int solve_level_dd(msg_ctx *c, int l, double lambda, int max_iter, double stop_e
   // more than the extra launch).
   auto control = [&](int phase, int slot) -> int {
     msg::CtrlArgs ap = a;
-    ap.phase = phase;
     ap.slot = slot;
     ProfScope ps(KC_CONTROL, s, 0);
-    hipLaunchKernelGGL(msg::k_control, dim3(B), dim3(msg::CTRL_THREADS), 0, s, c->st, c->part_e, c->part_n, ap,
-                       c->flags_d, tr);
-    HIPCHK(hipGetLastError());
-    return MSG_OK;
+    return launch_control(phase, c->data_term, B, c->st, c->part_e, c->part_n, ap, c->flags_d, tr, s);
   };
 
   hipLaunchKernelGGL(k_state_init, dim3(cdiv(B, 64)), dim3(64), 0, s, c->st, B, lambda);
@@ -1350,10 +1387,22 @@ int msg_ctx_buffer(msg_ctx *c, int which, int level, void **ptr) {
 }  // extern "C"
 
 namespace {
+// Sums of the partials of candidate 0, one workgroup each, in a fixed order: out[p] = the data energy
+// (times dscale), out[batch + p] = E_reg of pair p. out may be pinned host memory.
+__global__ void __launch_bounds__(256)
+k_energy_sums(const double *__restrict__ part, int nblk, int batch, double dscale, double *__restrict__ out) {
+  __shared__ double red[4];
+  const int p = blockIdx.x % batch, term = blockIdx.x / batch;
+  const double *src = part + msg::part_index(msg::DT_SSD, p, 0, term, nblk);
+  double a = 0;
+#pragma unroll 8
+  for (int b = threadIdx.x; b < nblk; b += 256) a += src[b];
+  a = msg::block_sum<256>(a, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = term ? a : a * dscale;
+}
+
+// Energy pass at phi for every pair: e_data = E_SSD, or the x-shift rows' mean NCC energy.
 template <typename S>
-// Energy pass at phi for every pair, reduced on the host. SSD: e_data = E_SSD. NCC: e_data = E_NCC and,
-// if st_out is given, the pair states the NCC variation reads (reference and template statistics,
-// E_NCC at phi).
 int energy_impl(const void *R, const void *T, const void *phi, int n, int batch, int data_term, double *e_data,
                        double *e_reg, hipStream_t s, double yreg = 0) {
   const int nb = energy_blocks<S>(n, data_term);
@@ -1363,20 +1412,18 @@ int energy_impl(const void *R, const void *T, const void *phi, int n, int batch,
   hipLaunchKernelGGL(k_state_init, dim3(cdiv(batch, 64)), dim3(64), 0, s, (PairState *)stp, batch, 0.0);
   HIPCHK(hipGetLastError());
   CHK(launch_energy<S>((const S *)R, (const S *)T, (const S *)phi, (const S *)phi, (const S *)phi, n,
-                       (const PairState *)stp, (double *)part, batch, s, data_term, 0, 0, true, yreg));
-  std::vector<double> hp(energy_part_size(n, batch));
-  HIPCHK(hipMemcpyAsync(hp.data(), part, sizeof(double) * hp.size(), hipMemcpyDeviceToHost, s));
+                       (const PairState *)stp, (double *)part, batch, s, data_term, 0, 0, false, yreg));
+  // x-shift: the rows' NCC energies averaged over the rows (FELineShiftRegisEnergy::apply)
+  void *sums = nullptr;
+  CHK(pinned_get(sizeof(double) * 2 * batch, &sums));
+  hipLaunchKernelGGL(k_energy_sums, dim3(2 * batch), dim3(256), 0, s, (const double *)part, nb, batch,
+                     data_term == msg::DT_XSHIFT ? 1.0 / n : 1.0, (double *)sums);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
-  auto sum = [&](size_t off) {
-    double a = 0;
-    for (int i = 0; i < nb; ++i) a += hp[off + i];
-    return a;
-  };
+  const double *h = (const double *)sums;
   for (int p = 0; p < batch; ++p) {
-    // x-shift: the rows' NCC energies averaged over the rows (FELineShiftRegisEnergy::apply)
-    const double dscale = data_term == msg::DT_XSHIFT ? 1.0 / n : 1.0;
-    if (e_data) e_data[p] = sum(msg::part_index(msg::DT_SSD, p, 0, 0, nb)) * dscale;
-    if (e_reg) e_reg[p] = sum(msg::part_index(msg::DT_SSD, p, 0, 1, nb));
+    if (e_data) e_data[p] = h[p];
+    if (e_reg) e_reg[p] = h[batch + p];
   }
   return MSG_OK;
 }
@@ -1398,15 +1445,12 @@ int ncc_energy_impl(const void *R, const void *T, const void *phi, int n, int ba
   a.max_iter = 1;  // leaves the pairs active: the variation kernel then takes part
   a.stop_eps = 0;
   a.spec = 1;
-  a.data_term = msg::DT_NCC;
   a.npairs = batch;
   CHK(ncc_reference_stats<S>((const S *)R, n, st, (double *)part, nullptr, batch, a, nullptr, nullptr, s));
   CHK(launch_energy<S>((const S *)R, (const S *)T, (const S *)phi, (const S *)phi, (const S *)phi, n, st,
                        (double *)part, batch, s, msg::DT_NCC));
-  a.phase = msg::PH_LEVEL_INIT;
-  hipLaunchKernelGGL(msg::k_control, dim3(batch), dim3(msg::CTRL_THREADS), 0, s, st, (const double *)part,
-                     (const double *)nullptr, a, (int *)nullptr, (msg::IterTrace *)nullptr);
-  HIPCHK(hipGetLastError());
+  CHK(launch_control(msg::PH_LEVEL_INIT, msg::DT_NCC, batch, st, (const double *)part, (const double *)nullptr, a,
+                     (int *)nullptr, (msg::IterTrace *)nullptr, s));
   std::vector<PairState> hs(batch);
   HIPCHK(hipMemcpyAsync(hs.data(), st, sizeof(PairState) * batch, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
@@ -1551,18 +1595,6 @@ size_t noalloc_energy_bytes(int n, int batch, size_t *off_part, size_t *off_sum)
   return st + part + sizeof(double) * 2 * (size_t)batch;
 }
 
-// Sums of the partials in block order (the order msg_energy sums them on the host): out[p] = E_SSD,
-// out[batch + p] = E_reg of pair p.
-__global__ void k_energy_sums(const double *__restrict__ part, int nblk, int batch, double *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 2 * batch) return;
-  const int p = i % batch, term = i / batch;
-  const double *src = part + msg::part_index(msg::DT_SSD, p, 0, term, nblk);
-  double a = 0;
-  for (int b = 0; b < nblk; ++b) a += src[b];
-  out[i] = a;
-}
-
 template <typename S>
 int energy_noalloc_impl(const void *R, const void *T, const void *phi, int n, int batch, double *e_ssd,
                         double *e_reg, hipStream_t s) {
@@ -1601,8 +1633,7 @@ int energy_noalloc_impl(const void *R, const void *T, const void *phi, int n, in
                        (const S *)phi, (const S *)phi, (const S *)phi, n, h, (int)((n - 1) * h), st, part, g.ntx,
                        g.nty, batch);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_energy_sums, dim3(cdiv(2 * batch, 64)), dim3(64), 0, s, (const double *)part, g.nblk, batch,
-                     sums);
+  hipLaunchKernelGGL(k_energy_sums, dim3(2 * batch), dim3(256), 0, s, (const double *)part, g.nblk, batch, 1.0, sums);
   HIPCHK(hipGetLastError());
   if (e_ssd) HIPCHK(hipMemcpyAsync(e_ssd, sums, sizeof(double) * batch, hipMemcpyDeviceToHost, s));
   if (e_reg) HIPCHK(hipMemcpyAsync(e_reg, sums + batch, sizeof(double) * batch, hipMemcpyDeviceToHost, s));
@@ -1640,13 +1671,15 @@ int h1_impl(const void *in, void *out, int n, int nfields, double sigma, hipStre
     b.x2[m] = (S *)p2;
     b.x[m] = (S *)p3;
   }
-  void *top, *tmpout;
-  CHK(scratch_get(2, (size_t)n * n * nfields * sizeof(S), &top));
-  CHK(scratch_get(3, (size_t)n * n * nfields * sizeof(S), &tmpout));
+  const size_t bytes = (size_t)n * n * nfields * sizeof(S);
+  void *top, *dst = out;
+  CHK(scratch_get(2, bytes, &top));
   b.x2_top = (S *)top;
-  // write into a temporary so that in == out is allowed
-  CHK(launch_vcycle<S>((const S *)in, 0, (S *)tmpout, l, b, nullptr, sigma, nfields, nullptr, (const S *)nullptr, s));
-  HIPCHK(hipMemcpyAsync(out, tmpout, (size_t)n * n * nfields * sizeof(S), hipMemcpyDeviceToDevice, s));
+  // into a temporary where in and out overlap: the last pass reads the input beyond its own tile
+  const bool overlap = (const char *)in < (const char *)out + bytes && (const char *)out < (const char *)in + bytes;
+  if (overlap) CHK(scratch_get(3, bytes, &dst));
+  CHK(launch_vcycle<S>((const S *)in, 0, (S *)dst, l, b, nullptr, sigma, nfields, nullptr, (const S *)nullptr, s));
+  if (overlap) HIPCHK(hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToDevice, s));
   HIPCHK(hipStreamSynchronize(s));
   return MSG_OK;
 }

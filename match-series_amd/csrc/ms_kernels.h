@@ -85,36 +85,27 @@ __device__ __forceinline__ void reduce_arrays_n(const double *base, int len, dou
   __syncthreads();
 }
 
-// nt (<= CTRL_MAXT) arrays: sweeps of at most 8 arrays
-__device__ __forceinline__ void reduce_arrays(const double *base, int nt, int len, double *out) {
-  __shared__ double red[8][RED_THREADS];
-  __shared__ double red2[8][16];
-  static_assert(CTRL_THREADS >= RED_THREADS, "the reduction's threads are part of the control workgroup");
-  for (int t0 = 0; t0 < nt; t0 += 8) {
-    const int m = nt - t0 < 8 ? nt - t0 : 8;
-    const double *b = base + (size_t)t0 * len;
-    switch (m) {
-      case 8: reduce_arrays_n<8>(b, len, out + t0, red, red2); break;
-      case 7: reduce_arrays_n<7>(b, len, out + t0, red, red2); break;
-      case 6: reduce_arrays_n<6>(b, len, out + t0, red, red2); break;
-      case 5: reduce_arrays_n<5>(b, len, out + t0, red, red2); break;
-      case 4: reduce_arrays_n<4>(b, len, out + t0, red, red2); break;
-      case 3: reduce_arrays_n<3>(b, len, out + t0, red, red2); break;
-      case 2: reduce_arrays_n<2>(b, len, out + t0, red, red2); break;
-      default: reduce_arrays_n<1>(b, len, out + t0, red, red2); break;
-    }
+// NT (<= CTRL_MAXT) arrays, in sweeps of at most 8
+template <int NT>
+__device__ __forceinline__ void reduce_arrays(const double *base, int len, double *out) {
+  __shared__ double red[NT < 8 ? NT : 8][RED_THREADS];
+  __shared__ double red2[NT < 8 ? NT : 8][16];
+  static_assert(CTRL_THREADS >= RED_THREADS && NT <= CTRL_MAXT, "the reduction's threads are part of the control workgroup");
+  if constexpr (NT <= 8) {
+    reduce_arrays_n<NT>(base, len, out, red, red2);
+  } else {
+    reduce_arrays_n<8>(base, len, out, red, red2);
+    reduce_arrays_n<NT - 8>(base + (size_t)8 * len, len, out + 8, red, red2);
   }
 }
 
 struct CtrlArgs {
-  int phase;
   int nblk_energy;   // partial count per candidate and term
   int nblk_norm;     // partials per field and term of the V-cycle's last pass
   double lambda, stop_eps;
   int max_iter;
   int spec;          // candidates per energy pass (1..MAX_CAND)
   int trace_cap;
-  int data_term;     // DT_SSD, DT_NCC or DT_CONS
   int npairs;        // pairs of the batch (NCC: the reference statistics follow the candidates' partials)
   int sigma_fixed;   // 1: filter width fixed at sigma0 (H1GradientDescent, gradientDescent.h:639-650)
   double sigma0;
@@ -413,20 +404,40 @@ __device__ __forceinline__ void armijo_run(PairState &s, int spec, double tol, I
   finish_iteration(s, 0.0, trace, trace_cap, pair, slot);  // unreachable guard
 }
 
+// The first part of armijo_run, at the start of an iteration: no evaluation is known yet (no candidates,
+// no last evaluations), so it either plans the first pass or ends without a step.
+__device__ __forceinline__ void armijo_begin(PairState &s, int spec, IterTrace *trace, int trace_cap, int pair, int slot) {
+  for (;;) {
+    if (!(s.a_Df >= 0 || !isfinite(s.energy))) {
+      armijo_plan(s, spec);
+      return;
+    }
+    s.evals++;  // the reference evaluates E(tau0) before these checks
+    if (s.dirmode != DIR_CG) break;
+    s.tau_first = 0;
+    s.olddir_zero = 1;
+    armijo_start(s, DIR_GRAD, s.Dfz, 0.0);
+  }
+  finish_iteration(s, 0.0, trace, trace_cap, pair, slot);
+}
+
 // Runs one control phase for one pair with the whole workgroup (the reductions need every thread)
-// on the workgroup's copy s of the pair state.
+// on the workgroup's copy s of the pair state. A kernel per phase and data term: one kernel for all of
+// them was 45 KB of code, whose fetches cost more than its arithmetic (5.0 us per phase of one pair at
+// 512^2; so, with 4 to 10 KB: 3.7 us at the start of an iteration, 4.6 us per step).
+template <int PH, int DT>
 __device__ __forceinline__ void control_pair(int pair, PairState &s, const double *__restrict__ part_e,
                              const double *__restrict__ part_n, const CtrlArgs &a, int *__restrict__ flags,
                              IterTrace *__restrict__ trace) {
   __shared__ double sums[CTRL_MAXT];
   const bool participates = s.active && !s.searching;
 
-  if (a.phase == PH_NCC_REF0 || a.phase == PH_NCC_REF1) {
+  if constexpr (PH == PH_NCC_REF0 || PH == PH_NCC_REF1) {
     const int nb = a.nblk_energy;
-    reduce_arrays(part_e + part_index_ref(a.npairs, pair, 0, nb), a.phase == PH_NCC_REF1 ? 2 : 1, nb, sums);
-    const double r1 = sums[0], r2 = a.phase == PH_NCC_REF1 ? sums[1] : 0;
+    reduce_arrays<PH == PH_NCC_REF1 ? 2 : 1>(part_e + part_index_ref(a.npairs, pair, 0, nb), nb, sums);
+    const double r1 = sums[0], r2 = PH == PH_NCC_REF1 ? sums[1] : 0;
     if (threadIdx.x == 0) {
-      if (a.phase == PH_NCC_REF0) {
+      if constexpr (PH == PH_NCC_REF0) {
         s.ncc_rm = r1;  // 1'Mr
       } else {
         s.ncc_rb = r1;  // 1'M(r - m_r)
@@ -434,10 +445,11 @@ __device__ __forceinline__ void control_pair(int pair, PairState &s, const doubl
         s.ncc_c = s.ncc_rm;  // the first template moments are taken about the reference's mean
       }
     }
-  } else if ((a.phase == PH_LEVEL_INIT || a.phase == PH_ARMIJO_STEP) && a.data_term == DT_NCC) {
+  } else if constexpr ((PH == PH_LEVEL_INIT || PH == PH_ARMIJO_STEP) && DT == DT_NCC) {
     const int nc = s.ncand;
     const int nb = a.nblk_energy;
-    reduce_arrays(part_e + part_index(DT_NCC, pair, 0, 0, nb), 4 * nc, nb, sums);  // candidate k, term t at 4k+t
+    // candidate k, term t at 4k+t; slots beyond nc hold older values, which nothing reads
+    if (nc > 0) reduce_arrays<4 * PLAN_CAND>(part_e + part_index(DT_NCC, pair, 0, 0, nb), nb, sums);
     if (threadIdx.x == 0) {
       for (int k = 0; k < nc; ++k) {
         double vt;
@@ -452,10 +464,10 @@ __device__ __forceinline__ void control_pair(int pair, PairState &s, const doubl
         s.cand_V[k] = vt;
       }
     }
-  } else if ((a.phase == PH_LEVEL_INIT || a.phase == PH_ARMIJO_STEP) && a.data_term == DT_XSHIFT) {
+  } else if constexpr ((PH == PH_LEVEL_INIT || PH == PH_ARMIJO_STEP) && DT == DT_XSHIFT) {
     // rows' NCC energies summed, then divided by the number of rows (FELineShiftRegisEnergy::apply)
     const int nc = s.ncand;
-    reduce_arrays(part_e + part_index(DT_SSD, pair, 0, 0, a.nblk_energy), 2 * nc, a.nblk_energy, sums);
+    if (nc > 0) reduce_arrays<2 * PLAN_CAND>(part_e + part_index(DT_SSD, pair, 0, 0, a.nblk_energy), a.nblk_energy, sums);
     if (threadIdx.x == 0) {
       for (int k = 0; k < nc; ++k) {
         double D = sums[2 * k];
@@ -470,9 +482,9 @@ __device__ __forceinline__ void control_pair(int pair, PairState &s, const doubl
       }
       s.cand_ex = 0;
     }
-  } else if (a.phase == PH_LEVEL_INIT || a.phase == PH_ARMIJO_STEP) {
+  } else if constexpr (PH == PH_LEVEL_INIT || PH == PH_ARMIJO_STEP) {
     const int nc = s.ncand;
-    reduce_arrays(part_e + part_index(DT_SSD, pair, 0, 0, a.nblk_energy), 2 * nc, a.nblk_energy, sums);
+    if (nc > 0) reduce_arrays<2 * PLAN_CAND>(part_e + part_index(DT_SSD, pair, 0, 0, a.nblk_energy), a.nblk_energy, sums);
     if (threadIdx.x == 0) {
       for (int k = 0; k < nc; ++k) {
         double E = 0;
@@ -491,9 +503,9 @@ __device__ __forceinline__ void control_pair(int pair, PairState &s, const doubl
       }
     }
   }
-  if (a.phase == PH_LEVEL_INIT || a.phase == PH_ARMIJO_STEP) {
+  if constexpr (PH == PH_LEVEL_INIT || PH == PH_ARMIJO_STEP) {
     if (threadIdx.x == 0) {
-      if (a.phase == PH_LEVEL_INIT) {
+      if constexpr (PH == PH_LEVEL_INIT) {
         s.ncc_d = s.cand_D[0];
         s.ncc_m = s.ncc_c = s.cand_M[0];
         s.ncc_v = s.cand_V[0];
@@ -518,12 +530,12 @@ __device__ __forceinline__ void control_pair(int pair, PairState &s, const doubl
         armijo_run(s, a.spec, a.exact_tol, trace, a.trace_cap, pair, a.slot);
       }
     }
-  } else if (a.phase == PH_ARMIJO_INIT) {
+  } else if constexpr (PH == PH_ARMIJO_INIT) {
     // the previous iteration's update has run (stream order): free its slot
     if (threadIdx.x == 0) s.step_tau[a.slot ^ 1] = 0;
     if (!participates) return;
     // field f, term t at f * NORM_TERMS + t
-    reduce_arrays(part_n + (size_t)(2 * pair) * NORM_TERMS * a.nblk_norm, 2 * NORM_TERMS, a.nblk_norm, sums);
+    reduce_arrays<2 * NORM_TERMS>(part_n + (size_t)(2 * pair) * NORM_TERMS * a.nblk_norm, a.nblk_norm, sums);
     if (threadIdx.x == 0) {
       double zz = 0, Dfz = 0, Dfd = 0;
       zz += sums[0];
@@ -552,12 +564,13 @@ __device__ __forceinline__ void control_pair(int pair, PairState &s, const doubl
       s.tau_first = 0;
       armijo_start(s, DIR_CG, Df, s.tau);
       s.searching = 1;
-      armijo_run(s, a.spec, a.exact_tol, trace, a.trace_cap, pair, a.slot);
+      armijo_begin(s, a.spec, trace, a.trace_cap, pair, a.slot);
     }
   }
   if (threadIdx.x == 0 && flags) flags[pair] = (s.searching ? 1 : 0) | (s.active ? 2 : 0);
 }
 
+template <int PH, int DT>
 __global__ void __launch_bounds__(CTRL_THREADS)
 k_control(PairState *__restrict__ st, const double *__restrict__ part_e, const double *__restrict__ part_n, CtrlArgs a,
           int *__restrict__ flags, IterTrace *__restrict__ trace) {
@@ -570,7 +583,7 @@ k_control(PairState *__restrict__ st, const double *__restrict__ part_e, const d
   unsigned *g = reinterpret_cast<unsigned *>(st + pair), *l = reinterpret_cast<unsigned *>(&ss);
   for (int i = threadIdx.x; i < NW; i += CTRL_THREADS) l[i] = g[i];
   __syncthreads();
-  control_pair(pair, ss, part_e, part_n, a, flags, trace);
+  control_pair<PH, DT>(pair, ss, part_e, part_n, a, flags, trace);
   __syncthreads();
   for (int i = threadIdx.x; i < NW; i += CTRL_THREADS) g[i] = l[i];
 }
