@@ -1757,10 +1757,8 @@ int compose_impl(const void *phi1, const void *phi2, void *result, int n, hipStr
   ProfScope ps(KC_COMPOSE, s, 0);
   const int nn = n * n;
   const int nblk = cdiv(nn, 256);
-  void *bc, *rhs, *invd, *x, *g, *hb, *h2, *d0, *d1, *def, *part, *parta, *partb, *U, *nsel, *sel_tmp, *stp, *donep;
+  void *bc, *x, *g, *hb, *h2, *d0, *d1, *def, *part, *parta, *partb, *U, *nsel, *sel_tmp, *stp, *donep;
   CHK(scratch_get(70, sizeof(double) * 2 * nn, &bc));
-  CHK(scratch_get(71, sizeof(double) * 2 * nn, &rhs));
-  CHK(scratch_get(72, sizeof(double) * nn, &invd));
   CHK(scratch_get(73, sizeof(double) * 2 * nn, &x));
   CHK(scratch_get(74, sizeof(double) * 2 * nn, &g));
   CHK(scratch_get(75, sizeof(double) * 2 * nn, &hb));
@@ -1780,8 +1778,6 @@ int compose_impl(const void *phi1, const void *phi2, void *result, int n, hipStr
   const dim3 g1(nblk), b(256);
   hipLaunchKernelGGL((msg::k_compose_init<S>), g1, b, 0, s, (const S *)phi1, (const S *)phi2, (double *)bc,
                      (unsigned char *)def, n);
-  hipLaunchKernelGGL(msg::k_compose_rhs, dim3(cdiv(2 * nn, 256)), b, 0, s, (const double *)bc,
-                     (const unsigned char *)def, (double *)rhs, (double *)invd, n);
   HIPCHK(hipGetLastError());
   // the undefined nodes, in index order
   size_t tbytes = 0;
@@ -1792,21 +1788,24 @@ int compose_impl(const void *phi1, const void *phi2, void *result, int n, hipStr
   HIPCHK(hipcub::DeviceSelect::If(sel_tmp, tbytes, hipcub::CountingInputIterator<int>(0), (int *)U, (int *)nsel, nn,
                                   pred, s));
   // the start value is the result's previous content (PCGInverse::apply starts from its Dest)
-  CHK(convert(result, sizeof(S) == 8 ? MSG_F64 : MSG_F32, x, MSG_F64, 2 * (size_t)nn, s));
-  hipLaunchKernelGGL(msg::k_cg_start, dim3(nblk, 2), b, 0, s, (const double *)x, (const double *)rhs,
-                     (const unsigned char *)def, (const double *)invd, (double *)g, (double *)hb, (double *)d0,
-                     (double *)part, n, nblk);
+  hipLaunchKernelGGL((msg::k_cg_start<S>), dim3(nblk, 2), b, 0, s, (const S *)result, (const double *)bc,
+                     (const unsigned char *)def, (double *)x, (double *)g, (double *)hb, (double *)d0, (double *)part, n,
+                     nblk);
   hipLaunchKernelGGL(msg::k_cg_init, dim3(2), b, 0, s, (const double *)part, nblk, sb, done);
   HIPCHK(hipGetLastError());
-  int nu = 0;
-  HIPCHK(hipMemcpyAsync(&nu, nsel, sizeof(int), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
+  // the number of undefined nodes and the done flags after the start (k_cg_init may already have met the
+  // stopping rule), in one look
+  FlagSnap *fs = nullptr;
+  CHK(flag_snap(&fs));
+  HIPCHK(hipMemcpyAsync(fs->h + 4, nsel, sizeof(int), hipMemcpyDeviceToHost, s));
+  HIPCHK(hipMemcpyAsync(fs->h + 2, done, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
+  HIPCHK(hipEventRecord(fs->ev[1], s));
+  HIPCHK(hipEventSynchronize(fs->ev[1]));
+  const int nu = fs->h[4];
   const int nbu = std::max(1, cdiv(nu, 256));
   double *dbuf[2] = {(double *)d0, (double *)d1};
   // Blocks of 8 iterations, each followed by a snapshot of the done flags; the host checks a block's
   // snapshot while the next block runs (iterations past convergence change nothing).
-  FlagSnap *fs = nullptr;
-  CHK(flag_snap(&fs));
   int k = 0;
   auto block = [&](int blk) -> int {
     for (int r = 0; r < 8 && k <= 1000; ++r, ++k) {
@@ -1816,18 +1815,14 @@ int compose_impl(const void *phi1, const void *phi2, void *result, int n, hipStr
                          (const double *)hb, (double *)h2, (const double *)partb, (double *)parta, nbu,
                          (const msg::CgState *)sb, sa, done, n);
       hipLaunchKernelGGL(msg::k_cg_b, dim3(nbu, 2), b, 0, s, (const int *)U, nu, (double *)x, (const double *)dc,
-                         (double *)g, (double *)hb, (const double *)h2, (const double *)invd, (const double *)parta,
-                         (double *)partb, nbu, (const msg::CgState *)sa, sb, (const int *)done, n);
+                         (double *)g, (double *)hb, (const double *)h2, (const double *)parta, (double *)partb, nbu,
+                         (const msg::CgState *)sa, sb, (const int *)done, n);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(fs->h + 2 * (blk & 1), done, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
     HIPCHK(hipEventRecord(fs->ev[blk & 1], s));
     return MSG_OK;
   };
-  // the state after the start (k_cg_init may already have met the stopping rule)
-  HIPCHK(hipMemcpyAsync(fs->h + 2, done, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipEventRecord(fs->ev[1], s));
-  HIPCHK(hipEventSynchronize(fs->ev[1]));
   if (!(fs->h[2] && fs->h[3])) {
     CHK(block(0));
     for (int blk = 0;; ++blk) {
@@ -1837,7 +1832,7 @@ int compose_impl(const void *phi1, const void *phi2, void *result, int n, hipStr
       if ((fs->h[2 * (blk & 1)] && fs->h[2 * (blk & 1) + 1]) || !more) break;
     }
   }
-  hipLaunchKernelGGL((msg::k_cg_finish<S>), dim3(cdiv(2 * nn, 256)), b, 0, s, (const double *)x, (const double *)rhs,
+  hipLaunchKernelGGL((msg::k_cg_finish<S>), dim3(cdiv(2 * nn, 256)), b, 0, s, (const double *)x, (const double *)bc,
                      (const unsigned char *)def, (const msg::CgState *)sb, (S *)result, n);
   HIPCHK(hipGetLastError());
   return MSG_OK;

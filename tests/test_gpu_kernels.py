@@ -178,3 +178,20 @@ def test_unet_widths(gpu, scales, base, B, H, W):
         for a, k in ((c["woff"], 9 * c["cout"] * (c["cin1"] + c["cin2"])), (c["boff"], c["cout"])):
             s = slice(a, a + k)
             assert gap(g[s], ref_g[s]) < max(1e-2, 4 * gap(alt_g[s], ref_g[s])), a
+
+
+@pytest.mark.parametrize("n", [2, 4, 16, 64])
+@pytest.mark.parametrize("pixels", [0.0, 0.4, 6.0])
+def test_compose_borders(gpu, n, pixels):
+    """No undefined node, a few, and whole borders and corners of them (every form of a stiffness row),
+    from a start value of its own: FP64 fields against the oracle, which runs the same recurrence."""
+    rng = np.random.default_rng(n)
+    h = 1.0 / (n - 1)
+    y, x = np.mgrid[0:n, 0:n] / n
+    p1 = 0.3 * h * rng.normal(size=(2, n, n))
+    p2 = pixels * h * np.stack([np.sin(3 * x + y) - 0.3, np.cos(2 * y - x) - 0.4])
+    start = 0.2 * h * rng.normal(size=(2, n, n))
+    got = host(gpu.compose(dev(p1, torch.float64), dev(p2, torch.float64), dev(start, torch.float64)))
+    want = O.compose(p1, p2, start)
+    # both stop at |residual|^2 < 1e-16; rounding moves the iterates by far less than what that leaves
+    assert np.abs(got - want).max() < 1e-10 * max(np.abs(want).max(), h)
