@@ -296,6 +296,18 @@ int energy_blocks(int n, int data_term) {
   return data_term == msg::DT_XSHIFT ? n : energy_geom(n, is_f32_ssd<S>(data_term)).nblk;
 }
 
+// Calls f with the threads per row and nodes per thread of an x-shift row of n nodes as constants.
+template <typename F>
+void xshift_shape(int n, const F &f) {
+  using std::integral_constant;
+  if (n <= 64) f(integral_constant<int, 64>(), integral_constant<int, 1>());
+  else if (n == 128) f(integral_constant<int, 128>(), integral_constant<int, 1>());
+  else if (n == 256) f(integral_constant<int, 256>(), integral_constant<int, 1>());
+  else if (n == 512) f(integral_constant<int, 256>(), integral_constant<int, 2>());
+  else if (n == 1024) f(integral_constant<int, 256>(), integral_constant<int, 4>());
+  else f(integral_constant<int, 256>(), integral_constant<int, 8>());
+}
+
 // The images of the data term: R, T (SSD, NCC) or, for DT_CONS, the npsi deformations in T.
 template <typename S>
 int launch_energy(const S *R, const S *T, const S *phi, const S *z, const S *dold, int n, const PairState *st,
@@ -306,8 +318,11 @@ int launch_energy(const S *R, const S *T, const S *phi, const S *z, const S *dol
   const double h = 1.0 / (double)(n - 1);
   const int width = (int)((n - 1) * h);
   if (data_term == msg::DT_XSHIFT)
-    hipLaunchKernelGGL((msg::k_energy_xshift<S>), dim3(n * npairs), dim3(msg::XS_THREADS), 3 * n * sizeof(double), s,
-                       R, T, phi, z, dold, n, h, yreg, st, part, npairs);
+    xshift_shape(n, [&](auto th, auto pn) {
+      hipLaunchKernelGGL((msg::k_energy_xshift<S, decltype(th)::value, decltype(pn)::value>), dim3(n * npairs),
+                         dim3(decltype(th)::value), n * sizeof(double), s, R, T, phi, z, dold, n,
+                         h, yreg, st, part, npairs);
+    });
   else if (data_term == msg::DT_CONS)
     hipLaunchKernelGGL((msg::k_energy_cons<S>), dim3(g.nblk * npairs), dim3(256), 0, s, T, npsi, phi, z, dold, n, h,
                        width, st, part, g.ntx, g.nty, npairs);
@@ -346,8 +361,11 @@ int launch_grad(const S *R, const S *T, const S *phi, S *DE, int n, const PairSt
   const double h = 1.0 / (double)(n - 1);
   const int width = (int)((n - 1) * h);
   if (data_term == msg::DT_XSHIFT)
-    hipLaunchKernelGGL((msg::k_grad_xshift<S>), dim3(n * npairs), dim3(msg::XS_THREADS), 3 * n * sizeof(double), s, R,
-                       T, phi, DE, n, h, yreg, st, lambda, npairs);
+    xshift_shape(n, [&](auto th, auto pn) {
+      hipLaunchKernelGGL((msg::k_grad_xshift<S, decltype(th)::value, decltype(pn)::value>), dim3(n * npairs),
+                         dim3(decltype(th)::value), n * sizeof(double), s, R, T, phi, DE, n, h, yreg, st, lambda,
+                         npairs);
+    });
   else if (data_term == msg::DT_CONS)
     hipLaunchKernelGGL((msg::k_grad<S, msg::DT_CONS>), dim3(ntx * nty * npairs), dim3(256), 0, s, R, T, phi, DE, n, h,
                        width, st, lambda, ntx, nty, npairs, npsi);

@@ -195,3 +195,28 @@ def test_compose_borders(gpu, n, pixels):
     want = O.compose(p1, p2, start)
     # both stop at |residual|^2 < 1e-16; rounding moves the iterates by far less than what that leaves
     assert np.abs(got - want).max() < 1e-10 * max(np.abs(want).max(), h)
+
+
+@pytest.mark.parametrize("n", [2, 4, 64, 128, 256, 512, 1024, 2048])
+def test_xshift_row_lengths(gpu, n):
+    """Every thread count and run length of the row kernels, displacements that leave the row at both
+    ends, a row that starts with NaN (left out): FP64 fields against the oracle. Rounding: sums of n
+    terms in another order, 1e-16 n at worst relative to terms of the result's size."""
+    rng = np.random.default_rng(n)
+    x = np.arange(n) / n
+    R = 1 + np.cumsum(rng.normal(size=(n, n)), axis=1) / n
+    T = np.roll(R, 1, axis=1) + 0.02 * rng.normal(size=(n, n))
+    phi = (3.0 * np.sin(7 * x[None, :] + np.arange(n)[:, None] / n) + 0.3 * rng.normal(size=(n, n))) / (n - 1)
+    if n >= 64:
+        R[n // 2, 0] = np.nan
+    args = (dev(R[None], torch.float64), dev(T[None], torch.float64),
+            dev(np.stack([phi, np.zeros_like(phi)])[None], torch.float64))
+    ed, er = gpu.xshift_energy(*args, 0.7)
+    g = host(gpu.xshift_gradient(*args, 5.0, 0.7))[0]
+    oe, orr = O.xshift_energy(R, T, phi, 0.7)
+    og = O.xshift_gradient(R, T, phi, 0.7, 5.0)
+    tol = 2e-16 * 8 * n
+    assert abs(ed[0] - oe) <= max(tol, 1e-14) * max(abs(oe), 1.0)
+    assert abs(er[0] - orr) <= max(tol, 1e-14) * abs(orr)
+    assert np.abs(g[0] - og).max() <= max(100 * tol, 1e-12) * np.abs(og).max()
+    assert (g[1] == 0).all()
