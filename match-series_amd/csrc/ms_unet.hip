@@ -1174,6 +1174,23 @@ int backward(msg_unet *u, const float *target, double *loss) {
   return MSG_OK;
 }
 
+// He initialisation from the seed (the padded input channels stay zero), zero biases. flatten: the generator
+// inlined into the loops, whatever else the file holds (a call per number doubles the two million draws' time).
+__attribute__((flatten)) void he_init(const msg_unet *u, unsigned long long seed, std::vector<float> &h) {
+  std::mt19937_64 rng(seed);
+  std::normal_distribution<double> nd(0.0, 1.0);
+  for (auto &c : u->convs) {
+    const int cin = c.cin1 + c.cin2;
+    const double sd = std::sqrt(2.0 / (9.0 * c.cin_real));
+    for (int t = 0; t < 9; ++t)
+      for (int o = 0; o < c.cout; ++o)
+        for (int i = 0; i < cin; ++i)
+          h[c.woff + ((long)t * c.cout + o) * cin + i] = (c.in1 != 0 || i < c.cin_real) ? (float)(sd * nd(rng)) : 0.f;
+  }
+  const double sdh = std::sqrt(1.0 / u->base);
+  for (int k = 0; k < 2 * u->base; ++k) h[u->whoff + k] = (float)(sdh * nd(rng));
+}
+
 }  // namespace
 
 extern "C" {
@@ -1212,20 +1229,8 @@ int msg_unet_create(msg_unet **net, int scales, int base_channels, unsigned long
     delete u;
     return ufail(MSG_ERR_HIP, "msg_unet_create: stream");
   }
-  // He initialisation from the seed (the padded input channels stay zero), zero biases
   std::vector<float> h(u->nparams, 0.f);
-  std::mt19937_64 rng(seed);
-  std::normal_distribution<double> nd(0.0, 1.0);
-  for (auto &c : u->convs) {
-    const int cin = c.cin1 + c.cin2;
-    const double sd = std::sqrt(2.0 / (9.0 * c.cin_real));
-    for (int t = 0; t < 9; ++t)
-      for (int o = 0; o < c.cout; ++o)
-        for (int i = 0; i < cin; ++i)
-          h[c.woff + ((long)t * c.cout + o) * cin + i] = (c.in1 != 0 || i < c.cin_real) ? (float)(sd * nd(rng)) : 0.f;
-  }
-  const double sdh = std::sqrt(1.0 / u->base);
-  for (int k = 0; k < 2 * u->base; ++k) h[u->whoff + k] = (float)(sdh * nd(rng));
+  he_init(u, seed, h);
   *net = u;
   return msg_unet_set_params(u, h.data());
 }
