@@ -480,12 +480,88 @@ __device__ __forceinline__ float heat_apply_f(const Get &get, int x, int y, int 
   return hs * lap + u;
 }
 
+// The fine passes' tiles of TX x 16 nodes with a 2-node halo in LDS (TX + 4 columns, 20 rows). A thread keeps
+// one of the TX columns, so its global and LDS addresses, the mirrored neighbours of a border column and
+// the bounds are worked out once and rows differ by constants; the 4 halo columns are a short extra step.
+// (n is a multiple of TX and 16: only halo rows and columns lie outside the grid.) Indexing every cell modulo
+// the halo's width took as many instructions as the sweeps: 8 pairs of 1024^2, the finest level down 59 -> 51 us
+// and up 90 -> 84 us (their memory traffic alone: 29 and 54 us).
+template <int TX>
+struct MgTile {
+  static constexpr int HX = TX + 4, G = 256 / TX;        // halo row length; rows in flight
+  static constexpr int LR = (MG32_HY + G - 1) / G;       // rows per thread: of the halo tile
+  static constexpr int SR = (MG32_HY - 2 + G - 1) / G;   // of the tile + 1
+  static constexpr int NHALO = 4 * MG32_HY;              // cells of the halo columns
+  int tx, g;           // column of the tile, row group
+  int x0, y0, n;
+  int xl, xr;          // LDS columns of the (mirrored) neighbours of column tx
+  int hr, hc, hx;      // the halo cell of this thread (tid < NHALO): row, LDS column, grid column
+  __device__ __forceinline__ MgTile(int tile, int ntx, int n_) : n(n_) {
+    tx = threadIdx.x % TX;
+    g = threadIdx.x / TX;
+    x0 = (tile % ntx) * TX;
+    y0 = (tile / ntx) * MG32_TY;
+    const int gx = x0 + tx, lx = tx + 2;
+    xl = gx > 0 ? lx - 1 : lx + 1;
+    xr = gx < n - 1 ? lx + 1 : lx - 1;
+    hr = threadIdx.x >> 2;
+    const int c = threadIdx.x & 3;
+    hc = c < 2 ? c : TX + c;
+    hx = x0 + hc - 2;
+  }
+  __device__ __forceinline__ bool row_in(int r) const { return (unsigned)(y0 + r - 2) < (unsigned)n; }
+  __device__ __forceinline__ bool halo_in() const {
+    return threadIdx.x < NHALO && (unsigned)hx < (unsigned)n && row_in(hr);
+  }
+  // clamped grid index of halo-tile row r, column of this thread / of its halo cell
+  __device__ __forceinline__ int at(int r) const { return min(max(y0 + r - 2, 0), n - 1) * n + x0 + tx; }
+  __device__ __forceinline__ int halo_at() const {
+    return min(max(y0 + hr - 2, 0), n - 1) * n + min(max(hx, 0), n - 1);
+  }
+};
+
+// One Jacobi sweep x + (rhs - A x) / diag on the tile + 1 (rows 1..18, columns 1..TX+2 of the halo tile), in
+// heat_apply_f's order of operations.
+template <int TX>
+__device__ __forceinline__ void mg_sweep_tile1(const MgTile<TX> &t, const float (*sr)[TX + 4], const float (*sx)[TX + 4],
+                                               float (*out)[TX + 4], float hs, float idg) {
+#pragma clang fp contract(fast)
+  auto cell = [&](int r, int lx, int xl, int xr) {
+    const int gy = t.y0 + r - 2;
+    const int yb = gy > 0 ? r - 1 : r + 1, yt = gy < t.n - 1 ? r + 1 : r - 1;
+    const float u = sx[r][lx];
+    const float lap = ((u - sx[r][xr]) + (u - sx[r][xl])) + ((u - sx[yt][lx]) + (u - sx[yb][lx]));
+    const float au = hs * lap + u;
+    out[r][lx] = (sr[r][lx] - au) * idg + u;
+  };
+#pragma unroll
+  for (int k = 0; k < MgTile<TX>::SR; ++k) {
+    const int r = 1 + t.g * MgTile<TX>::SR + k;
+    if (r < MG32_HY - 1 && t.row_in(r)) cell(r, t.tx + 2, t.xl, t.xr);
+  }
+  // the halo's inner columns: threads of the halo cells with column 1 or TX + 2
+  const int c = threadIdx.x & 3;
+  if ((c == 1 || c == 2) && t.hr >= 1 && t.hr < MG32_HY - 1 && t.halo_in())
+    cell(t.hr, t.hc, t.hx > 0 ? t.hc - 1 : t.hc + 1, t.hx < t.n - 1 ? t.hc + 1 : t.hc - 1);
+}
+
+// A u at a node of the tile (halo-tile row r)
+template <int TX>
+__device__ __forceinline__ float mg_heat_tile(const MgTile<TX> &t, const float (*sx)[TX + 4], int r, float hs) {
+#pragma clang fp contract(fast)
+  const int gy = t.y0 + r - 2, lx = t.tx + 2;
+  const int yb = gy > 0 ? r - 1 : r + 1, yt = gy < t.n - 1 ? r + 1 : r - 1;
+  const float u = sx[r][lx];
+  const float lap = ((u - sx[r][t.xr]) + (u - sx[r][t.xl])) + ((u - sx[yt][lx]) + (u - sx[yb][lx]));
+  return hs * lap + u;
+}
+
 template <int TX>
 __global__ void __launch_bounds__(256)
 k_mg_down_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x2out, float *__restrict__ rhsc, int n,
               const PairState *st, double sigma_default, int ntx, int nty, int nfields) {
 #pragma clang fp contract(fast)
-  constexpr int HX = TX + 4;
+  typedef MgTile<TX> Tile;
   const int tiles = ntx * nty;
   const int wg = xcd_remap(blockIdx.x, tiles * nfields);
   const int field = wg / tiles, tile = wg - field * tiles;
@@ -494,67 +570,50 @@ k_mg_down_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x2o
   float hs, idg;
   level_consts_f(st, pair, sigma_default, n, hs, idg);
 
-  __shared__ float sr[MG32_HY][HX];    // rhs on tile+2
-  __shared__ float s1[MG32_HY][HX];    // x1 on tile+2
-  __shared__ float s2[MG32_HY][HX];    // x2 on tile+1
-  __shared__ float sres[MG32_TY][TX];  // residual on tile
-  const size_t nn = (size_t)n * n;
-  const float *rp = rhs + field * nn;
-  const int x0 = (tile % ntx) * TX, y0 = (tile / ntx) * MG32_TY;
-  const int bx = x0 - 2, by = y0 - 2;
+  __shared__ float sr[MG32_HY][Tile::HX];  // rhs on tile+2
+  __shared__ float s1[MG32_HY][Tile::HX];  // x1 on tile+2
+  __shared__ float s2[MG32_HY][Tile::HX];  // x2 on tile+1
+  __shared__ float sres[MG32_TY][TX];      // residual on tile
+  const Tile t(tile, ntx, n);
+  const float *rp = rhs + field * (size_t)n * n;
   const float sg = negate ? -1.f : 1.f;
 
-  // every load of the halo tile issued before the first is used (clamped indices; cells outside
-  // the grid are not stored), so a workgroup waits for one memory round trip, not one per sweep
-  constexpr int NH = HX * MG32_HY, PER = (NH + 255) / 256;
-  float hv[PER];
+  // every load issued before the first is used (clamped indices; cells outside the grid are not stored)
+  float hv[Tile::LR];
 #pragma unroll
-  for (int r = 0; r < PER; ++r) {
-    const int i = threadIdx.x + 256 * r;
-    const int lx = i % HX, ly = i / HX;
-    const int gx = bx + lx, gy = by + ly;
-    const bool ok = i < NH && gx >= 0 && gy >= 0 && gx < n && gy < n;
-    hv[r] = rp[ok ? gx + gy * n : 0];
-  }
+  for (int k = 0; k < Tile::LR; ++k) hv[k] = rp[t.at(t.g * Tile::LR + k)];
+  const float hh = rp[t.halo_at()];
 #pragma unroll
-  for (int r = 0; r < PER; ++r) {
-    const int i = threadIdx.x + 256 * r;
-    const int lx = i % HX, ly = i / HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (i < NH && gx >= 0 && gy >= 0 && gx < n && gy < n) {
-      const float v = sg * hv[r];
-      sr[ly][lx] = v;
-      s1[ly][lx] = v * idg;  // first Jacobi sweep from zero
+  for (int k = 0; k < Tile::LR; ++k) {
+    const int r = t.g * Tile::LR + k;
+    if (r < MG32_HY && t.row_in(r)) {
+      const float v = sg * hv[k];
+      sr[r][t.tx + 2] = v;
+      s1[r][t.tx + 2] = v * idg;  // first Jacobi sweep from zero
     }
   }
-  __syncthreads();
-  auto get1 = [&](int gx, int gy) { return s1[gy - by][gx - bx]; };
-  for (int i = threadIdx.x; i < HX * MG32_HY; i += 256) {
-    const int lx = i % HX, ly = i / HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (lx >= 1 && ly >= 1 && lx < HX - 1 && ly < MG32_HY - 1 && gx >= 0 && gy >= 0 && gx < n && gy < n)
-      s2[ly][lx] = (sr[ly][lx] - heat_apply_f(get1, gx, gy, n, hs)) * idg + s1[ly][lx];
+  if (t.halo_in()) {
+    const float v = sg * hh;
+    sr[t.hr][t.hc] = v;
+    s1[t.hr][t.hc] = v * idg;
   }
   __syncthreads();
-  auto get2 = [&](int gx, int gy) { return s2[gy - by][gx - bx]; };
-  float *xo = x2out + field * nn;
-  for (int i = threadIdx.x; i < TX * MG32_TY; i += 256) {
-    const int tx = i % TX, ty = i / TX;
-    const int gx = x0 + tx, gy = y0 + ty;
-    if (gx < n && gy < n) {
-      sres[ty][tx] = sr[ty + 2][tx + 2] - heat_apply_f(get2, gx, gy, n, hs);
-      xo[gx + gy * n] = s2[ty + 2][tx + 2];
-    }
+  mg_sweep_tile1<TX>(t, sr, s1, s2, hs, idg);
+  __syncthreads();
+  float *xo = x2out + field * (size_t)n * n + (size_t)t.y0 * n + t.x0 + t.tx;
+#pragma unroll
+  for (int k = 0; k < MG32_TY / Tile::G; ++k) {
+    const int r = t.g + Tile::G * k;
+    sres[r][t.tx] = sr[r + 2][t.tx + 2] - mg_heat_tile<TX>(t, s2, r + 2, hs);
+    xo[(size_t)r * n] = s2[r + 2][t.tx + 2];
   }
   __syncthreads();
   const int nc = n / 2;
-  float *rc = rhsc + field * (size_t)nc * nc;
+  float *rc = rhsc + field * (size_t)nc * nc + (size_t)(t.y0 / 2) * nc + t.x0 / 2;
   for (int i = threadIdx.x; i < (TX / 2) * (MG32_TY / 2); i += 256) {
     const int cx = i % (TX / 2), cy = i / (TX / 2);
-    const int gcx = x0 / 2 + cx, gcy = y0 / 2 + cy;
-    if (gcx < nc && gcy < nc)
-      rc[gcx + gcy * nc] =
-          0.25f * ((sres[2 * cy][2 * cx] + sres[2 * cy][2 * cx + 1]) + (sres[2 * cy + 1][2 * cx] + sres[2 * cy + 1][2 * cx + 1]));
+    rc[(size_t)cy * nc + cx] =
+        0.25f * ((sres[2 * cy][2 * cx] + sres[2 * cy][2 * cx + 1]) + (sres[2 * cy + 1][2 * cx] + sres[2 * cy + 1][2 * cx + 1]));
   }
 }
 
@@ -564,7 +623,7 @@ k_mg_up_f32(const float *__restrict__ x2in, const float *__restrict__ xc, const 
             float *__restrict__ xout, int n, const PairState *st, double sigma_default, int ntx, int nty, int nfields,
             const float *__restrict__ dold, double *__restrict__ nrm_part) {
 #pragma clang fp contract(fast)
-  constexpr int HX = TX + 4;
+  typedef MgTile<TX> Tile;
   const int tiles = ntx * nty;
   const int wg = xcd_remap(blockIdx.x, tiles * nfields);
   const int field = wg / tiles, tile = wg - field * tiles;
@@ -573,90 +632,72 @@ k_mg_up_f32(const float *__restrict__ x2in, const float *__restrict__ xc, const 
   float hs, idg;
   level_consts_f(st, pair, sigma_default, n, hs, idg);
 
-  __shared__ float sx[MG32_HY][HX];  // x on tile+2
-  __shared__ float sr[MG32_HY][HX];  // rhs on tile+1
-  __shared__ float s3[MG32_HY][HX];  // x3 on tile+1
+  __shared__ float sx[MG32_HY][Tile::HX];  // x on tile+2
+  __shared__ float sr[MG32_HY][Tile::HX];  // rhs on tile+2
+  __shared__ float s3[MG32_HY][Tile::HX];  // x3 on tile+1
   __shared__ double red[4 * NORM_TERMS];
+  const Tile t(tile, ntx, n);
   const size_t nn = (size_t)n * n;
   const int nc = n / 2;
   const float *x2p = x2in + field * nn, *rp = rhs + field * nn, *xcp = xc + field * (size_t)nc * nc;
-  const int x0 = (tile % ntx) * TX, y0 = (tile / ntx) * MG32_TY;
-  const int bx = x0 - 2, by = y0 - 2;
   const float sg = negate ? -1.f : 1.f;
-  // the previous direction at this thread's output nodes, loaded now so the load overlaps the sweeps
-  constexpr int OUT_PER_THREAD = TX * MG32_TY / 256;
-  float dprev[OUT_PER_THREAD];
-  if (nrm_part) {  // uniform: every load issued at once, from clamped indices
-#pragma unroll
-    for (int k = 0; k < OUT_PER_THREAD; ++k) {
-      const int i = threadIdx.x + 256 * k;
-      const int gx = x0 + i % TX, gy = y0 + i / TX;
-      const float v = dold[field * nn + ((gx < n && gy < n) ? gx + gy * n : 0)];
-      dprev[k] = (gx < n && gy < n) ? v : 0.f;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < OUT_PER_THREAD; ++k) dprev[k] = 0.f;
-  }
+  const size_t o0 = field * nn + (size_t)t.y0 * n + t.x0 + t.tx;  // this thread's column of the tile
+  constexpr int OUT = MG32_TY / Tile::G;                          // output rows per thread: g + G k
 
-  // every load of the halo tile issued before the first is used (clamped indices; cells outside
-  // the grid are not stored)
-  constexpr int NH = HX * MG32_HY, PER = (NH + 255) / 256;
-  float hx2[PER], hxc[PER], hr[PER];
+  // every load issued before the first is used (clamped indices; cells outside the grid are not stored);
+  // the previous direction at the output nodes among them
+  float dprev[OUT];
 #pragma unroll
-  for (int r = 0; r < PER; ++r) {
-    const int i = threadIdx.x + 256 * r;
-    const int lx = i % HX, ly = i / HX;
-    const int gx = bx + lx, gy = by + ly;
-    const bool ok = i < NH && gx >= 0 && gy >= 0 && gx < n && gy < n;
-    const int gi = ok ? gx + gy * n : 0, ci = ok ? (gx >> 1) + (gy >> 1) * nc : 0;
-    hx2[r] = x2p[gi];
-    hxc[r] = xcp[ci];
-    hr[r] = rp[gi];
+  for (int k = 0; k < OUT; ++k) dprev[k] = 0.f;
+  if (nrm_part) {
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) dprev[k] = dold[o0 + (size_t)(t.g + Tile::G * k) * n];
   }
+  float hx2[Tile::LR], hxc[Tile::LR], hr[Tile::LR];
 #pragma unroll
-  for (int r = 0; r < PER; ++r) {
-    const int i = threadIdx.x + 256 * r;
-    const int lx = i % HX, ly = i / HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (i < NH && gx >= 0 && gy >= 0 && gx < n && gy < n) {
-      sx[ly][lx] = hx2[r] + hxc[r];
-      sr[ly][lx] = sg * hr[r];
+  for (int k = 0; k < Tile::LR; ++k) {
+    const int r = t.g * Tile::LR + k, gi = t.at(r);
+    hx2[k] = x2p[gi];
+    hr[k] = rp[gi];
+    hxc[k] = xcp[(min(max(t.y0 + r - 2, 0), n - 1) >> 1) * nc + ((t.x0 + t.tx) >> 1)];
+  }
+  const int gh = t.halo_at();
+  const float hh2 = x2p[gh], hhr = rp[gh];
+  const float hhc = xcp[(min(max(t.y0 + t.hr - 2, 0), n - 1) >> 1) * nc + (min(max(t.hx, 0), n - 1) >> 1)];
+#pragma unroll
+  for (int k = 0; k < Tile::LR; ++k) {
+    const int r = t.g * Tile::LR + k;
+    if (r < MG32_HY && t.row_in(r)) {
+      sx[r][t.tx + 2] = hx2[k] + hxc[k];
+      sr[r][t.tx + 2] = sg * hr[k];
     }
   }
-  __syncthreads();
-  auto getx = [&](int gx, int gy) { return sx[gy - by][gx - bx]; };
-  for (int i = threadIdx.x; i < HX * MG32_HY; i += 256) {
-    const int lx = i % HX, ly = i / HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (lx >= 1 && ly >= 1 && lx < HX - 1 && ly < MG32_HY - 1 && gx >= 0 && gy >= 0 && gx < n && gy < n)
-      s3[ly][lx] = (sr[ly][lx] - heat_apply_f(getx, gx, gy, n, hs)) * idg + sx[ly][lx];
+  if (t.halo_in()) {
+    sx[t.hr][t.hc] = hh2 + hhc;
+    sr[t.hr][t.hc] = sg * hhr;
   }
   __syncthreads();
-  auto get3 = [&](int gx, int gy) { return s3[gy - by][gx - bx]; };
-  float *xo = xout + field * nn;
+  mg_sweep_tile1<TX>(t, sr, sx, s3, hs, idg);
+  __syncthreads();
   double acc[NORM_TERMS] = {0., 0., 0., 0.};  // <z,z>, <DE,z>, <DE,d_old>, <DE,DE> (DE = the raw input)
 #pragma unroll
-  for (int k = 0; k < OUT_PER_THREAD; ++k) {
-    const int i = threadIdx.x + 256 * k;
-    const int tx = i % TX, ty = i / TX;
-    const int gx = x0 + tx, gy = y0 + ty;
-    if (gx < n && gy < n) {
-      const float o = (sr[ty + 2][tx + 2] - heat_apply_f(get3, gx, gy, n, hs)) * idg + s3[ty + 2][tx + 2];
-      xo[gx + gy * n] = o;
-      if (nrm_part) {
-        const double od = (double)o, de = (double)(sg * sr[ty + 2][tx + 2]);  // the raw input
-        acc[0] += od * od;
-        acc[1] += de * od;
-        acc[2] += de * (double)dprev[k];
-        acc[3] += de * de;
-      }
+  for (int k = 0; k < OUT; ++k) {
+    const int r = t.g + Tile::G * k;
+    const float rv = sr[r + 2][t.tx + 2];
+    const float o = (rv - mg_heat_tile<TX>(t, s3, r + 2, hs)) * idg + s3[r + 2][t.tx + 2];
+    xout[o0 + (size_t)r * n] = o;
+    if (nrm_part) {
+      const double od = (double)o, de = (double)(sg * rv);  // the raw input
+      acc[0] += od * od;
+      acc[1] += de * od;
+      acc[2] += de * (double)dprev[k];
+      acc[3] += de * de;
     }
   }
   if (nrm_part) {
     block_sum_n<NORM_TERMS>(acc, red);
     if (threadIdx.x == 0)
-      for (int t = 0; t < NORM_TERMS; ++t) nrm_part[((size_t)field * NORM_TERMS + t) * tiles + tile] = acc[t];
+      for (int q = 0; q < NORM_TERMS; ++q) nrm_part[((size_t)field * NORM_TERMS + q) * tiles + tile] = acc[q];
   }
 }
 
