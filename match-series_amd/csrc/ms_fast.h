@@ -19,37 +19,15 @@ __device__ __forceinline__ float qpyf(int q) { return (q & 1) ? (float)MSG_QP1 :
 // basis value of dof b at quad point q (compile-time constants once the loops are unrolled)
 __device__ __forceinline__ float bqf(int b, int q) { return (float)bq(b, q); }
 
-// One axis of a deformed quad point: the position e + u in grid units (e the element's lower node)
-// clipped to [0, n-1] as transformAndClipCoord does; `in` is false on a clipped axis. The element
-// index stays in [0, n-2] for every input (NaN included).
-__device__ __forceinline__ void clip_rel(int e, float u, int n, int &el, float &loc, bool &in) {
-  const float lo = -(float)e, hi = (float)(n - 1 - e);
+// One axis of a deformed quad point: the position e + u in grid units (lo = -e, hi = n-1-e relative to the
+// element e) clipped to [0, n-1] as transformAndClipCoord does: `fl` is the element hit relative to e and
+// `loc` the position in it; `in` is false on a clipped axis. The element hit stays in [0, n-2] for every input
+// (med3 takes a NaN to lo); at the upper bound it is the last one, with loc = 1 exactly.
+__device__ __forceinline__ void clip_rel(float u, float lo, float hi, float &fl, float &loc, bool &in) {
   in = (u >= lo) && (u < hi);
-  const float uc = fmaxf(u, lo);  // NaN -> lo
-  const float fl = floorf(uc);
-  if (uc < hi) {
-    el = e + (int)fl;
-    loc = uc - fl;
-  } else {
-    el = n - 2;
-    loc = 1.f;
-  }
-}
-
-struct HitF {
-  int i0;  // lower-left node of the element hit
-  float lx, ly;
-  bool inx, iny;
-};
-
-// quad point of element (ex, ey) at ux, uy grid units from the element's lower node
-__device__ __forceinline__ HitF hit_rel(int ex, int ey, float ux, float uy, int n) {
-  HitF r;
-  int elx, ely;
-  clip_rel(ex, ux, n, elx, r.lx, r.inx);
-  clip_rel(ey, uy, n, ely, r.ly, r.iny);
-  r.i0 = elx + ely * n;
-  return r;
+  const float uc = __builtin_amdgcn_fmed3f(u, lo, hi);
+  fl = fminf(floorf(uc), hi - 1.f);
+  loc = uc - fl;
 }
 
 // Values of the Q1 interpolant of the element's nodal values p at the 4 quad points (q = 2 qx + qy),
@@ -71,22 +49,6 @@ __device__ __forceinline__ void quad_values(const float p[4], float v[4]) {
 // Resource word 3 is the gfx9-family raw-buffer format (32-bit data, no swizzle).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t image_rsrc(const float *p, int count) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), (short)0, count * 4, 0x00020000);
-}
-__device__ __forceinline__ float ld_rsrc(__amdgpu_buffer_rsrc_t r, unsigned idx) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, idx * 4u, 0, 0));
-}
-
-// bilinear value at the hit; t receives the 4 nodal values
-__device__ __forceinline__ float bilin_f(__amdgpu_buffer_rsrc_t T, const HitF &p, int n, float t[4]) {
-#pragma clang fp contract(fast)
-  const unsigned o = (unsigned)p.i0, on = o + (unsigned)n;
-  t[0] = ld_rsrc(T, o);
-  t[1] = ld_rsrc(T, o + 1u);
-  t[2] = ld_rsrc(T, on);
-  t[3] = ld_rsrc(T, on + 1u);
-  const float a = p.lx * (t[1] - t[0]) + t[0];
-  const float b = p.lx * (t[3] - t[2]) + t[2];
-  return p.ly * (b - a) + a;
 }
 
 // a^T K_loc b of the Q1 stiffness matrix in the difference form of stiff_form, as its edge and
@@ -115,18 +77,29 @@ __device__ __forceinline__ void clamp_rel(float u, float lo, float hi, int &off,
   loc = uc - fl;
 }
 
-// bilinear value of T at byte offset vo + (lx, ly) (reads past the image return 0 and meet a weight of
-// 0); the upper row's loads take the row pitch as their scalar offset
-__device__ __forceinline__ float bilin_at(__amdgpu_buffer_rsrc_t T, unsigned vo, int n, float lx, float ly) {
-#pragma clang fp contract(fast)
+// The 4 nodal values of T around byte offset vo (reads past the image return 0); the upper row's loads take
+// the row pitch as their scalar offset.
+__device__ __forceinline__ void gather4(__amdgpu_buffer_rsrc_t T, unsigned vo, int n, float t[4]) {
   const unsigned pitch = (unsigned)n * 4u;
   auto ld = [&](unsigned extra, unsigned so) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(T, vo + extra, so, 0));
   };
-  const float t0 = ld(0u, 0u), t1 = ld(4u, 0u), t2 = ld(0u, pitch), t3 = ld(4u, pitch);
-  const float a = lx * (t1 - t0) + t0;
-  const float b = lx * (t3 - t2) + t2;
+  t[0] = ld(0u, 0u);
+  t[1] = ld(4u, 0u);
+  t[2] = ld(0u, pitch);
+  t[3] = ld(4u, pitch);
+}
+__device__ __forceinline__ float bilin(const float t[4], float lx, float ly) {
+#pragma clang fp contract(fast)
+  const float a = lx * (t[1] - t[0]) + t[0];
+  const float b = lx * (t[3] - t[2]) + t[2];
   return ly * (b - a) + a;
+}
+// bilinear value of T at byte offset vo + (lx, ly) (a value read past the image meets a weight of 0)
+__device__ __forceinline__ float bilin_at(__amdgpu_buffer_rsrc_t T, unsigned vo, int n, float lx, float ly) {
+  float t[4];
+  gather4(T, vo, n, t);
+  return bilin(t, lx, ly);
 }
 
 // ================================================================================================
@@ -344,6 +317,69 @@ k_energy_exact_f32(const float *__restrict__ R, const float *__restrict__ T, con
 // ================================================================================================
 // SSD variation DE = F_SSD + lambda K phi (k_grad<S, DT_SSD> in FP32 arithmetic).
 // ================================================================================================
+// Contributions of one element to its 4 nodes (b = x + 2 y), from its nodal positions f0, f1 and reference
+// values rn: the force cf and 6 K phi, ck, per dof and component.
+template <bool FIDX>
+__device__ __forceinline__ void grad_elem_f(__amdgpu_buffer_rsrc_t Trs, int ex, int ey, int n, float nm1, float wv,
+                                            const float f0[4], const float f1[4], const float rn[4],
+                                            float cf[4][2], float ck[4][2]) {
+#pragma clang fp contract(fast)
+  float nl[4][2], ox4[4], oy4[4], r4[4];
+  quad_values(f0, ox4);
+  quad_values(f1, oy4);
+  quad_values(rn, r4);
+  const float lox = -(float)ex, hix = (float)(n - 1 - ex), loy = -(float)ey, hiy = (float)(n - 1 - ey);
+  const int gbase = ex + ey * n;
+  const float base4 = 4.f * (float)gbase, pitch4 = 4.f * (float)n;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float fx, fy, lx, ly;
+    bool inx, iny;
+    clip_rel(ox4[q] * nm1 + qpxf(q), lox, hix, fx, lx, inx);
+    clip_rel(oy4[q] * nm1 + qpyf(q), loy, hiy, fy, ly, iny);
+    unsigned vo;
+    if constexpr (FIDX)  // 4 (gbase + fx + fy n): integers below 2^26 that are multiples of 4, exact in FP32
+      vo = (unsigned)(fy * pitch4 + (fx * 4.f + base4));
+    else
+      vo = (unsigned)(gbase + (int)fx + (int)fy * n) * 4u;
+    float t4[4];
+    gather4(Trs, vo, n, t4);
+    const float diff = bilin(t4, lx, ly) - r4[q];
+    // gradient of the bilinear T at the hit, in domain units
+    const float ax = t4[1] - t4[0], bx = t4[3] - t4[2];
+    const float ay = t4[2] - t4[0], by = t4[3] - t4[1];
+    const float gx = (ly * (bx - ax) + ax) * nm1;
+    const float gy = (lx * (by - ay) + ay) * nm1;
+    nl[q][0] = inx ? gx * diff : 0.f;
+    nl[q][1] = iny ? gy * diff : 0.f;
+  }
+#pragma unroll
+  for (int dof = 0; dof < 4; ++dof) {
+    float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      a0 += bqf(dof, q) * nl[q][0];
+      a1 += bqf(dof, q) * nl[q][1];
+    }
+    cf[dof][0] = wv * a0;
+    cf[dof][1] = wv * a1;
+  }
+  // 6 K_loc = [4 -1 -1 -2; -1 4 -2 -1; -1 -2 4 -1; -2 -1 -1 4] applied to the element's dofs. Its
+  // rows sum to zero, so row i is sum over j != i of K_ij (f_j - f_i): differences of close values
+  // instead of a sum that cancels to the FP32 ulp of f for smooth fields. The integer weights are
+  // exact; the factor lambda / 6 is applied in FP64 (FP32's 1/6 carries a 3e-8 bias).
+  auto stiff = [&](const float f[4], int c) {
+    const float d01 = f[1] - f[0], d02 = f[2] - f[0], d03 = f[3] - f[0];
+    const float d12 = f[2] - f[1], d13 = f[3] - f[1], d23 = f[3] - f[2];
+    ck[0][c] = -2.f * d03 + (-d02 - d01);
+    ck[1][c] = -d13 + (-2.f * d12 + d01);
+    ck[2][c] = -d23 + (2.f * d12 + d02);
+    ck[3][c] = d23 + (d13 + 2.f * d03);
+  };
+  stiff(f0, 0);
+  stiff(f1, 1);
+}
+
 __global__ void __launch_bounds__(256)
 k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float *__restrict__ phi,
            float *__restrict__ DE, int n, double vol_d, const PairState *st, double lambda_default, int ntx, int nty,
@@ -378,52 +414,15 @@ k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float
       f1[b] = py[g];
       rn[b] = Rp[g];
     }
-    float nl[4][2], ox4[4], oy4[4], r4[4];
-    quad_values(f0, ox4);
-    quad_values(f1, oy4);
-    quad_values(rn, r4);
+    float ef[4][2], ek[4][2];
+    grad_elem_f<true>(Trs, ex, ey, n, nm1, wv, f0, f1, rn, ef, ek);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const HitF hp = hit_rel(ex, ey, ox4[q] * nm1 + qpxf(q), oy4[q] * nm1 + qpyf(q), n);
-      float t4[4];
-      const float diff = bilin_f(Trs, hp, n, t4) - r4[q];
-      // gradient of the bilinear T at the hit, in domain units
-      const float ax = t4[1] - t4[0], bx = t4[3] - t4[2];
-      const float ay = t4[2] - t4[0], by = t4[3] - t4[1];
-      const float gx = (hp.ly * (bx - ax) + ax) * nm1;
-      const float gy = (hp.lx * (by - ay) + ay) * nm1;
-      nl[q][0] = hp.inx ? gx * diff : 0.f;
-      nl[q][1] = hp.iny ? gy * diff : 0.f;
-    }
+    for (int dof = 0; dof < 4; ++dof)
 #pragma unroll
-    for (int dof = 0; dof < 4; ++dof) {
-      float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        a0 += bqf(dof, q) * nl[q][0];
-        a1 += bqf(dof, q) * nl[q][1];
+      for (int c = 0; c < 2; ++c) {
+        cf[dof][c][e] = ef[dof][c];
+        ck[dof][c][e] = ek[dof][c];
       }
-      cf[dof][0][e] = wv * a0;
-      cf[dof][1][e] = wv * a1;
-    }
-    // 6 K_loc = [4 -1 -1 -2; -1 4 -2 -1; -1 -2 4 -1; -2 -1 -1 4] applied to the element's dofs. Its
-    // rows sum to zero, so row i is sum over j != i of K_ij (f_j - f_i): differences of close values
-    // instead of a sum that cancels to the FP32 ulp of f for smooth fields. The integer weights are
-    // exact; the factor lambda / 6 is applied in FP64 (FP32's 1/6 carries a 3e-8 bias).
-    const float kl[4][4] = {{4.f, -1.f, -1.f, -2.f}, {-1.f, 4.f, -2.f, -1.f}, {-1.f, -2.f, 4.f, -1.f},
-                            {-2.f, -1.f, -1.f, 4.f}};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (j == i) continue;
-        s0 += kl[i][j] * (f0[j] - f0[i]);
-        s1 += kl[i][j] * (f1[j] - f1[i]);
-      }
-      ck[i][0][e] = s0;
-      ck[i][1][e] = s1;
-    }
   }
   __syncthreads();
   const int x = x0 + (threadIdx.x % GR_TX), y = y0 + (threadIdx.x / GR_TX);
@@ -445,6 +444,118 @@ k_grad_f32(const float *__restrict__ R, const float *__restrict__ T, const float
   const int i = x + y * n;
   o[i] = (float)(lambda6 * (double)K0 + (double)F0);
   o[nn + i] = (float)(lambda6 * (double)K1 + (double)F1);
+}
+
+// The value of the lane to the left (0 in lane 0)
+__device__ __forceinline__ float lane_left(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+}
+// a + b, never fused with the product that b may be (as where the products pass through LDS)
+__device__ __forceinline__ float add_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+
+// The same variation for launches of GRAD_RUN_NODES nodes and more: a wave takes 64 element columns and the
+// rows of RUN nodes from below to above; a node's contributions from the element column to its left come by a
+// lane shift and those from the row below stay in registers, so there is no LDS and no barrier, node rows are
+// loaded once per element row instead of twice, and of the elements only 1/64 (columns) and 1/RUN (rows)
+// are worked on twice, where the 32 x 8 tiles take 5 passes of a wave for 4 waves of nodes. Same values as
+// k_grad_f32's, bit for bit. Bound by vector arithmetic (312 instructions per element, the tile kernel 417
+// before its clip and offsets took FP32 forms): 8 pairs of 1024^2, 106 us -> 102 us in tiles and 83 us here.
+// A run of 7 beat 4 and 5 (87, 86 us: more rows done twice) and 8 (87 us; 16: 100 us, too few waves at the end).
+// A wave's run is a chain of 8 elements at 1.6 us each, so small launches are faster in tiles: 512^2 6.9 us (runs
+// 12.0), 1024^2 16.4 (18.5), 2 x 1024^2 27.7 (25.1), 4 x 1024^2 49.3 (42.9): runs from 2^21 nodes on (so the
+// tiles never see an image of more than 4096^2, the bound of FIDX).
+constexpr long GRAD_RUN_NODES = 1l << 21;
+constexpr int GRR_TX = 63;  // nodes per wave and row (lane 0 only passes its element on)
+constexpr int GRR_RUN = 7;
+template <int RUN, bool FIDX>
+__global__ void __launch_bounds__(256)
+k_grad_run_f32(const float *__restrict__ R, const float *__restrict__ T, const float *__restrict__ phi,
+               float *__restrict__ DE, int n, double vol_d, const PairState *st, double lambda_default, int ntx,
+               int nty, int npairs) {
+#pragma clang fp contract(fast)
+  const int tiles = ntx * nty;
+  const int wg = xcd_remap(blockIdx.x, tiles * npairs);
+  const int pair = wg / tiles, tile = wg - pair * tiles;
+  if (st && !participates(st[pair])) return;
+  const double lambda6 = (st ? st[pair].lambda : lambda_default) * (1.0 / 6.0);
+
+  const size_t nn = (size_t)n * n;
+  const float *Rp = R + pair * nn, *Tp = T + pair * nn;
+  const __amdgpu_buffer_rsrc_t Trs = image_rsrc(Tp, (int)nn);
+  const float *px = phi + pair * 2 * nn, *py = px + nn;
+  const int lane = threadIdx.x & 63;
+  const int x = (tile % ntx) * GRR_TX - 1 + lane;  // element column, and the node stored by lanes 1 to 63
+  const int y0 = __builtin_amdgcn_readfirstlane(((tile / ntx) * 4 + (threadIdx.x >> 6)) * RUN);
+  if (y0 >= n) return;
+  const float nm1 = (float)(n - 1);
+  const float wv = (float)(0.25 * vol_d);  // quad weight * vol
+  const bool ok = x >= 0 && x < n - 1;
+  const int xa = min(max(x, 0), n - 1), xb = min(xa + 1, n - 1);
+  float *o0 = DE + pair * 2 * nn, *o1 = o0 + nn;
+
+  // slots 0, 1 the lower node row, 2, 3 the upper row, n* the row after it (loaded one element ahead)
+  float f0[4], f1[4], rn[4], g0[2], g1[2], gr[2];
+  auto load_row = [&](int y) {
+    const int r = min(max(y, 0), n - 1) * n;
+    g0[0] = px[r + xa];
+    g0[1] = px[r + xb];
+    g1[0] = py[r + xa];
+    g1[1] = py[r + xb];
+    gr[0] = Rp[r + xa];
+    gr[1] = Rp[r + xb];
+  };
+  auto take_row = [&]() {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      f0[2 + c] = g0[c];
+      f1[2 + c] = g1[c];
+      rn[2 + c] = gr[c];
+    }
+  };
+  load_row(y0 - 1);
+  take_row();
+  load_row(y0);
+  float F[2] = {0.f, 0.f}, K[2] = {0.f, 0.f};  // node (x, ey): the sums of the elements below it
+#pragma unroll 1
+  for (int j = 0; j <= RUN; ++j) {
+    const int ey = y0 - 1 + j;
+    if (ey >= n) break;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      f0[c] = f0[2 + c];
+      f1[c] = f1[2 + c];
+      rn[c] = rn[2 + c];
+    }
+    take_row();
+    load_row(ey + 2);
+    float ef[4][2], ek[4][2];
+    if (ey >= 0 && ey < n - 1 && ok) {
+      grad_elem_f<FIDX>(Trs, x, ey, n, nm1, wv, f0, f1, rn, ef, ek);
+    } else {
+#pragma unroll
+      for (int dof = 0; dof < 4; ++dof)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) ef[dof][c] = ek[dof][c] = 0.f;
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      F[c] = add_rounded(add_rounded(F[c], lane_left(ef[1][c])), ef[0][c]);
+      K[c] = add_rounded(add_rounded(K[c], lane_left(ek[1][c])), ek[0][c]);
+    }
+    if (j > 0 && lane > 0 && x < n) {
+      const int i = x + ey * n;
+      o0[i] = (float)(lambda6 * (double)K[0] + (double)F[0]);
+      o1[i] = (float)(lambda6 * (double)K[1] + (double)F[1]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      F[c] = add_rounded(lane_left(ef[3][c]), ef[2][c]);
+      K[c] = add_rounded(lane_left(ek[3][c]), ek[2][c]);
+    }
+  }
 }
 
 // ================================================================================================

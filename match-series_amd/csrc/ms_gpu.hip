@@ -353,6 +353,23 @@ int launch_energy(const S *R, const S *T, const S *phi, const S *z, const S *dol
   return MSG_OK;
 }
 
+void launch_grad_f32(const float *R, const float *T, const float *phi, float *DE, int n, double vol, const PairState *st,
+                     double lambda, int npairs, hipStream_t s) {
+  if ((long)n * n * npairs >= msg::GRAD_RUN_NODES) {
+    const int ntx = cdiv(n, msg::GRR_TX), nty = cdiv(n, 4 * msg::GRR_RUN);
+    if (n <= 4096)
+      hipLaunchKernelGGL((msg::k_grad_run_f32<msg::GRR_RUN, true>), dim3(ntx * nty * npairs), dim3(256), 0, s, R, T,
+                         phi, DE, n, vol, st, lambda, ntx, nty, npairs);
+    else
+      hipLaunchKernelGGL((msg::k_grad_run_f32<msg::GRR_RUN, false>), dim3(ntx * nty * npairs), dim3(256), 0, s, R, T,
+                         phi, DE, n, vol, st, lambda, ntx, nty, npairs);
+  } else {
+    const int ntx = cdiv(n, msg::GR_TX), nty = cdiv(n, msg::GR_TY);
+    hipLaunchKernelGGL(msg::k_grad_f32, dim3(ntx * nty * npairs), dim3(256), 0, s, R, T, phi, DE, n, vol, st, lambda,
+                       ntx, nty, npairs);
+  }
+}
+
 template <typename S>
 int launch_grad(const S *R, const S *T, const S *phi, S *DE, int n, const PairState *st, double lambda, int npairs,
                 hipStream_t s, int data_term, int npsi = 0, double yreg = 0) {
@@ -373,8 +390,7 @@ int launch_grad(const S *R, const S *T, const S *phi, S *DE, int n, const PairSt
     hipLaunchKernelGGL((msg::k_grad<S, msg::DT_NCC>), dim3(ntx * nty * npairs), dim3(256), 0, s, R, T, phi, DE, n, h,
                        width, st, lambda, ntx, nty, npairs, 0);
   else if constexpr (std::is_same<S, float>::value)
-    hipLaunchKernelGGL(msg::k_grad_f32, dim3(ntx * nty * npairs), dim3(256), 0, s, R, T, phi, DE, n, h * h, st, lambda,
-                       ntx, nty, npairs);
+    launch_grad_f32(R, T, phi, DE, n, h * h, st, lambda, npairs, s);
   else
     hipLaunchKernelGGL((msg::k_grad<S, msg::DT_SSD>), dim3(ntx * nty * npairs), dim3(256), 0, s, R, T, phi, DE, n, h,
                        width, st, lambda, ntx, nty, npairs, 0);

@@ -220,3 +220,37 @@ def test_xshift_row_lengths(gpu, n):
     assert abs(er[0] - orr) <= max(tol, 1e-14) * abs(orr)
     assert np.abs(g[0] - og).max() <= max(100 * tol, 1e-12) * np.abs(og).max()
     assert (g[1] == 0).all()
+
+
+@pytest.mark.parametrize("n,pairs", [(2, 1 << 19), (4, 1 << 17), (64, 513), (128, 128), (512, 8), (1024, 3)])
+def test_f32_gradient_runs_are_the_tiles(gpu, n, pairs):
+    """The FP32 SSD gradient of 2^21 nodes and more (element runs of whole waves) repeats the tiles' operations
+    and order: the same bits as the pairs in smaller launches, with positions inside, on and far outside the
+    domain and a NaN."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    R, T = (torch.rand(pairs, n, n, device="cuda", generator=g) for _ in range(2))
+    phi = torch.randn(pairs, 2, n, n, device="cuda", generator=g) * (4.0 / n)
+    phi[1] = 0.0
+    phi[2 % pairs, 0, n // 2, n // 3] = 1e30
+    phi[0, 1, n - 1, 0] = float("nan")
+    whole = gpu.gradient(R, T, phi, 50.0)
+    step = max(1, ((1 << 21) - 1) // (n * n))
+    for a in range(0, pairs, step):
+        part = gpu.gradient(R[a:a + step].contiguous(), T[a:a + step].contiguous(), phi[a:a + step].contiguous(), 50.0)
+        assert torch.equal(part.view(torch.int32), whole[a:a + step].contiguous().view(torch.int32)) or torch.equal(
+            torch.nan_to_num(part), torch.nan_to_num(whole[a:a + step]))
+
+
+def test_f32_gradient_above_4096(gpu):
+    """Above 4096^2 the gather offsets are integers. Smooth images (period 400 px or more): the FP32 differences
+    of neighbouring values carry 2^-24 / (2 pi / 400) = 4e-6 relative, so 2e-5 in L2 against the FP64 pass on
+    the same stored values."""
+    n = 8192
+    y = torch.linspace(0, 1, n, device="cuda", dtype=torch.float64)[:, None]
+    x = torch.linspace(0, 1, n, device="cuda", dtype=torch.float64)[None, :]
+    R = (0.5 + 0.4 * torch.sin(100 * x + 60 * y)).float()[None]
+    T = (0.5 + 0.4 * torch.cos(90 * x - 110 * y)).float()[None]
+    phi = torch.stack([1e-3 * torch.sin(9 * x + 4 * y), 1e-3 * torch.cos(5 * x - 8 * y)]).float()[None]
+    a = gpu.gradient(R, T, phi, 0.0).double()
+    b = gpu.gradient(R.double(), T.double(), phi.double(), 0.0)
+    assert ((a - b).norm() / b.norm()).item() < 2e-5
