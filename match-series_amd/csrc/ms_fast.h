@@ -818,7 +818,6 @@ k_mg_up_f32(const float *__restrict__ x2in, const float *__restrict__ xc, const 
 // it is formed and the prolongation is read on the fly by the first sweep of the up leg, so a level
 // costs 3 barriers down and 2 up. Node coordinates come from shifts and masks (a division by the
 // runtime level size would cost an integer-division sequence per node).
-constexpr int MGC_THREADS = 1024;
 constexpr int MGC_MAXL_F32 = 6;
 
 __global__ void __launch_bounds__(MGC_THREADS)
@@ -909,14 +908,8 @@ k_mg_coarse_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x
     sync();
   };
   auto block_sync = [] { __syncthreads(); };
-  // Levels of at most 64 nodes run in wave 0 alone: its instructions, LDS accesses included, execute
-  // in order for all lanes, so a wavefront fence (a compiler barrier) replaces the workgroup barrier.
-  auto wave_sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
-  constexpr int WAVE_LEVELS = 3;  // 8x8 nodes and below
+  auto wave_sync = [] { mgc_wave_sync(); };
+  constexpr int WAVE_LEVELS = MGC_WAVE_LEVELS;
   for (int l = L; l > WAVE_LEVELS; --l) down_level(l, (int)threadIdx.x, MGC_THREADS, block_sync);
   if (threadIdx.x < 64) {
     const int lw = L < WAVE_LEVELS ? L : WAVE_LEVELS;

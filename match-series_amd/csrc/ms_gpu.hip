@@ -484,7 +484,7 @@ void mg_coarse(dim3 g, hipStream_t s, const S *rhs, int negate, S *xout, int L, 
     hipLaunchKernelGGL(msg::k_mg_coarse_f32, g, dim3(msg::MGC_THREADS), 0, s, rhs, negate, xout, L, st, sigma, nfields,
                        dold, nrm_part);
   else
-    hipLaunchKernelGGL((msg::k_mg_coarse<S>), g, dim3(256), 0, s, rhs, negate, xout, L, st, sigma, nfields, dold,
+    hipLaunchKernelGGL((msg::k_mg_coarse<S>), g, dim3(msg::MGC_THREADS), 0, s, rhs, negate, xout, L, st, sigma, nfields, dold,
                        nrm_part);
 }
 template <typename S>
