@@ -591,46 +591,6 @@ __device__ __forceinline__ float heat_apply_f(const Get &get, int x, int y, int 
   return hs * lap + u;
 }
 
-// The fine passes' tiles of TX x 16 nodes with a 2-node halo in LDS (TX + 4 columns, 20 rows). A thread keeps
-// one of the TX columns, so its global and LDS addresses, the mirrored neighbours of a border column and
-// the bounds are worked out once and rows differ by constants; the 4 halo columns are a short extra step.
-// (n is a multiple of TX and 16: only halo rows and columns lie outside the grid.) Indexing every cell modulo
-// the halo's width took as many instructions as the sweeps: 8 pairs of 1024^2, the finest level down 59 -> 51 us
-// and up 90 -> 84 us (their memory traffic alone: 29 and 54 us).
-template <int TX>
-struct MgTile {
-  static constexpr int HX = TX + 4, G = 256 / TX;        // halo row length; rows in flight
-  static constexpr int LR = (MG32_HY + G - 1) / G;       // rows per thread: of the halo tile
-  static constexpr int SR = (MG32_HY - 2 + G - 1) / G;   // of the tile + 1
-  static constexpr int NHALO = 4 * MG32_HY;              // cells of the halo columns
-  int tx, g;           // column of the tile, row group
-  int x0, y0, n;
-  int xl, xr;          // LDS columns of the (mirrored) neighbours of column tx
-  int hr, hc, hx;      // the halo cell of this thread (tid < NHALO): row, LDS column, grid column
-  __device__ __forceinline__ MgTile(int tile, int ntx, int n_) : n(n_) {
-    tx = threadIdx.x % TX;
-    g = threadIdx.x / TX;
-    x0 = (tile % ntx) * TX;
-    y0 = (tile / ntx) * MG32_TY;
-    const int gx = x0 + tx, lx = tx + 2;
-    xl = gx > 0 ? lx - 1 : lx + 1;
-    xr = gx < n - 1 ? lx + 1 : lx - 1;
-    hr = threadIdx.x >> 2;
-    const int c = threadIdx.x & 3;
-    hc = c < 2 ? c : TX + c;
-    hx = x0 + hc - 2;
-  }
-  __device__ __forceinline__ bool row_in(int r) const { return (unsigned)(y0 + r - 2) < (unsigned)n; }
-  __device__ __forceinline__ bool halo_in() const {
-    return threadIdx.x < NHALO && (unsigned)hx < (unsigned)n && row_in(hr);
-  }
-  // clamped grid index of halo-tile row r, column of this thread / of its halo cell
-  __device__ __forceinline__ int at(int r) const { return min(max(y0 + r - 2, 0), n - 1) * n + x0 + tx; }
-  __device__ __forceinline__ int halo_at() const {
-    return min(max(y0 + hr - 2, 0), n - 1) * n + min(max(hx, 0), n - 1);
-  }
-};
-
 // One Jacobi sweep x + (rhs - A x) / diag on the tile + 1 (rows 1..18, columns 1..TX+2 of the halo tile), in
 // heat_apply_f's order of operations.
 template <int TX>
@@ -648,11 +608,11 @@ __device__ __forceinline__ void mg_sweep_tile1(const MgTile<TX> &t, const float 
 #pragma unroll
   for (int k = 0; k < MgTile<TX>::SR; ++k) {
     const int r = 1 + t.g * MgTile<TX>::SR + k;
-    if (r < MG32_HY - 1 && t.row_in(r)) cell(r, t.tx + 2, t.xl, t.xr);
+    if (r < MG_HY - 1 && t.row_in(r)) cell(r, t.tx + 2, t.xl, t.xr);
   }
   // the halo's inner columns: threads of the halo cells with column 1 or TX + 2
   const int c = threadIdx.x & 3;
-  if ((c == 1 || c == 2) && t.hr >= 1 && t.hr < MG32_HY - 1 && t.halo_in())
+  if ((c == 1 || c == 2) && t.hr >= 1 && t.hr < MG_HY - 1 && t.halo_in())
     cell(t.hr, t.hc, t.hx > 0 ? t.hc - 1 : t.hc + 1, t.hx < t.n - 1 ? t.hc + 1 : t.hc - 1);
 }
 
@@ -681,9 +641,9 @@ k_mg_down_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x2o
   float hs, idg;
   level_consts_f(st, pair, sigma_default, n, hs, idg);
 
-  __shared__ float sr[MG32_HY][Tile::HX];  // rhs on tile+2
-  __shared__ float s1[MG32_HY][Tile::HX];  // x1 on tile+2
-  __shared__ float s2[MG32_HY][Tile::HX];  // x2 on tile+1
+  __shared__ float sr[MG_HY][Tile::HX];  // rhs on tile+2
+  __shared__ float s1[MG_HY][Tile::HX];  // x1 on tile+2
+  __shared__ float s2[MG_HY][Tile::HX];  // x2 on tile+1
   __shared__ float sres[MG32_TY][TX];      // residual on tile
   const Tile t(tile, ntx, n);
   const float *rp = rhs + field * (size_t)n * n;
@@ -697,7 +657,7 @@ k_mg_down_f32(const float *__restrict__ rhs, int negate, float *__restrict__ x2o
 #pragma unroll
   for (int k = 0; k < Tile::LR; ++k) {
     const int r = t.g * Tile::LR + k;
-    if (r < MG32_HY && t.row_in(r)) {
+    if (r < MG_HY && t.row_in(r)) {
       const float v = sg * hv[k];
       sr[r][t.tx + 2] = v;
       s1[r][t.tx + 2] = v * idg;  // first Jacobi sweep from zero
@@ -743,9 +703,9 @@ k_mg_up_f32(const float *__restrict__ x2in, const float *__restrict__ xc, const 
   float hs, idg;
   level_consts_f(st, pair, sigma_default, n, hs, idg);
 
-  __shared__ float sx[MG32_HY][Tile::HX];  // x on tile+2
-  __shared__ float sr[MG32_HY][Tile::HX];  // rhs on tile+2
-  __shared__ float s3[MG32_HY][Tile::HX];  // x3 on tile+1
+  __shared__ float sx[MG_HY][Tile::HX];  // x on tile+2
+  __shared__ float sr[MG_HY][Tile::HX];  // rhs on tile+2
+  __shared__ float s3[MG_HY][Tile::HX];  // x3 on tile+1
   __shared__ double red[4 * NORM_TERMS];
   const Tile t(tile, ntx, n);
   const size_t nn = (size_t)n * n;
@@ -778,7 +738,7 @@ k_mg_up_f32(const float *__restrict__ x2in, const float *__restrict__ xc, const 
 #pragma unroll
   for (int k = 0; k < Tile::LR; ++k) {
     const int r = t.g * Tile::LR + k;
-    if (r < MG32_HY && t.row_in(r)) {
+    if (r < MG_HY && t.row_in(r)) {
       sx[r][t.tx + 2] = hx2[k] + hxc[k];
       sr[r][t.tx + 2] = sg * hr[k];
     }

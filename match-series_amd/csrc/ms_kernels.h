@@ -1158,11 +1158,11 @@ k_grad(const S *__restrict__ R, const S *__restrict__ T, const S *__restrict__ p
 // correction, then two Jacobi sweeps. Tiles with a 2-node halo live in LDS.
 // ================================================================================================
 constexpr int MG_TX = 32, MG_TY = 16;
-constexpr int MG_HX = MG_TX + 4, MG_HY = MG_TY + 4;
+constexpr int MG_HY = MG_TY + 4;
 // FP32 fields: tiles of 64 x 16 nodes (4 per thread) on levels of 1024^2 and above -- 512 workgroups
 // per field at 1024^2, resident at once, and a halo of 1.33x the tile instead of 1.41x -- and of
 // 32 x 16 below, where a workgroup's latency, not the level's traffic, sets the pass's time.
-constexpr int MG32_TY = 16, MG32_HY = MG32_TY + 4;
+constexpr int MG32_TY = MG_TY;
 constexpr int MG32_TX_WIDE = 64, MG32_WIDE_FROM = 1024;
 
 __device__ __forceinline__ void level_consts(const PairState *st, int pair, double sigma_default, int n, double &hs,
@@ -1174,10 +1174,88 @@ __device__ __forceinline__ void level_consts(const PairState *st, int pair, doub
   diag = make_div(1 + 4 * tau * s);
 }
 
+// The fine passes' tiles of TX x 16 nodes with a 2-node halo in LDS (TX + 4 columns, 20 rows). A thread keeps
+// one of the TX columns, so its global and LDS addresses, the mirrored neighbours of a border column and
+// the bounds are worked out once and rows differ by constants; the 4 halo columns are a short extra step.
+// (n is a multiple of TX and 16: only halo rows and columns lie outside the grid.) Indexing every cell modulo
+// the halo's width took as many instructions as the sweeps: 8 pairs of 1024^2, the finest level down 59 -> 51 us
+// and up 90 -> 84 us (their memory traffic alone: 29 and 54 us); FP64, 2 pairs of 1024^2, where away from the
+// grid's border heat_apply's cases go too, 29 -> 22.6 and 43 -> 39 us.
+template <int TX>
+struct MgTile {
+  static constexpr int HX = TX + 4, G = 256 / TX;        // halo row length; rows in flight
+  static constexpr int LR = (MG_HY + G - 1) / G;       // rows per thread: of the halo tile
+  static constexpr int SR = (MG_HY - 2 + G - 1) / G;   // of the tile + 1
+  static constexpr int NHALO = 4 * MG_HY;              // cells of the halo columns
+  int tx, g;           // column of the tile, row group
+  int x0, y0, n;
+  int xl, xr;          // LDS columns of the (mirrored) neighbours of column tx
+  int hr, hc, hx;      // the halo cell of this thread (tid < NHALO): row, LDS column, grid column
+  __device__ __forceinline__ MgTile(int tile, int ntx, int n_) : n(n_) {
+    tx = threadIdx.x % TX;
+    g = threadIdx.x / TX;
+    x0 = (tile % ntx) * TX;
+    y0 = (tile / ntx) * MG32_TY;
+    const int gx = x0 + tx, lx = tx + 2;
+    xl = gx > 0 ? lx - 1 : lx + 1;
+    xr = gx < n - 1 ? lx + 1 : lx - 1;
+    hr = threadIdx.x >> 2;
+    const int c = threadIdx.x & 3;
+    hc = c < 2 ? c : TX + c;
+    hx = x0 + hc - 2;
+  }
+  // no halo cell outside the grid, nor on its border (uniform)
+  __device__ __forceinline__ bool inner() const { return x0 > 0 && y0 > 0 && x0 + TX < n && y0 + MG_TY < n; }
+  __device__ __forceinline__ bool row_in(int r) const { return (unsigned)(y0 + r - 2) < (unsigned)n; }
+  __device__ __forceinline__ bool halo_in() const {
+    return threadIdx.x < NHALO && (unsigned)hx < (unsigned)n && row_in(hr);
+  }
+  // clamped grid index of halo-tile row r, column of this thread / of its halo cell
+  __device__ __forceinline__ int at(int r) const { return min(max(y0 + r - 2, 0), n - 1) * n + x0 + tx; }
+  __device__ __forceinline__ int halo_at() const {
+    return min(max(y0 + hr - 2, 0), n - 1) * n + min(max(hx, 0), n - 1);
+  }
+};
+
+// A u at row r, LDS column lx of a halo tile of the FP64 passes: on tiles away from the grid's border
+// (INNER, uniform) without heat_apply's cases.
+template <bool INNER, int TX>
+__device__ __forceinline__ double heat_at(const MgTile<TX> &t, const double (*u)[TX + 4], int r, int lx, double hs) {
+  if constexpr (INNER) {
+    const double c = u[r][lx];
+    double b = 0.0;
+    b -= u[r][lx + 1];
+    b -= u[r][lx - 1];
+    b -= u[r + 1][lx];
+    b -= u[r - 1][lx];
+    return c + hs * (c * 4 + b);
+  } else {
+    auto get = [&](int gx, int gy) { return u[gy - t.y0 + 2][gx - t.x0 + 2]; };
+    return heat_apply(get, t.x0 + lx - 2, t.y0 + r - 2, t.n, hs);
+  }
+}
+// One Jacobi sweep x + (rhs - A x) / diag on the tile + 1 (rows 1..18, columns 1..TX+2 of the halo tile).
+template <bool INNER, int TX>
+__device__ __forceinline__ void sweep_tile1(const MgTile<TX> &t, const double (*sr)[TX + 4], const double (*sx)[TX + 4],
+                                            double (*out)[TX + 4], double hs, const Div &diag) {
+  auto cell = [&](int r, int lx) {
+    const double v = sr[r][lx] - heat_at<INNER>(t, sx, r, lx, hs);
+    out[r][lx] = sx[r][lx] + 1.0 * v / diag;
+  };
+#pragma unroll
+  for (int k = 0; k < MgTile<TX>::SR; ++k) {
+    const int r = 1 + t.g * MgTile<TX>::SR + k;
+    if (r < MG_HY - 1 && (INNER || t.row_in(r))) cell(r, t.tx + 2);
+  }
+  const int c = threadIdx.x & 3;
+  if ((c == 1 || c == 2) && t.hr >= 1 && t.hr < MG_HY - 1 && (INNER || t.halo_in())) cell(t.hr, t.hc);
+}
+
 template <typename S>
 __global__ void __launch_bounds__(256)
 k_mg_down(const S *__restrict__ rhs, int negate, S *__restrict__ x2out, S *__restrict__ rhsc, int n,
           const PairState *st, double sigma_default, int ntx, int nty, int nfields) {
+  typedef MgTile<MG_TX> Tile;
   const int tiles = ntx * nty;
   const int wg = xcd_remap(blockIdx.x, tiles * nfields);
   const int field = wg / tiles, tile = wg - field * tiles;
@@ -1187,62 +1265,65 @@ k_mg_down(const S *__restrict__ rhs, int negate, S *__restrict__ x2out, S *__res
   Div diag;
   level_consts(st, pair, sigma_default, n, hs, diag);
 
-  __shared__ double sr[MG_HY][MG_HX];   // rhs on tile+2
-  __shared__ double s1[MG_HY][MG_HX];   // x1 on tile+2
-  __shared__ double s2[MG_HY][MG_HX];   // x2 on tile+1
-  __shared__ double sres[MG_TY][MG_TX]; // residual on tile
-  const size_t nn = (size_t)n * n;
-  const S *rp = rhs + field * nn;
-  const int x0 = (tile % ntx) * MG_TX, y0 = (tile / ntx) * MG_TY;
-  const int bx = x0 - 2, by = y0 - 2;  // LDS origin
+  __shared__ double sr[MG_HY][Tile::HX];  // rhs on tile+2
+  __shared__ double s1[MG_HY][Tile::HX];  // x1 on tile+2, then the residual on the tile
+  __shared__ double s2[MG_HY][Tile::HX];  // x2 on tile+1
+  const Tile t(tile, ntx, n);
+  const S *rp = rhs + field * (size_t)n * n;
 
-  for (int i = threadIdx.x; i < MG_HX * MG_HY; i += 256) {
-    const int lx = i % MG_HX, ly = i / MG_HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (gx >= 0 && gy >= 0 && gx < n && gy < n) {
-      double v = ld(rp, gx + gy * n);
-      if (negate) v = -v;
-      sr[ly][lx] = v;
-      s1[ly][lx] = v / diag;  // 0 + (1.0 * (rhs - A 0)) / diag
+  // every load issued before the first is used (clamped indices; cells outside the grid are not stored)
+  double hv[Tile::LR];
+#pragma unroll
+  for (int k = 0; k < Tile::LR; ++k) hv[k] = ld(rp, t.at(t.g * Tile::LR + k));
+  const double hh = ld(rp, t.halo_at());
+#pragma unroll
+  for (int k = 0; k < Tile::LR; ++k) {
+    const int r = t.g * Tile::LR + k;
+    if (r < MG_HY && t.row_in(r)) {
+      const double v = negate ? -hv[k] : hv[k];
+      sr[r][t.tx + 2] = v;
+      s1[r][t.tx + 2] = v / diag;  // 0 + (1.0 * (rhs - A 0)) / diag
     }
   }
-  __syncthreads();
-  auto get1 = [&](int gx, int gy) { return s1[gy - by][gx - bx]; };
-  for (int i = threadIdx.x; i < MG_HX * MG_HY; i += 256) {
-    const int lx = i % MG_HX, ly = i / MG_HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (lx >= 1 && ly >= 1 && lx < MG_HX - 1 && ly < MG_HY - 1 && gx >= 0 && gy >= 0 && gx < n && gy < n) {
-      const double ax = heat_apply(get1, gx, gy, n, hs);
-      const double v = sr[ly][lx] - ax;
-      s2[ly][lx] = s1[ly][lx] + 1.0 * v / diag;
-    }
+  if (t.halo_in()) {
+    const double v = negate ? -hh : hh;
+    sr[t.hr][t.hc] = v;
+    s1[t.hr][t.hc] = v / diag;
   }
   __syncthreads();
-  auto get2 = [&](int gx, int gy) { return s2[gy - by][gx - bx]; };
-  S *xo = x2out + field * nn;
-  for (int i = threadIdx.x; i < MG_TX * MG_TY; i += 256) {
-    const int tx = i % MG_TX, ty = i / MG_TX;
-    const int gx = x0 + tx, gy = y0 + ty;
-    if (gx < n && gy < n) {
-      const double ax = heat_apply(get2, gx, gy, n, hs);
-      sres[ty][tx] = sr[ty + 2][tx + 2] - ax;
-      xo[gx + gy * n] = static_cast<S>(s2[ty + 2][tx + 2]);
+  double res[MG_TY / Tile::G];
+  auto sweeps = [&](auto inner) {
+    constexpr bool INNER = decltype(inner)::value;
+    sweep_tile1<INNER>(t, sr, s1, s2, hs, diag);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < MG_TY / Tile::G; ++k) {
+      const int r = t.g + Tile::G * k + 2;
+      res[k] = sr[r][t.tx + 2] - heat_at<INNER>(t, s2, r, t.tx + 2, hs);
     }
+  };
+  if (t.inner())
+    sweeps(std::true_type());
+  else
+    sweeps(std::false_type());
+  S *xo = x2out + field * (size_t)n * n + (size_t)t.y0 * n + t.x0 + t.tx;
+#pragma unroll
+  for (int k = 0; k < MG_TY / Tile::G; ++k) {
+    const int r = t.g + Tile::G * k;
+    s1[r][t.tx] = res[k];
+    xo[(size_t)r * n] = static_cast<S>(s2[r + 2][t.tx + 2]);
   }
   __syncthreads();
   const int nc = n / 2;
-  S *rc = rhsc + field * (size_t)nc * nc;
+  S *rc = rhsc + field * (size_t)nc * nc + (size_t)(t.y0 / 2) * nc + t.x0 / 2;
   for (int i = threadIdx.x; i < (MG_TX / 2) * (MG_TY / 2); i += 256) {
     const int cx = i % (MG_TX / 2), cy = i / (MG_TX / 2);
-    const int gcx = x0 / 2 + cx, gcy = y0 / 2 + cy;
-    if (gcx < nc && gcy < nc) {
-      double v = 0;
-      v += sres[2 * cy][2 * cx];
-      v += sres[2 * cy][2 * cx + 1];
-      v += sres[2 * cy + 1][2 * cx];
-      v += sres[2 * cy + 1][2 * cx + 1];
-      rc[gcx + gcy * nc] = static_cast<S>((1.0 / 4.0) * v);
-    }
+    double v = 0;
+    v += s1[2 * cy][2 * cx];
+    v += s1[2 * cy][2 * cx + 1];
+    v += s1[2 * cy + 1][2 * cx];
+    v += s1[2 * cy + 1][2 * cx + 1];
+    rc[(size_t)cy * nc + cx] = static_cast<S>((1.0 / 4.0) * v);
   }
 }
 
@@ -1251,6 +1332,7 @@ __global__ void __launch_bounds__(256)
 k_mg_up(const S *__restrict__ x2in, const S *__restrict__ xc, const S *__restrict__ rhs, int negate,
         S *__restrict__ xout, int n, const PairState *st, double sigma_default, int ntx, int nty,
         int nfields, const S *__restrict__ dold, double *__restrict__ nrm_part) {
+  typedef MgTile<MG_TX> Tile;
   const int tiles = ntx * nty;
   const int wg = xcd_remap(blockIdx.x, tiles * nfields);
   const int field = wg / tiles, tile = wg - field * tiles;
@@ -1260,61 +1342,77 @@ k_mg_up(const S *__restrict__ x2in, const S *__restrict__ xc, const S *__restric
   Div diag;
   level_consts(st, pair, sigma_default, n, hs, diag);
 
-  __shared__ double sx[MG_HY][MG_HX];  // x on tile+2
-  __shared__ double sr[MG_HY][MG_HX];  // rhs on tile+1
-  __shared__ double s3[MG_HY][MG_HX];  // x3 on tile+1
+  __shared__ double sx[MG_HY][Tile::HX];  // x on tile+2
+  __shared__ double sr[MG_HY][Tile::HX];  // rhs on tile+2
+  __shared__ double s3[MG_HY][Tile::HX];  // x3 on tile+1
   __shared__ double red[4 * NORM_TERMS];
+  const Tile t(tile, ntx, n);
   const size_t nn = (size_t)n * n;
   const int nc = n / 2;
   const S *x2p = x2in + field * nn, *rp = rhs + field * nn, *xcp = xc + field * (size_t)nc * nc;
-  const int x0 = (tile % ntx) * MG_TX, y0 = (tile / ntx) * MG_TY;
-  const int bx = x0 - 2, by = y0 - 2;
+  const size_t o0 = field * nn + (size_t)t.y0 * n + t.x0 + t.tx;  // this thread's column of the tile
+  constexpr int OUT = MG_TY / Tile::G;                            // output rows per thread: g + G k
 
-  for (int i = threadIdx.x; i < MG_HX * MG_HY; i += 256) {
-    const int lx = i % MG_HX, ly = i / MG_HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (gx >= 0 && gy >= 0 && gx < n && gy < n) {
-      sx[ly][lx] = ld(x2p, gx + gy * n) + ld(xcp, (gx >> 1) + (gy >> 1) * nc);
-      double v = ld(rp, gx + gy * n);
-      sr[ly][lx] = negate ? -v : v;
+  // every load issued before the first is used (clamped indices; cells outside the grid are not stored);
+  // the previous direction at the output nodes among them
+  double dprev[OUT];
+  if (nrm_part) {
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) dprev[k] = ld(dold, o0 + (size_t)(t.g + Tile::G * k) * n);
+  }
+  double hx2[Tile::LR], hxc[Tile::LR], hr[Tile::LR];
+#pragma unroll
+  for (int k = 0; k < Tile::LR; ++k) {
+    const int r = t.g * Tile::LR + k, gi = t.at(r);
+    hx2[k] = ld(x2p, gi);
+    hr[k] = ld(rp, gi);
+    hxc[k] = ld(xcp, (min(max(t.y0 + r - 2, 0), n - 1) >> 1) * nc + ((t.x0 + t.tx) >> 1));
+  }
+  const int gh = t.halo_at();
+  const double hh2 = ld(x2p, gh), hhr = ld(rp, gh);
+  const double hhc = ld(xcp, (min(max(t.y0 + t.hr - 2, 0), n - 1) >> 1) * nc + (min(max(t.hx, 0), n - 1) >> 1));
+#pragma unroll
+  for (int k = 0; k < Tile::LR; ++k) {
+    const int r = t.g * Tile::LR + k;
+    if (r < MG_HY && t.row_in(r)) {
+      sx[r][t.tx + 2] = hx2[k] + hxc[k];
+      sr[r][t.tx + 2] = negate ? -hr[k] : hr[k];
     }
   }
-  __syncthreads();
-  auto getx = [&](int gx, int gy) { return sx[gy - by][gx - bx]; };
-  for (int i = threadIdx.x; i < MG_HX * MG_HY; i += 256) {
-    const int lx = i % MG_HX, ly = i / MG_HX;
-    const int gx = bx + lx, gy = by + ly;
-    if (lx >= 1 && ly >= 1 && lx < MG_HX - 1 && ly < MG_HY - 1 && gx >= 0 && gy >= 0 && gx < n && gy < n) {
-      const double ax = heat_apply(getx, gx, gy, n, hs);
-      const double v = sr[ly][lx] - ax;
-      s3[ly][lx] = sx[ly][lx] + 1.0 * v / diag;
-    }
+  if (t.halo_in()) {
+    sx[t.hr][t.hc] = hh2 + hhc;
+    sr[t.hr][t.hc] = negate ? -hhr : hhr;
   }
   __syncthreads();
-  auto get3 = [&](int gx, int gy) { return s3[gy - by][gx - bx]; };
-  S *xo = xout + field * nn;
   double acc[NORM_TERMS] = {0., 0., 0., 0.};  // <z,z>, <DE,z>, <DE,d_old>, <DE,DE> (DE = the raw input)
-  for (int i = threadIdx.x; i < MG_TX * MG_TY; i += 256) {
-    const int tx = i % MG_TX, ty = i / MG_TX;
-    const int gx = x0 + tx, gy = y0 + ty;
-    if (gx < n && gy < n) {
-      const double ax = heat_apply(get3, gx, gy, n, hs);
-      const double v = sr[ty + 2][tx + 2] - ax;
-      const S o = static_cast<S>(s3[ty + 2][tx + 2] + 1.0 * v / diag);
-      xo[gx + gy * n] = o;
+  auto sweeps = [&](auto inner) {
+    constexpr bool INNER = decltype(inner)::value;
+    sweep_tile1<INNER>(t, sr, sx, s3, hs, diag);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) {
+      const int r = t.g + Tile::G * k;
+      const double b = sr[r + 2][t.tx + 2];
+      const double v = b - heat_at<INNER>(t, s3, r + 2, t.tx + 2, hs);
+      const S o = static_cast<S>(s3[r + 2][t.tx + 2] + 1.0 * v / diag);
+      xout[o0 + (size_t)r * n] = o;
       if (nrm_part) {
-        const double od = static_cast<double>(o), de = ld(rp, gx + gy * n);
+        const double od = static_cast<double>(o), de = negate ? -b : b;
         acc[0] += od * od;
         acc[1] += de * od;
-        acc[2] += de * ld(dold + field * nn, gx + gy * n);
+        acc[2] += de * dprev[k];
         acc[3] += de * de;
       }
     }
-  }
+  };
+  if (t.inner())
+    sweeps(std::true_type());
+  else
+    sweeps(std::false_type());
   if (nrm_part) {
     block_sum_n<NORM_TERMS>(acc, red);
     if (threadIdx.x == 0)
-      for (int t = 0; t < NORM_TERMS; ++t) nrm_part[((size_t)field * NORM_TERMS + t) * tiles + tile] = acc[t];
+      for (int q = 0; q < NORM_TERMS; ++q) nrm_part[((size_t)field * NORM_TERMS + q) * tiles + tile] = acc[q];
   }
 }
 
