@@ -1179,8 +1179,8 @@ __device__ __forceinline__ void level_consts(const PairState *st, int pair, doub
 // the bounds are worked out once and rows differ by constants; the 4 halo columns are a short extra step.
 // (n is a multiple of TX and 16: only halo rows and columns lie outside the grid.) Indexing every cell modulo
 // the halo's width took as many instructions as the sweeps: 8 pairs of 1024^2, the finest level down 59 -> 51 us
-// and up 90 -> 84 us (their memory traffic alone: 29 and 54 us); FP64, 2 pairs of 1024^2, where away from the
-// grid's border heat_apply's cases go too, 29 -> 22.6 and 43 -> 39 us.
+// and up 90 -> 84 us (their memory traffic alone: 29 and 54 us). FP64, 2 pairs of 1024^2, where the tiles away
+// from the grid's border skip heat_apply's cases too, over a solve's launches: down 23.6 -> 18.5, up 29.6 -> 28.0 us.
 template <int TX>
 struct MgTile {
   static constexpr int HX = TX + 4, G = 256 / TX;        // halo row length; rows in flight
