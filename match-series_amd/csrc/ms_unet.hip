@@ -506,11 +506,44 @@ k_conv3x3_wgrad(ConvIn in, const bf16 *__restrict__ dz, float *__restrict__ part
   }
 }
 
-// dw[i] = sum over chunks of part[chunk][i]: a workgroup takes 64 elements, its 4 waves every fourth chunk
-// in order (8 loads in flight each), their sums added in order. (One thread per element over all chunks:
-// 188 us per training step of 8 pairs of 256^2; so: 111 us, of more partial sums.)
+// out[c] = sum over rows r of part[r * stride + off(c)], one workgroup per column c: each thread sums
+// the rows r = t, t + 256, ... in order, then a fixed tree over the 256 threads (deterministic).
+// Bias gradients (rows: the blocks of k_relu_grad; beyond 1024 channels a pixel's channels span several
+// rows) and the head's partials use it.
+__device__ __forceinline__ void col_sum(const float *__restrict__ part, int c, int nrows, long stride, int C,
+                                        float *__restrict__ out, float (&s)[256]) {
+  float a = 0.f;
+  const int per = (int)((C + stride - 1) / stride);  // rows per pixel
+#pragma unroll 4
+  for (int r = (int)(c / stride) + per * (int)threadIdx.x; r < nrows; r += per * 256) a += part[(long)r * stride + c % stride];
+  s[threadIdx.x] = a;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if ((int)threadIdx.x < k) s[threadIdx.x] += s[threadIdx.x + k];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[c] = s[0];
+}
 __global__ void __launch_bounds__(256)
-k_sum_chunks(const float *__restrict__ part, int nchunks, long n, float *__restrict__ dw) {
+k_col_sum(const float *__restrict__ part, int nrows, long stride, int C, float *__restrict__ out) {
+  __shared__ float s[256];
+  col_sum(part, blockIdx.x, nrows, stride, C, out, s);
+}
+
+// The sums of a layer's gradients. Weights, dw[i] = sum over chunks of part[chunk][i]: a workgroup takes 64
+// elements, its 4 waves every fourth chunk in order (8 loads in flight each), their sums added in order. (One
+// thread per element over all chunks: 188 us per training step of 8 pairs of 256^2; so: 111 us, of more partial
+// sums.) The last C workgroups form the bias gradients (col_sum) in the shade of the others: as a launch per layer
+// of their own they took 72 us of a step (gradient with its copy to the host: 2.29 -> 2.24 ms).
+__global__ void __launch_bounds__(256)
+k_layer_sums(const float *__restrict__ part, int nchunks, long n, float *__restrict__ dw,
+             const float *__restrict__ bpart, int nrows, long stride, int C, float *__restrict__ db) {
+  __shared__ float s[256];
+  const int nwg = (int)((n + 63) / 64);
+  if ((int)blockIdx.x >= nwg) {  // uniform
+    col_sum(bpart, (int)blockIdx.x - nwg, nrows, stride, C, db, s);
+    return;
+  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long i = (long)blockIdx.x * 64 + lane, j = i < n ? i : n - 1;
   float a = 0.f;
@@ -524,10 +557,9 @@ k_sum_chunks(const float *__restrict__ part, int nchunks, long n, float *__restr
 #pragma unroll
     for (int k = 0; k < 8; ++k) a += c0 + 4 * k < nchunks ? v[k] : 0.f;
   }
-  __shared__ float s[4][64];
-  s[wave][lane] = a;
+  s[threadIdx.x] = a;
   __syncthreads();
-  if (wave == 0 && i < n) dw[i] = ((s[0][lane] + s[1][lane]) + s[2][lane]) + s[3][lane];
+  if (wave == 0 && i < n) dw[i] = ((s[lane] + s[64 + lane]) + s[128 + lane]) + s[192 + lane];
 }
 
 // Where the gradient of an activation comes from: its own buffer; or, for the upsampled source of a
@@ -594,27 +626,6 @@ k_relu_grad(GradSrc s, const bf16 *__restrict__ y, bf16 *__restrict__ dz, long n
     for (int k = c; k < RELU_BLOCK; k += win) a += sum[k];
     bpart[(long)blockIdx.x * win + c] = a;
   }
-}
-
-// out[c] = sum over rows r of part[r * stride + off(c)], one workgroup per column c: each thread sums
-// the rows r = t, t + 256, ... in order, then a fixed tree over the 256 threads (deterministic).
-// Bias gradients (rows: the blocks of k_relu_grad; beyond 1024 channels a pixel's channels span several
-// rows) and the head's partials use it.
-__global__ void __launch_bounds__(256)
-k_col_sum(const float *__restrict__ part, int nrows, long stride, int C, float *__restrict__ out) {
-  const int c = blockIdx.x;
-  float a = 0.f;
-  const int per = (int)((C + stride - 1) / stride);  // rows per pixel
-#pragma unroll 4
-  for (int r = (int)(c / stride) + per * (int)threadIdx.x; r < nrows; r += per * 256) a += part[(long)r * stride + c % stride];
-  __shared__ float s[256];
-  s[threadIdx.x] = a;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) s[threadIdx.x] += s[threadIdx.x + k];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[c] = s[0];
 }
 
 // 2x2 average pooling, NHWC bf16: y[b][yy][x][c] = mean of x[b][2yy..][2x..][c]; 8 channels per thread
@@ -1130,9 +1141,6 @@ int backward(msg_unet *u, const float *target, double *loss) {
                          logc, Hs, Ws, u->bpart.as<float>());
     }
     UHIP(hipGetLastError());
-    hipLaunchKernelGGL(k_col_sum, dim3(c.cout), dim3(256), 0, u->s, u->bpart.as<float>(), nb, (long)win, c.cout,
-                       g + c.boff);
-    UHIP(hipGetLastError());
     const ConvIn in = conv_input(u, c);
     const int cin = c.cin1 + c.cin2;
     const WgradGeom wg = wgrad_geom(B, Hs, Ws, cin, c.cout);
@@ -1149,7 +1157,8 @@ int backward(msg_unet *u, const float *target, double *loss) {
       hipLaunchKernelGGL((k_conv3x3_wgrad<1, 1, 16>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
     UHIP(hipGetLastError());
     const long nw = 9L * c.cout * cin;
-    hipLaunchKernelGGL(k_sum_chunks, dim3(cdivu(nw, 64)), dim3(256), 0, u->s, pt, wg.nsplit, nw, g + c.woff);
+    hipLaunchKernelGGL(k_layer_sums, dim3(cdivu(nw, 64) + c.cout), dim3(256), 0, u->s, pt, wg.nsplit, nw, g + c.woff,
+                       u->bpart.as<float>(), nb, (long)win, c.cout, g + c.boff);
     UHIP(hipGetLastError());
     if (k == 0) continue;  // no gradient for the input
     // gradient of the input (FP32): of both sources for a decoder convolution, which the two activations'
