@@ -68,9 +68,10 @@ __device__ __forceinline__ float step_at<float>(float f, double tau, float d) {
 // rounded reciprocal r. x / d is x r corrected twice by its exact remainder: x r is within 2 ulp, the
 // first correction makes it faithful, and a faithful quotient corrected with a correctly rounded
 // reciprocal is the correctly rounded one (Markstein 1990), so the result is that of a division bit for
-// bit. The fix-up returns the division's value for zeros, infinities and NaN. Six operations; a division
-// is about a dozen with a quarter-rate reciprocal (variation, energy and V-cycle of three FP64 pairs of
-// 512^2: 251 -> 236 us).
+// bit where the remainders are exact: d and r normal, x = 0 or |x| >= 2^-969 (below, within 2 ulp). The
+// fix-up returns the division's value for zeros, infinities, NaN and, though the corrections of an infinite
+// x r are NaN, the infinity of a quotient beyond the range. Six operations; a division is about a dozen
+// with a quarter-rate reciprocal (variation, energy and V-cycle of three FP64 pairs of 512^2: 251 -> 236 us).
 struct Div {
   double d, r;
 };

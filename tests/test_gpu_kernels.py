@@ -254,3 +254,36 @@ def test_f32_gradient_above_4096(gpu):
     a = gpu.gradient(R, T, phi, 0.0).double()
     b = gpu.gradient(R.double(), T.double(), phi.double(), 0.0)
     assert ((a - b).norm() / b.norm()).item() < 2e-5
+
+
+@pytest.mark.parametrize("op", ["ncc", "compose", "xshift"])
+def test_displacements_beyond_the_range(gpu, op):
+    """Finite displacements whose value in pixels overflows FP64 (from 2.9e306 domain units on, at 63 pixels a
+    unit; the kernels divide by a corrected reciprocal) and infinite ones are positions beyond the grid as any
+    other: the data terms and the composition are those of a displacement of 2e4 pixels, bit for bit (weight 0
+    on the regulariser, whose own value overflows)."""
+    n, h = 64, 1.0 / 63
+    rng = np.random.default_rng(11)
+    R, T = 1 + np.cumsum(rng.normal(size=(2, 1, n, n)), axis=3) / n
+    base = 0.4 * h * rng.normal(size=(2, n, n))
+
+    def fields(huge):
+        p = base.copy()
+        for k, (y, x) in enumerate(((5, 9), (20, 3), (33, 50), (62, 62), (0, 30), (41, 0))):  # no shared element
+            p[k % 2 if op != "xshift" else 0, y, x] = huge if k < 3 else -huge
+        return dev(p[None], torch.float64)
+
+    a = (dev(R, torch.float64), dev(T, torch.float64))
+
+    def run(huge, gradient):
+        p = fields(huge)
+        if op == "ncc":
+            return [gpu.ncc_energy(*a, p)[0]] + ([host(gpu.ncc_gradient(*a, p, 0.0))] if gradient else [])
+        if op == "xshift":
+            return [gpu.xshift_energy(*a, p, 0.7)[0]] + ([host(gpu.xshift_gradient(*a, p, 0.0, 0.7))] if gradient else [])
+        return [host(gpu.compose(dev(base, torch.float64), p[0]))]
+
+    for huge in (3e306, 5e306, 1e307, 1.7e308, np.inf):  # just beyond 2^1024 pixels, far beyond
+        gradient = huge <= 1e307  # 0 times the stiffness row of the larger ones is NaN
+        for got, want in zip(run(huge, gradient), run(2e4 * h, gradient)):
+            assert np.isfinite(want).all() and np.array_equal(got, want)
