@@ -143,7 +143,7 @@ def loss_and_grad(params, x_in, target, scales, base, bf16=True, acc32=False):
         dw = np.zeros((9, c["cout"], cin))
         for t in range(9):
             dy, dx = t // 3 - 1, t % 3 - 1
-            dw[t] = np.einsum("bhwo,bhwi->oi", dz, xp[:, 1 + dy:1 + dy + H, 1 + dx:1 + dx + W, :])
+            dw[t] = np.tensordot(dz, xp[:, 1 + dy:1 + dy + H, 1 + dx:1 + dx + W, :], axes=([0, 1, 2], [0, 1, 2]))
         g[c["woff"]:c["woff"] + dw.size] = dw.ravel()
         if k == 0:
             continue
