@@ -477,15 +477,30 @@ int mg_norm_blocks(int l, int coarse_max) {
 }
 
 // The V-cycle kernels of a field type: FP32 arithmetic for FP32 fields, FP64 for FP64 fields.
+// FP64 coarse levels: a wave at 8x8 and below, 4 at 16x16, at 32x32 one node per thread as long as every field
+// has a compute unit to itself (a workgroup of 1024 leaves no room for a second) and 4 waves, five workgroups to a
+// unit, beyond. With 1024 threads for every level and count: smoothing of 8192 pairs of 8x8 382 us, so 49 us; 2048 pairs of
+// 32x32 208 -> 92 us; 128 pairs of 32x32 30.7 us (4 waves 34.0), 192 pairs 42.2 -> 35.9 us.
+constexpr int MGC_WIDE_FIELDS = 256;
 template <typename S>
 void mg_coarse(dim3 g, hipStream_t s, const S *rhs, int negate, S *xout, int L, const PairState *st, double sigma,
                int nfields, const S *dold, double *nrm_part) {
   if constexpr (std::is_same<S, float>::value)
     hipLaunchKernelGGL(msg::k_mg_coarse_f32, g, dim3(msg::MGC_THREADS), 0, s, rhs, negate, xout, L, st, sigma, nfields,
                        dold, nrm_part);
-  else
-    hipLaunchKernelGGL((msg::k_mg_coarse<S>), g, dim3(msg::MGC_THREADS), 0, s, rhs, negate, xout, L, st, sigma, nfields, dold,
-                       nrm_part);
+  else {
+#define COARSE(ML, TH) \
+  hipLaunchKernelGGL((msg::k_mg_coarse<S, ML, TH>), g, dim3(TH), 0, s, rhs, negate, xout, L, st, sigma, nfields, dold, nrm_part)
+    if (L <= 3)
+      COARSE(3, 64);
+    else if (L == 4)
+      COARSE(4, 256);
+    else if (nfields <= MGC_WIDE_FIELDS)
+      COARSE(5, msg::MGC_THREADS);
+    else
+      COARSE(5, 256);
+#undef COARSE
+  }
 }
 template <typename S>
 void mg_down(dim3 g, hipStream_t s, const S *rhs, int negate, S *x2out, S *rhsc, int n, const PairState *st,

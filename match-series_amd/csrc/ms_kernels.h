@@ -1416,14 +1416,16 @@ k_mg_up(const S *__restrict__ x2in, const S *__restrict__ xc, const S *__restric
   }
 }
 
-// Whole V-cycle below (and including) a level of at most 32x32 nodes in one workgroup of MGC_THREADS threads,
-// in LDS. With n equal to the registration level this is the complete metric; otherwise it is the coarse
-// part of the cycle started by k_mg_down.
-// A chain of barriers with a node or less per thread between them, so the fewer and shorter the links the
+// Whole V-cycle below (and including) a level of at most 32x32 nodes in one workgroup, in LDS. With n
+// equal to the registration level this is the complete metric; otherwise it is the coarse part of the cycle
+// started by k_mg_down.
+// A chain of barriers with few nodes per thread between them, so the fewer and shorter the links the
 // better: the sweeps write a second buffer instead of updating in place, the residual is restricted as it is formed,
 // the prolongation is read on the fly by the first sweep of the up leg (3 barriers a level down and 2 up, 65 in
 // all before), a 32x32 level is one node per thread, and levels of at most 8x8 nodes run in wave 0 alone
 // behind compiler barriers: 20 to 24 us -> 15.7 us for a level of 32x32, the same bits.
+// MAXL bounds the level, TH is the workgroup: threads without a node hold a compute unit's slots and LDS idle, which
+// is free while every field's workgroup is resident and not beyond (mg_coarse chooses, with the times).
 constexpr int MGC_THREADS = 1024;
 constexpr int MGC_WAVE_LEVELS = 3;  // 8x8 nodes and below
 constexpr int MGC_MAXL = 5;
@@ -1437,8 +1439,8 @@ __device__ __forceinline__ void mgc_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename S>
-__global__ void __launch_bounds__(MGC_THREADS)
+template <typename S, int MAXL, int TH>
+__global__ void __launch_bounds__(TH)
 k_mg_coarse(const S *__restrict__ rhs, int negate, S *__restrict__ xout, int L, const PairState *st,
             double sigma_default, int nfields, const S *__restrict__ dold, double *__restrict__ nrm_part) {
   const int field = blockIdx.x;
@@ -1446,21 +1448,26 @@ k_mg_coarse(const S *__restrict__ rhs, int negate, S *__restrict__ xout, int L, 
   if (st && !participates(st[pair])) return;
   const double sigma = st ? st[pair].sigma : sigma_default;
   const double tau = 0.5 * (sigma * sigma);
-  __shared__ double X[MGC_OFF[MGC_MAXL + 1]], B[MGC_OFF[MGC_MAXL + 1]], Y[1 << (2 * MGC_MAXL)];
-  __shared__ double red[(MGC_THREADS / 64) * NORM_TERMS];
-  __shared__ Div dg[MGC_MAXL + 1];  // the levels' Jacobi diagonals, divided once
+  constexpr int MAXN = 1 << (2 * MAXL);
+  __shared__ double X[MGC_OFF[MAXL + 1]], B[MGC_OFF[MAXL + 1]], Y[MAXN];
+  __shared__ double red[(TH / 64) * NORM_TERMS];
+  __shared__ Div dg[MAXL + 1];  // the levels' Jacobi diagonals, divided once
   const int n = 1 << L;
   const int nn = n * n;
   const S *rp = rhs + (size_t)field * nn;
   const int tid = threadIdx.x;
-  const double raw = ld(rp, min(tid, nn - 1));
-  // the scalar products are summed by 256 threads; their operands load now, behind the sweeps
-  constexpr int PER = (1 << (2 * MGC_MAXL)) / 256;
+  constexpr int NPT = MAXN / TH;  // nodes per thread
+  double raw[NPT];
+#pragma unroll
+  for (int k = 0; k < NPT; ++k) raw[k] = ld(rp, min(tid + TH * k, nn - 1));
+  // the scalar products are summed by 256 threads (all, where there are fewer); their operands load now, behind
+  // the sweeps
+  constexpr int NT = TH < 256 ? TH : 256, PER = MAXN / NT;
   double rv[PER], ov[PER];
-  if (nrm_part && tid < 256) {
+  if (nrm_part && tid < NT) {
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-      const int i = min(tid + 256 * k, nn - 1);
+      const int i = min(tid + NT * k, nn - 1);
       rv[k] = ld(rp, i);
       ov[k] = ld(dold + (size_t)field * nn, i);
     }
@@ -1470,7 +1477,11 @@ k_mg_coarse(const S *__restrict__ rhs, int negate, S *__restrict__ xout, int L, 
     const double s = (double)((m - 1) * (m - 1));
     dg[tid] = make_div(1 + 4 * tau * s);
   }
-  if (tid < nn) B[MGC_OFF[L] + tid] = negate ? -raw : raw;
+#pragma unroll
+  for (int k = 0; k < NPT; ++k) {
+    const int i = tid + TH * k;
+    if (i < nn) B[MGC_OFF[L] + i] = negate ? -raw[k] : raw[k];
+  }
   __syncthreads();
 
   // x + (b - A x) / diag at a node, x read by get
@@ -1525,7 +1536,7 @@ k_mg_coarse(const S *__restrict__ rhs, int negate, S *__restrict__ xout, int L, 
   };
   auto block_sync = [] { __syncthreads(); };
   auto wave_sync = [] { mgc_wave_sync(); };
-  for (int l = L; l > MGC_WAVE_LEVELS; --l) down_level(l, MGC_THREADS, block_sync);
+  for (int l = L; l > MGC_WAVE_LEVELS; --l) down_level(l, TH, block_sync);
   if (tid < 64) {
     const int lw = min(L, MGC_WAVE_LEVELS);
     for (int l = lw; l >= 1; --l) down_level(l, 64, wave_sync);
@@ -1540,15 +1551,15 @@ k_mg_coarse(const S *__restrict__ rhs, int negate, S *__restrict__ xout, int L, 
     for (int l = 1; l <= lw; ++l) up_level(l, 64, wave_sync);
   }
   __syncthreads();
-  for (int l = MGC_WAVE_LEVELS + 1; l <= L; ++l) up_level(l, MGC_THREADS, block_sync);
+  for (int l = MGC_WAVE_LEVELS + 1; l <= L; ++l) up_level(l, TH, block_sync);
   S *xo = xout + (size_t)field * nn;
-  if (tid < nn) xo[tid] = static_cast<S>(X[MGC_OFF[L] + tid]);
+  for (int i = tid; i < nn; i += TH) xo[i] = static_cast<S>(X[MGC_OFF[L] + i]);
   if (nrm_part) {
     double acc[NORM_TERMS] = {0., 0., 0., 0.};  // <z,z>, <DE,z>, <DE,d_old>, <DE,DE> (DE = the raw input)
-    if (tid < 256) {
+    if (tid < NT) {
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
-        const int i = tid + 256 * k;
+        const int i = tid + NT * k;
         if (i < nn) {
           const double od = static_cast<double>(static_cast<S>(X[MGC_OFF[L] + i])), de = rv[k];
           acc[0] += od * od;
@@ -1558,7 +1569,7 @@ k_mg_coarse(const S *__restrict__ rhs, int negate, S *__restrict__ xout, int L, 
         }
       }
     }
-    block_sum_n<NORM_TERMS, MGC_THREADS>(acc, red);
+    block_sum_n<NORM_TERMS, TH>(acc, red);
     if (tid == 0)
       for (int t = 0; t < NORM_TERMS; ++t) nrm_part[(size_t)field * NORM_TERMS + t] = acc[t];
   }

@@ -310,3 +310,52 @@ def test_displacements_beyond_the_range(gpu, op):
         gradient = huge <= 1e307  # 0 times the stiffness row of the larger ones is NaN
         for got, want in zip(run(huge, gradient), run(2e4 * h, gradient)):
             assert np.isfinite(want).all() and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n", [2, 4, 8, 16, 32, 64])
+def test_f64_coarse_workgroups(gpu, n):
+    """The FP64 coarse V-cycle's workgroup depends on the level and, at 32^2, on the number of fields (more than
+    256 take narrower ones); the operations and the scalar products' sums do not: fields smoothed and levels
+    solved in a batch of 129 pairs are those of small batches bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    phi = torch.randn(129, 2, n, n, device="cuda", generator=g, dtype=torch.float64)
+    whole = gpu.h1_smooth(phi, 0.125)
+    for a in (0, 64, 128):
+        assert torch.equal(gpu.h1_smooth(phi[a:a + 64].contiguous(), 0.125), whole[a:a + 64])
+    if n < 8:
+        return
+    R = torch.rand(129, n, n, device="cuda", generator=g, dtype=torch.float64)
+    T = 0.6 * R + 0.4 * R.roll(1, 2)
+    out = []
+    for a, b in ((0, 129), (0, 2), (127, 129)):
+        c = gpu.Context(n.bit_length() - 1, b - a, gpu.F64)
+        c.set_images_device(R[a:b].contiguous(), T[a:b].contiguous())
+        c.set_deformations_device(torch.zeros(b - a, 2, n, n, device="cuda", dtype=torch.float64))
+        e = np.array(c.solve_level(n.bit_length() - 1, 10.0, 5, -1.0)[0])
+        f = torch.empty(b - a, 2, n, n, device="cuda", dtype=torch.float64)
+        c.get_deformations_device(f)
+        c.close()
+        out.append((e, f))
+    for (e, f), (a, b) in zip(out[1:], ((0, 2), (127, 129))):
+        assert np.array_equal(e, out[0][0][a:b]) and torch.equal(f, out[0][1][a:b])
+
+
+def shortest(fn, calls=25):
+    """The shortest of some calls, in seconds (every entry point waits for its result)."""
+    import time
+    best = 1e9
+    for _ in range(calls):
+        torch.cuda.synchronize()
+        a = time.perf_counter()
+        fn()
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - a)
+    return best
+
+
+def test_many_small_fields_keep_the_rate(gpu):
+    """8192 pairs of 8^2 FP64 fields are 64 workgroups a compute unit of one wave: 2 times a single pair's call,
+    whose launch dominates (16 times where every field took 1024 threads); 5 allowed."""
+    phi = torch.randn(8192, 2, 8, 8, device="cuda", dtype=torch.float64)
+    one = phi[:1].contiguous()
+    assert shortest(lambda: gpu.h1_smooth(phi, 0.125)) < 5 * shortest(lambda: gpu.h1_smooth(one, 0.125))
