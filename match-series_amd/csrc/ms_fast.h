@@ -456,18 +456,22 @@ __device__ __forceinline__ float add_rounded(float a, float b) {
   return a + b;
 }
 
-// The same variation for launches of GRAD_RUN_NODES nodes and more: a wave takes 64 element columns and the
-// rows of RUN nodes from below to above; a node's contributions from the element column to its left come by a
-// lane shift and those from the row below stay in registers, so there is no LDS and no barrier, node rows are
-// loaded once per element row instead of twice, and of the elements only 1/64 (columns) and 1/RUN (rows)
-// are worked on twice, where the 32 x 8 tiles take 5 passes of a wave for 4 waves of nodes. Same values as
-// k_grad_f32's, bit for bit. Bound by vector arithmetic (312 instructions per element, the tile kernel 417
+// The same variation for launches of GRAD_RUN_NODES nodes and more of grids from GRAD_RUN_GRID^2 on: a wave
+// takes 64 element columns and the rows of RUN nodes from below to above; a node's contributions from the element
+// column to its left come by a lane shift and those from the row below stay in registers, so there is no LDS and no
+// barrier, node rows are loaded once per element row instead of twice, and of the elements only 1/64 (columns) and
+// 1/RUN (rows) are worked on twice, where the 32 x 8 tiles take 5 passes of a wave for 4 waves of nodes. Same values
+// as k_grad_f32's, bit for bit (a sum of zeros alone may differ in the zero's sign). Bound by vector arithmetic (312 instructions per element, the tile kernel 417
 // before its clip and offsets took FP32 forms): 8 pairs of 1024^2, 106 us -> 102 us in tiles and 83 us here.
 // A run of 7 beat 4 and 5 (87, 86 us: more rows done twice) and 8 (87 us; 16: 100 us, too few waves at the end).
 // A wave's run is a chain of 8 elements at 1.6 us each, so small launches are faster in tiles: 512^2 6.9 us (runs
-// 12.0), 1024^2 16.4 (18.5), 2 x 1024^2 27.7 (25.1), 4 x 1024^2 49.3 (42.9): runs from 2^21 nodes on (so the
-// tiles never see an image of more than 4096^2, the bound of FIDX).
+// 12.0), 1024^2 16.4 (18.5), 2 x 1024^2 27.7 (25.1), 4 x 1024^2 49.3 (42.9): runs from 2^21 nodes on. And a run's 63
+// columns fit small grids badly (64^2: one node in the second column of waves), tiles of 32 x 8 well, whole calls of
+// 2^22 nodes: 8^2 139 us (runs 261), 32^2 73 (128), 64^2 76 (112), 128^2 78 (82), 256^2 78 (81; of 2^23 nodes 130 and
+// 126), 512^2 78.5 (77.0; 131 and 119): runs from 512^2 on. (So the tiles never see an image of more than 1024^2; FIDX
+// holds to 4096^2.)
 constexpr long GRAD_RUN_NODES = 1l << 21;
+constexpr int GRAD_RUN_GRID = 512;
 constexpr int GRR_TX = 63;  // nodes per wave and row (lane 0 only passes its element on)
 constexpr int GRR_RUN = 7;
 template <int RUN, bool FIDX>

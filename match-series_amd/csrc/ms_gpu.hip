@@ -355,7 +355,7 @@ int launch_energy(const S *R, const S *T, const S *phi, const S *z, const S *dol
 
 void launch_grad_f32(const float *R, const float *T, const float *phi, float *DE, int n, double vol, const PairState *st,
                      double lambda, int npairs, hipStream_t s) {
-  if ((long)n * n * npairs >= msg::GRAD_RUN_NODES) {
+  if (n >= msg::GRAD_RUN_GRID && (long)n * n * npairs >= msg::GRAD_RUN_NODES) {
     const int ntx = cdiv(n, msg::GRR_TX), nty = cdiv(n, 4 * msg::GRR_RUN);
     if (n <= 4096)
       hipLaunchKernelGGL((msg::k_grad_run_f32<msg::GRR_RUN, true>), dim3(ntx * nty * npairs), dim3(256), 0, s, R, T,
