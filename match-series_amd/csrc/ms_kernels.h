@@ -1683,40 +1683,45 @@ __global__ void k_resample_rect(const S *__restrict__ src, int w, int h, S *__re
 // FastDeformImage (L140-162; clamp) and the NaN-extended variant of L226-256 (mode 2).
 // img: nimg images; phi: one field per image (or one shared field if phi_shared). n is a power of two,
 // logn its logarithm. Bound by HBM (phi, the image and the result once, 16 B per FP32 pixel). A workgroup
-// takes WARP_RUN x 256 pixels of one image: coordinates by shifts, and a thread's WARP_RUN pixels step by
-// step together, displacements, then the 4 neighbours each, so a wave waits for two memory round trips in
-// WARP_RUN pixels. Pixels outside gather from clamped nodes and are replaced by a select (no branches).
-// 31 frames of 1024^2 in FP32: 192 -> 118 us (4.5 TB/s) against one pixel per thread with 64-bit index
-// divisions.
+// takes tiles of 256 columns (or the whole width) and a thread RUN pixels one below another, step by step
+// together, displacements, then the 4 neighbours each, so a wave waits for two memory round trips in RUN pixels
+// and neighbouring rows meet in its cache lines. Pixels outside gather from clamped nodes and are replaced by a
+// select (no branches). 31 frames of 1024^2 in FP32, whole calls: 200 us with one pixel per thread and 64-bit index
+// divisions; 132 us so (4.5 TB/s), where the field is noisy (1.5 pixels) 205 and 137 us; FP64 226 and 197, noisy 261
+// and 229 us. RUN = 4 pixels in a row, 256 apart, instead: 135 us, but 205 us where noisy (FP64 206 and 378 us), four
+// rows' neighbours at once being more than a compute unit's L1 holds. Few pixels have nothing to overlap:
+// 128^2 20.7 us with RUN = 1, 21.7 with 4; from WARP_RUN_PIXELS (512 workgroups of 4) on the latter is no slower:
+// 512^2 x 2 22.8 and 23.1 us, in FP64 up to 25.6 and 23.2.
 constexpr int WARP_RUN = 4;
+constexpr long WARP_RUN_PIXELS = 1l << 19;
 
-template <typename S>
+template <typename S, int RUN>
 __global__ void __launch_bounds__(256)
 k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out, int n, int logn, int nblk,
        int phi_shared, int mode, double ext, int nearest) {
-  const int f = blockIdx.x / nblk;
+  const int f = blockIdx.x / nblk, tile = blockIdx.x - f * nblk;
   const int cnt = n * n;
-  const int j0 = (blockIdx.x - f * nblk) * (256 * WARP_RUN) + threadIdx.x;
+  const int logw = logn < 8 ? logn : 8;  // a tile's columns; its 256 RUN >> logw rows
+  const int x = ((tile & ((n >> logw) - 1)) << logw) + (threadIdx.x & ((1 << logw) - 1));
+  const int y0 = (tile >> (logn - logw)) * ((256 * RUN) >> logw) + (threadIdx.x >> logw) * RUN;
   const double h = 1.0 / (double)(n - 1);
   const S *ph = phi + (phi_shared ? 0 : (size_t)f * 2 * cnt);
   const S *im = img + (size_t)f * cnt;
   S *o = out + (size_t)f * cnt;
   const double hi = (double)(n - 1);
-  S p0[WARP_RUN], p1[WARP_RUN];
+  S p0[RUN], p1[RUN];
 #pragma unroll
-  for (int k = 0; k < WARP_RUN; ++k) {
-    const int j = min(j0 + 256 * k, cnt - 1);
+  for (int k = 0; k < RUN; ++k) {
+    const int j = min(x + (y0 + k) * n, cnt - 1);
     p0[k] = ph[j];
     p1[k] = ph[(size_t)cnt + j];
   }
-  double X[WARP_RUN], Y[WARP_RUN];
-  S v[WARP_RUN][4];
-  bool inside[WARP_RUN];
+  double X[RUN], Y[RUN];
+  S v[RUN][4];
+  bool inside[RUN];
 #pragma unroll
-  for (int k = 0; k < WARP_RUN; ++k) {
-    const int j = min(j0 + 256 * k, cnt - 1);
-    const int x = j & (n - 1), y = j >> logn;
-    double dx = x + (double)p0[k] / h, dy = y + (double)p1[k] / h;
+  for (int k = 0; k < RUN; ++k) {
+    double dx = x + (double)p0[k] / h, dy = (y0 + k) + (double)p1[k] / h;
     inside[k] = true;
     if (mode == 1) {  // clamp
       dx = dx < 0 ? 0 : (dx > hi ? hi : dx);
@@ -1739,12 +1744,12 @@ k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out
     v[k][3] = c[n + 1];
   }
 #pragma unroll
-  for (int k = 0; k < WARP_RUN; ++k) {
+  for (int k = 0; k < RUN; ++k) {
     const double v0 = v[k][0], v1 = v[k][1], v2 = v[k][2], v3 = v[k][3];
     const double r0 = (1 - X[k]) * v0 + X[k] * v1;
     const double r1 = (1 - X[k]) * (1 - Y[k]) * v0 + X[k] * (1 - Y[k]) * v1 + (1 - X[k]) * Y[k] * v2 + X[k] * Y[k] * v3;
     const double r = inside[k] ? (Y[k] == 0 ? r0 : r1) : (mode == 2 ? __builtin_nan("") : ext);
-    if (j0 + 256 * k < cnt) o[j0 + 256 * k] = static_cast<S>(r);
+    if (y0 + k < n) o[x + (y0 + k) * n] = static_cast<S>(r);
   }
 }
 
