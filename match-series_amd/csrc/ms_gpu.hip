@@ -1921,6 +1921,40 @@ int stats_impl(const void *stack, int nimg, int n, double fill, void *mean, void
   return MSG_OK;
 }
 
+// Normalisation by launches over all images: a count per digit, then the scaling; PT elements per thread.
+template <typename S, int PT>
+int normalize_sweeps(S *img, int nn, int nimg, int i0, int i1, int saturate, int min_to_zero, hipStream_t s) {
+  constexpr int P = msg::SelKey<S>::PASSES;
+  const int per = std::min(nimg, 1024);  // images per sweep: bounds the counts (16 KiB per image and digit)
+  const size_t words = (size_t)P * per * 2 * msg::SEL_BINS;
+  void *hist, *st;
+  CHK(scratch_get(81, sizeof(unsigned) * words, &hist));
+  CHK(scratch_get(82, sizeof(msg::SelState) * (P + 1) * per * 2, &st));
+  for (int k0 = 0; k0 < nimg; k0 += per) {
+    const int m = std::min(per, nimg - k0);
+    S *im = img + (size_t)k0 * nn;
+    const dim3 g(cdiv(nn, PT * msg::SEL_THREADS), m), b(msg::SEL_THREADS);
+    const size_t w = (size_t)P * m * 2 * msg::SEL_BINS;
+    hipLaunchKernelGGL(msg::k_fill_u32, dim3((unsigned)std::min<size_t>((w + 255) / 256, 4096)), b, 0, s,
+                       (unsigned *)hist, w, 0u);
+    for (int p = 0; p < P; ++p)
+      hipLaunchKernelGGL((msg::k_sel_count<S, PT>), g, b, 0, s, (const S *)im, nn, m, p, (unsigned)i0, (unsigned)i1,
+                         (unsigned *)hist, (msg::SelState *)st);
+    hipLaunchKernelGGL((msg::k_normalize<S, PT>), g, b, 0, s, im, nn, m, (unsigned)i0, (unsigned)i1,
+                       (const unsigned *)hist, (const msg::SelState *)st, saturate, min_to_zero);
+    HIPCHK(hipGetLastError());
+  }
+  return MSG_OK;
+}
+
+// Images of up to 64^2 in one launch; up to 512^2, 2^20 pixels in all, with 8 pixels per thread, so that a launch has
+// workgroups enough; larger ones with 32 (fewer workgroups, which each find the digit and add up counts). Whole calls
+// in us, one workgroup / 8 / 32 per thread: 64^2 in FP32 26 / 37 / 40, 24 x 64^2 26 / 39 / 42, 64^2 in FP64 33 / 58 / 61;
+// 128^2 in FP32 42 / 36 / 45, in FP64 60 / 52 / 72; 256^2 in FP64 145 / 52 / 75, 4 x 512^2 in FP32 - / 45 / 49,
+// 1024^2 - / 56 / 52, 24 x 256^2 - / 51 / 51.
+constexpr int NORM_ONE = 64 * 64, NORM_SHORT = 512 * 512;
+constexpr long NORM_SHORT_ALL = 1 << 20;
+
 template <typename S>
 int normalize_impl(void *img, int n, int nimg, double pct, int min_to_zero, hipStream_t s) {
   const int nn = n * n;
@@ -1932,27 +1966,15 @@ int normalize_impl(void *img, int n, int nimg, double pct, int min_to_zero, hipS
     i0 = std::min(std::max(i0, 0), m1);
     i1 = std::min(std::max(i1, 0), m1);
   }
-  constexpr int P = msg::SelKey<S>::PASSES;
-  const int per = std::min(nimg, 1024);  // images per sweep: bounds the counts (16 KiB per image and digit)
-  const size_t words = (size_t)P * per * 2 * msg::SEL_BINS;
-  void *hist, *st;
-  CHK(scratch_get(81, sizeof(unsigned) * words, &hist));
-  CHK(scratch_get(82, sizeof(msg::SelState) * (P + 1) * per * 2, &st));
-  for (int k0 = 0; k0 < nimg; k0 += per) {
-    const int m = std::min(per, nimg - k0);
-    S *im = (S *)img + (size_t)k0 * nn;
-    const dim3 g(cdiv(nn, msg::SEL_CHUNK), m), b(msg::SEL_THREADS);
-    const size_t w = (size_t)P * m * 2 * msg::SEL_BINS;
-    hipLaunchKernelGGL(msg::k_fill_u32, dim3((unsigned)std::min<size_t>((w + 255) / 256, 4096)), b, 0, s,
-                       (unsigned *)hist, w, 0u);
-    for (int p = 0; p < P; ++p)
-      hipLaunchKernelGGL((msg::k_sel_count<S>), g, b, 0, s, (const S *)im, nn, m, p, (unsigned)i0, (unsigned)i1,
-                         (unsigned *)hist, (msg::SelState *)st);
-    hipLaunchKernelGGL((msg::k_normalize<S>), g, b, 0, s, im, nn, m, (unsigned)i0, (unsigned)i1,
-                       (const unsigned *)hist, (const msg::SelState *)st, pct >= 0 ? 1 : 0, min_to_zero);
+  if (nn <= NORM_ONE) {
+    hipLaunchKernelGGL((msg::k_normalize_one<S>), dim3(nimg), dim3(msg::SEL1_THREADS), 0, s, (S *)img, nn, (unsigned)i0,
+                       (unsigned)i1, pct >= 0 ? 1 : 0, min_to_zero);
     HIPCHK(hipGetLastError());
+    return MSG_OK;
   }
-  return MSG_OK;
+  if (nn <= NORM_SHORT && (long)nn * nimg <= NORM_SHORT_ALL)
+    return normalize_sweeps<S, 8>((S *)img, nn, nimg, i0, i1, pct >= 0, min_to_zero, s);
+  return normalize_sweeps<S, 32>((S *)img, nn, nimg, i0, i1, pct >= 0, min_to_zero, s);
 }
 
 template <typename S>

@@ -174,12 +174,12 @@ k_series_stats_sort(const S *__restrict__ stack, int nimg, int nn, double fill, 
 // there. Pass p counts digit p of the elements that share the digits found so far, once per rank (one
 // histogram serves both ranks while their prefixes agree); the next pass, and the normalisation after the
 // last, find their rank's digit from those counts, every workgroup for itself (2048 counts from L2).
-// Bound by one read of the images per digit (3 for FP32, 6 for FP64) and, for one image, by its 5 small
-// launches. 24 frames of 1024^2 in FP32: 160 us with the copy of the frames, where one library sort
+// Bound by one read of the images per digit (3 for FP32, 6 for FP64) and, for one image, by its 5 or 8 small
+// launches (small images: k_normalize_one). 24 frames of 1024^2 in FP32: 160 us with the copy of the frames, where one library sort
 // after another took 3.71 ms (21 launches and about 150 us per frame).
 // ------------------------------------------------------------------------------------------------
 constexpr int SEL_BITS = 11, SEL_BINS = 1 << SEL_BITS;
-constexpr int SEL_THREADS = 256, SEL_PER_THREAD = 32, SEL_CHUNK = SEL_THREADS * SEL_PER_THREAD;
+constexpr int SEL_THREADS = 256;
 
 template <typename S>
 struct SelKey;
@@ -219,18 +219,18 @@ struct SelState {
   unsigned rank, pad;
 };
 
-// The digit that holds `rank` in counts h[SEL_BINS] and the rank within it, for every thread of the
-// workgroup. tmp: 4 + 2 words of LDS.
-__device__ __forceinline__ void sel_digit(const unsigned *__restrict__ h, unsigned rank, unsigned *tmp,
-                                          unsigned &digit, unsigned &rest) {
-  constexpr int PER = SEL_BINS / SEL_THREADS;
+// The digit that holds `rank` in counts h[SEL_BINS] and the rank within it, found by TH threads (t: the thread among
+// them) and left in tmp[TH / 64], tmp[TH / 64 + 1]. tmp: TH / 64 + 2 words of LDS. Barriers of the whole workgroup.
+template <int TH>
+__device__ __forceinline__ void sel_find(const unsigned *__restrict__ h, unsigned rank, unsigned *tmp, int t) {
+  constexpr int PER = SEL_BINS / TH, NW = TH / 64;
   unsigned c[PER], mine = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    c[k] = h[threadIdx.x * PER + k];
+    c[k] = h[t * PER + k];
     mine += c[k];
   }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = t & 63, wid = t >> 6;
   unsigned inc = mine;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -251,12 +251,17 @@ __device__ __forceinline__ void sel_digit(const unsigned *__restrict__ h, unsign
         r -= c[j];
         ++k;
       }
-    tmp[4] = threadIdx.x * PER + k;
-    tmp[5] = r;
+    tmp[NW] = t * PER + k;
+    tmp[NW + 1] = r;
   }
   __syncthreads();
-  digit = tmp[4];
-  rest = tmp[5];
+}
+// The same for every thread of a workgroup of SEL_THREADS.
+__device__ __forceinline__ void sel_digit(const unsigned *__restrict__ h, unsigned rank, unsigned *tmp,
+                                          unsigned &digit, unsigned &rest) {
+  sel_find<SEL_THREADS>(h, rank, tmp, threadIdx.x);
+  digit = tmp[SEL_THREADS / 64];
+  rest = tmp[SEL_THREADS / 64 + 1];
 }
 
 // State of both ranks of image `img` before digit p, from the state before digit p - 1 and that digit's
@@ -290,8 +295,8 @@ __device__ __forceinline__ void sel_advance(const unsigned *__restrict__ hist, c
   }
 }
 
-// Counts of digit p. Grid (chunks of SEL_CHUNK elements, images).
-template <typename S>
+// Counts of digit p. Grid (chunks of PT elements per thread, images).
+template <typename S, int PT>
 __global__ void __launch_bounds__(SEL_THREADS)
 k_sel_count(const S *__restrict__ imgs, int nn, int nimg, int p, unsigned rank0, unsigned rank1,
             unsigned *__restrict__ hist, SelState *__restrict__ st) {
@@ -313,9 +318,9 @@ k_sel_count(const S *__restrict__ imgs, int nn, int nimg, int p, unsigned rank0,
   const int top = p == 0 ? 0 : sel_shift<S>(p - 1);  // bits below the prefix
   const unsigned mask = p == 0 ? SEL_BINS - 1 : (unsigned)((1u << (top - shift)) - 1u);
   const K p0 = (K)s[0].prefix, p1 = (K)s[1].prefix;
-  const int i0 = blockIdx.x * SEL_CHUNK + threadIdx.x;
+  const int i0 = blockIdx.x * (PT * SEL_THREADS) + threadIdx.x;
   constexpr int RUN = 8;  // loads in flight per thread
-  for (int k = 0; k < SEL_PER_THREAD; k += RUN) {
+  for (int k = 0; k < PT; k += RUN) {
     S v[RUN];
 #pragma unroll
     for (int r = 0; r < RUN; ++r) {
@@ -340,11 +345,27 @@ k_sel_count(const S *__restrict__ imgs, int nn, int nimg, int p, unsigned rank0,
   }
 }
 
-// prepareMultilevelArray (registration.h:331-347) with the image's elements of rank0 and rank1:
+// prepareMultilevelArray (registration.h:331-347) with the image's elements of rank0 and rank1, lo and hi:
 // saturate: clamp to [lo, hi], subtract the minimum (lo) and divide by the maximum (hi - lo);
 // otherwise lo, hi are the extrema: subtract the minimum if negative or min_to_zero, divide by the
-// (shifted) maximum. Grid as k_sel_count.
-template <typename S>
+// (shifted) maximum.
+struct NormScale {
+  double lo, hi, mx;
+  bool saturate, shifted;
+  __device__ __forceinline__ NormScale(double l, double h, int sat, int min_to_zero)
+      : lo(l), hi(h), saturate(sat), shifted(sat || l < 0. || min_to_zero) {
+    mx = shifted ? hi + -1 * lo : hi;  // getMaxValue() of the shifted image
+  }
+  __device__ __forceinline__ double operator()(double v) const {
+    if (saturate) v = v < lo ? lo : (v > hi ? hi : v);
+    if (shifted) v += -1 * lo;  // addToAll(-1 * getMinValue())
+    if (mx != 0) v /= mx;
+    return v;
+  }
+};
+
+// Grid as k_sel_count.
+template <typename S, int PT>
 __global__ void __launch_bounds__(SEL_THREADS)
 k_normalize(S *__restrict__ imgs, int nn, int nimg, unsigned rank0, unsigned rank1, const unsigned *__restrict__ hist,
             const SelState *__restrict__ st, int saturate, int min_to_zero) {
@@ -353,13 +374,12 @@ k_normalize(S *__restrict__ imgs, int nn, int nimg, unsigned rank0, unsigned ran
   const int img = blockIdx.y;
   SelState s[2];
   sel_advance<S>(hist, st, img, nimg, SelKey<S>::PASSES, rank0, rank1, tmp, s);
-  const double lo = (double)SelKey<S>::value((K)s[0].prefix), hi = (double)SelKey<S>::value((K)s[1].prefix);
-  const bool shifted = saturate || lo < 0. || min_to_zero;
-  const double mx = shifted ? hi + -1 * lo : hi;  // getMaxValue() of the shifted image
+  const NormScale sc((double)SelKey<S>::value((K)s[0].prefix), (double)SelKey<S>::value((K)s[1].prefix), saturate,
+                     min_to_zero);
   S *im = imgs + (size_t)img * nn;
-  const int i0 = blockIdx.x * SEL_CHUNK + threadIdx.x;
+  const int i0 = blockIdx.x * (PT * SEL_THREADS) + threadIdx.x;
   constexpr int RUN = 8;
-  for (int k = 0; k < SEL_PER_THREAD; k += RUN) {
+  for (int k = 0; k < PT; k += RUN) {
     S in[RUN];
 #pragma unroll
     for (int r = 0; r < RUN; ++r) {
@@ -369,13 +389,82 @@ k_normalize(S *__restrict__ imgs, int nn, int nimg, unsigned rank0, unsigned ran
 #pragma unroll
     for (int r = 0; r < RUN; ++r) {
       const int i = i0 + (k + r) * SEL_THREADS;
-      double v = (double)in[r];
-      if (saturate) v = v < lo ? lo : (v > hi ? hi : v);
-      if (shifted) v += -1 * lo;  // addToAll(-1 * getMinValue())
-      if (mx != 0) v /= mx;
+      const double v = sc((double)in[r]);
       if (i < nn) im[i] = static_cast<S>(v);
     }
   }
+}
+
+// The same for small images in one launch: a workgroup takes an image through all digits, its counts in LDS. Bound by
+// the chain of its barriers and LDS round trips, about 1.5 us a digit. One image of 64^2, whole call: FP32 40 us in 5
+// launches, 26 us so, FP64 61 us in 8 launches and 33 us (a library's sort of it: 34 and 41 us).
+constexpr int SEL1_THREADS = 1024;
+
+// Counts digit d of the lanes with `take` set; those that share the first one's digit in one addition, so that
+// an image of one value (all lanes on one word of LDS) takes no longer than another (FP64 64^2: 16 us less).
+// (The sweeps of larger images do without: it costs others 2 us of a workgroup's pass.)
+__device__ __forceinline__ void sel_add(unsigned *h, unsigned d, bool take) {
+  const unsigned long long act = __ballot(take);
+  if (!act) return;
+  const int first = __ffsll((long long)act) - 1;
+  const unsigned d0 = __builtin_amdgcn_readlane(d, first);
+  const unsigned long long same = __ballot(take && d == d0);
+  if ((int)(threadIdx.x & 63) == first)
+    atomicAdd(&h[d0], (unsigned)__popcll(same));
+  else if (take && d != d0)
+    atomicAdd(&h[d], 1u);
+}
+
+template <typename S>
+__global__ void __launch_bounds__(SEL1_THREADS)
+k_normalize_one(S *__restrict__ imgs, int nn, unsigned rank0, unsigned rank1, int saturate, int min_to_zero) {
+  typedef typename SelKey<S>::type K;
+  __shared__ unsigned h[2][SEL_BINS];
+  constexpr int HALF = SEL1_THREADS / 2;  // threads that look for a rank's digit
+  __shared__ unsigned tmp[2][HALF / 64 + 2];
+  S *im = imgs + (size_t)blockIdx.x * nn;
+  K prefix[2] = {0, 0};
+  unsigned rank[2] = {rank0, rank1};
+  constexpr int RUN = 4;  // loads in flight per thread
+  const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63), lane = threadIdx.x & 63;
+  auto sweep = [&](const auto &f) {  // f(index, value, inside the image), by whole waves
+    for (int w = wave0; w < nn; w += RUN * SEL1_THREADS) {
+      S v[RUN];
+#pragma unroll
+      for (int r = 0; r < RUN; ++r) v[r] = im[min(w + r * SEL1_THREADS + lane, nn - 1)];
+#pragma unroll
+      for (int r = 0; r < RUN; ++r) {
+        const int i = w + r * SEL1_THREADS + lane;
+        if (w + r * SEL1_THREADS < nn) f(i, v[r], i < nn);
+      }
+    }
+  };
+  for (int p = 0; p < SelKey<S>::PASSES; ++p) {
+    const int shift = sel_shift<S>(p), top = p == 0 ? 0 : sel_shift<S>(p - 1);
+    const int w = p == 0 ? SEL_BITS : top - shift;
+    const unsigned mask = (1u << w) - 1u;
+    const bool two = prefix[0] != prefix[1];
+    for (int i = threadIdx.x; i < SEL_BINS; i += SEL1_THREADS) h[0][i] = h[1][i] = 0;
+    __syncthreads();
+    sweep([&](int, S v, bool in) {
+      const K key = SelKey<S>::key(v);
+      const unsigned d = (unsigned)(key >> shift) & mask;
+      sel_add(h[0], d, in && (p == 0 || (key >> top) == prefix[0]));
+      if (two) sel_add(h[1], d, in && (key >> top) == prefix[1]);
+    });
+    __syncthreads();
+    const int half = wave0 / HALF;
+    sel_find<HALF>(h[two ? half : 0], rank[half], tmp[half], threadIdx.x % HALF);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      prefix[r] = (prefix[r] << w) | tmp[r][HALF / 64];
+      rank[r] = tmp[r][HALF / 64 + 1];
+    }
+  }
+  const NormScale sc((double)SelKey<S>::value(prefix[0]), (double)SelKey<S>::value(prefix[1]), saturate, min_to_zero);
+  sweep([&](int i, S v, bool in) {
+    if (in) im[i] = static_cast<S>(sc((double)v));
+  });
 }
 
 }  // namespace msg

@@ -27,11 +27,11 @@ def host(t):
     return t.detach().cpu().double().numpy()
 
 
-@pytest.mark.parametrize("n,frames", [(2, 3), (4, 1), (64, 5), (128, 2), (256, 3)])
+@pytest.mark.parametrize("n,frames", [(2, 3), (4, 1), (64, 5), (128, 2), (256, 3), (8, 2), (32, 3), (512, 5)])
 @pytest.mark.parametrize("code", [0, 1])
 def test_normalize_ranks(gpu, n, frames, code):
     """The radix-selected bounds are the sorted image's elements: images below, at and above one
-    workgroup's chunk, few distinct values, values of both signs over many binades, constant images,
+    workgroup's chunk (one launch up to 64^2, above it 8 or 32 pixels per thread), few distinct values, values of both signs over many binades, constant images,
     infinities. The result then repeats the definition's operations in FP64, so it is exact up to the
     rounding to the storage type."""
     rng = np.random.default_rng(n + frames)
@@ -401,3 +401,11 @@ def test_warp_of_noisy_fields_keeps_the_rate(gpu):
     phi = torch.randn(31, 2, 1024, 1024, device="cuda", dtype=torch.float64) * (1.5 / 1024)
     still = torch.zeros_like(phi)
     assert shortest(lambda: gpu.warp(img, phi)) < 1.5 * shortest(lambda: gpu.warp(img, still))
+
+
+def test_normalize_of_a_small_image_is_one_launch(gpu):
+    """An FP64 image of 16^2 is normalised in about 1.2 times the time of its warp, one launch each (2.5 times in
+    eight launches); 1.8 allowed."""
+    img = torch.rand(1, 16, 16, device="cuda", dtype=torch.float64)
+    phi = torch.zeros(1, 2, 16, 16, device="cuda", dtype=torch.float64)
+    assert shortest(lambda: gpu.normalize(img, 0.15)) < 1.8 * shortest(lambda: gpu.warp(img, phi))
