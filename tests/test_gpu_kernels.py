@@ -409,3 +409,14 @@ def test_normalize_of_a_small_image_is_one_launch(gpu):
     img = torch.rand(1, 16, 16, device="cuda", dtype=torch.float64)
     phi = torch.zeros(1, 2, 16, 16, device="cuda", dtype=torch.float64)
     assert shortest(lambda: gpu.normalize(img, 0.15)) < 1.8 * shortest(lambda: gpu.warp(img, phi))
+
+
+def test_unet_of_wide_layers_keeps_the_rate(gpu):
+    """One image through 256 to 2048 channels is 8 times the operations of 8 images through 32 to 256, and takes 7
+    times as long (15 times where a step of the wide layers waited for its own loads); 10 allowed."""
+    wide, narrow = gpu.UNet(4, 256, seed=1), gpu.UNet(4, 32, seed=1)
+    x = torch.rand(8, 2, 256, 256, device="cuda")
+    one = x[:1].contiguous()
+    assert shortest(lambda: wide.forward(one)) < 10 * shortest(lambda: narrow.forward(x))
+    wide.close()
+    narrow.close()
