@@ -29,6 +29,7 @@
 #include <mutex>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace msg {
@@ -321,17 +322,18 @@ k_conv3x3_tile(ConvIn in, const bf16 *__restrict__ w, const float *__restrict__ 
     }
 }
 
-// Any multiple of 64 input channels (32 NT output), the input read through the caches: for the networks
-// whose input tile does not fit LDS. One wave: 32 NT output channels and 32 NP consecutive pixels of one
+// Any multiples of 64 input and output channels, the input read through the caches: for the networks
+// whose input tile does not fit LDS. One wave: 64 output channels and 32 NP consecutive pixels of one
 // image row (W % (32 NP) == 0); four waves per workgroup along the pixels. Wide layers are small images with few
 // waves, so what bounds it is the way to L2: the operands of 4 steps (of 16 channels) are in flight while the 4
 // steps before them multiply. A forward of 4 scales from 256 channels at 256^2 (512 to 2048 channels here): 6.4 ms
 // with a step's loads waited for by the step, 6.8 ms so from packed weights (a new line each step), 3.1 ms now (4
 // images: 23.9, 15.9, 10.7 ms; 13.5 ms at one wave per SIMD, which the registers of four tiles would take unbounded).
-template <int NT, int NP, typename OutT>
+template <int NP, typename OutT>
 __global__ void __launch_bounds__(256, 2)
 k_conv3x3(ConvIn in, const bf16 *__restrict__ w, const float *__restrict__ bias, OutT *__restrict__ y, int B, int H,
           int W, int cout, int relu) {
+  constexpr int NT = 2;  // tiles of 32 output channels
   const int cin = in.c1 + in.c2;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long M = (long)B * H * W;
@@ -944,7 +946,7 @@ struct WgradGeom {
 WgradGeom wgrad_geom(int B, int H, int W, int cin, int cout) {
   WgradGeom g;
   g.wm = cout % 64 == 0 ? 2 : 1;
-  g.wn = cin % 64 == 0 ? 2 : 1;
+  g.wn = g.wm == 2 && cin % 64 == 0 ? 2 : 1;
   g.rows = g.wm * g.wn == 1 ? 16 : 8;
   g.nblocks = (cout / (32 * g.wm)) * cdivu(cin, 32 * g.wn);
   const int ntile = B * (H / g.rows) * (W / 32);
@@ -1000,26 +1002,18 @@ void conv_tile(msg_unet *u, ConvIn in, const bf16 *w, const float *bias, OutT *y
 
 // H and W are multiples of 32, cout of 32. Tiles by what LDS holds (16 rows of up to 64 input channels, 8
 // of 96, 4 beyond) and by the work there is: the largest NT x NP that still gives every SIMD two waves, or
-// one with 2 x 2.
+// one with 2 x 2. Only the channel counts that occur have kernels (base a power of two from 32 on): BF16 results
+// from 16, 32, 64, 96, 128, 192, 256, 384 and more channels, FP32 results (data gradients) from powers of two, 32
+// results or 96 from up to 96 channels only, other counts are multiples of 64.
 template <typename OutT>
 int launch_conv(msg_unet *u, ConvIn in, const bf16 *w, const float *bias, OutT *y, int cout, int relu, int H, int W) {
+  constexpr bool FWD = sizeof(OutT) == 2;
   const int cin = in.c1 + in.c2;
   const long rows = (long)u->B * H * (W / 32);  // tiles of 32 pixels
   auto waves = [&](int nt, int np) { return rows / np * (cout / (32 * nt)); };
   const bool two = cout % 64 == 0, four = cout % 128 == 0;
-  bool done = true;
+  bool done = two || cin < 128;
 #define CONV(CIN, WM, WR, NT, NP) conv_tile<CIN, WM, WR, NT, NP>(u, in, w, bias, y, cout, relu, H, W)
-#define CONV_SMALL(CIN)                             \
-  do {                                              \
-    if (two && waves(2, 4) >= 2048)                 \
-      CONV(CIN, 1, 4, 2, 4);                        \
-    else if (!two && waves(1, 4) >= 2048)           \
-      CONV(CIN, 1, 4, 1, 4);                        \
-    else if (two && waves(2, 2) >= 1024)            \
-      CONV(CIN, 1, 4, 2, 2);                        \
-    else                                            \
-      CONV(CIN, 1, 4, 1, 2);                        \
-  } while (0)
 #define CONV_LARGE(CIN)                             \
   do {                                              \
     if (four && waves(2, 2) >= 1024)                \
@@ -1027,44 +1021,66 @@ int launch_conv(msg_unet *u, ConvIn in, const bf16 *w, const float *bias, OutT *
     else                                            \
       CONV(CIN, 2, 2, 1, 2);                        \
   } while (0)
-  if (cin == 16 && waves(1, 4) >= 1024)
-    CONV(16, 1, 4, 1, 4);
-  else if (cin == 16)
-    CONV(16, 1, 4, 1, 2);
-  else if (cin == 32)
-    CONV_SMALL(32);
-  else if (cin == 64)
-    CONV_SMALL(64);
-  else if (cin == 96 && waves(1, 4) >= 1024)
-    CONV(96, 1, 2, 1, 4);
-  else if (cin == 96)
-    CONV(96, 1, 4, 1, 2);
-  else if (cin == 128 && two)
-    CONV_LARGE(128);
-  else if (cin == 192 && two && waves(2, 2) >= 1024)
-    CONV(192, 1, 2, 2, 2);
-  else if (cin == 192 && two)
-    CONV(192, 2, 2, 1, 2);
-  else if (cin == 256 && two)
-    CONV_LARGE(256);
-  else if (cin == 384 && two)
-    CONV_LARGE(384);
-  else
-    done = false;
+  // 32 and 64 channels; the wide single-row tile where the results are not a multiple of 64
+  auto small = [&](auto c) {
+    constexpr int CIN = decltype(c)::value;
+    if (two && waves(2, 4) >= 2048) {
+      CONV(CIN, 1, 4, 2, 4);
+      return;
+    }
+    if constexpr (CIN == 32 || !FWD)
+      if (!two && waves(1, 4) >= 2048) {
+        CONV(CIN, 1, 4, 1, 4);
+        return;
+      }
+    if (two && waves(2, 2) >= 1024)
+      CONV(CIN, 1, 4, 2, 2);
+    else
+      CONV(CIN, 1, 4, 1, 2);
+  };
+  if (done) {
+    if (cin == 32)
+      small(std::integral_constant<int, 32>());
+    else if (cin == 64)
+      small(std::integral_constant<int, 64>());
+    else if (cin == 128)
+      CONV_LARGE(128);
+    else if (cin == 256)
+      CONV_LARGE(256);
+    else
+      done = false;
+    if constexpr (FWD) {
+      if (!done) {
+        done = true;
+        if (cin == 16 && waves(1, 4) >= 1024)
+          CONV(16, 1, 4, 1, 4);
+        else if (cin == 16)
+          CONV(16, 1, 4, 1, 2);
+        else if (cin == 96 && waves(1, 4) >= 1024)
+          CONV(96, 1, 2, 1, 4);
+        else if (cin == 96)
+          CONV(96, 1, 4, 1, 2);
+        else if (cin == 192 && waves(2, 2) >= 1024)
+          CONV(192, 1, 2, 2, 2);
+        else if (cin == 192)
+          CONV(192, 2, 2, 1, 2);
+        else if (cin == 384)
+          CONV_LARGE(384);
+        else
+          done = false;
+      }
+    }
+  }
 #undef CONV
-#undef CONV_SMALL
 #undef CONV_LARGE
   if (!done) {  // the input tile does not fit LDS
+    if (!two || cin % 64 != 0) return ufail(MSG_ERR_ARG, "a convolution between channel counts that no network has");
     const int np = (W % 64 == 0) ? 2 : 1;
-    const dim3 grid(cdivu((long)u->B * H * W, 128 * np), cout / (two ? 64 : 32));
-    if (two && np == 2)
-      hipLaunchKernelGGL((k_conv3x3<2, 2, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
-    else if (two)
-      hipLaunchKernelGGL((k_conv3x3<2, 1, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
-    else if (np == 2)
-      hipLaunchKernelGGL((k_conv3x3<1, 2, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
+    const dim3 grid(cdivu((long)u->B * H * W, 128 * np), cout / 64);
+    if (np == 2)
+      hipLaunchKernelGGL((k_conv3x3<2, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
     else
-      hipLaunchKernelGGL((k_conv3x3<1, 1, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
+      hipLaunchKernelGGL((k_conv3x3<1, OutT>), grid, dim3(256), 0, u->s, in, w, bias, y, u->B, H, W, cout, relu);
   }
   UHIP(hipGetLastError());
   return MSG_OK;
@@ -1164,8 +1180,6 @@ int backward(msg_unet *u, const float *target, double *loss) {
       hipLaunchKernelGGL((k_conv3x3_wgrad<2, 2, 8>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
     else if (wg.wm == 2)
       hipLaunchKernelGGL((k_conv3x3_wgrad<2, 1, 8>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
-    else if (wg.wn == 2)
-      hipLaunchKernelGGL((k_conv3x3_wgrad<1, 2, 8>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
     else
       hipLaunchKernelGGL((k_conv3x3_wgrad<1, 1, 16>), gw, dim3(256), 0, u->s, in, zp, pt, B, Hs, Ws, c.cout, wg.nsplit);
     UHIP(hipGetLastError());
