@@ -93,7 +93,7 @@ struct ConvIn {
   int c1, c2, up1;
 };
 
-// 16 bytes per lane from global memory straight to LDS, no registers in between: lane l's to dst + 16 l
+// 16 bytes per lane from global memory straight to LDS, no registers in between: lane l's to dst + 16 l, dst aligned
 // (dst is the same for the whole wave; inactive lanes write nothing). Complete after lds_loads_done.
 __device__ __forceinline__ void load_to_lds(const bf16 *src, bf16 *dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
@@ -207,7 +207,7 @@ k_conv3x3_tile(ConvIn in, const bf16 *__restrict__ w, const float *__restrict__ 
   constexpr bool ALDS = CIN <= 32;
   constexpr int PERM = SEG % 16 == 0 ? 15 : SEG % 8 == 0 ? 7 : SEG % 4 == 0 ? 3 : 1;  // slot bits permuted
   constexpr int G = NKS <= 4 || NKS == 6 ? NKS : 4, NG = 9 * NKS / G;  // steps per group, groups
-  __shared__ bf16 sx[NLD * 8 + (ALDS ? WM * NT * WF : 2 * TH)];  // pixels; weights or what touching them returns
+  __shared__ alignas(16) bf16 sx[NLD * 8 + (ALDS ? WM * NT * WF : 2 * TH)];  // pixels; weights or what touching them returns
   bf16 *sw = sx + NLD * 8;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave % WM, wr = wave / WM;
   const int wave0 = __builtin_amdgcn_readfirstlane(wave * 64);
@@ -433,7 +433,7 @@ k_conv3x3_wgrad(ConvIn in, const bf16 *__restrict__ dz, float *__restrict__ part
                 int nsplit) {
   constexpr int KS = 4 / (WM * WN), RW = R / KS, HC = 34;
   constexpr int ZPIX = R * 32, XPIX = (R + 2) * HC;
-  __shared__ bf16 lds[(ZPIX * WM + XPIX * WN) * 32];
+  __shared__ alignas(16) bf16 lds[(ZPIX * WM + XPIX * WN) * 32];
   static_assert(sizeof(lds) >= 3 * 16 * 64 * sizeof(float), "the final sum over the row shares reuses the tile");
   bf16 *sz = lds, *sx = lds + ZPIX * WM * 32;
   const int cin = in.c1 + in.c2;
