@@ -358,8 +358,9 @@ int msg_match_series_batch(int dtype, int njobs, const msg_series_job *jobs);
  * level `level`; phi: device output field. energy/iterations: host outputs (may be NULL). */
 int msg_reduce_deformations(int dtype, const void *deformations, int n, int level, int max_iter, double stop_eps,
                             void *phi, double *energy, int *iterations);
-/* msg_match_series keeps its device contexts for reuse by later calls of the same shape (no
- * counterpart in the reference); this frees them. */
+/* msg_match_series keeps its device contexts for reuse by later calls of the same shape, msg_energy and
+ * msg_xshift_energy keep a few blocks of pinned memory for their results (no counterpart in the
+ * reference); this frees them. */
 int msg_release_cache(void);
 
 /* ------------------------------------------------------------------------------------------------

@@ -122,29 +122,65 @@ int flag_snap(FlagSnap **out) {
   return MSG_OK;
 }
 
-// Pinned host memory of a thread and device for small results that a kernel writes itself (grown, kept):
-// the caller reads them after the stream is synchronised, with no copy launched.
-struct PinnedBuf {
-  void *p = nullptr;
-  size_t n = 0;
+// Pinned host memory for small results that a kernel writes itself: the caller reads them after the stream is
+// synchronised, with no copy launched. A call borrows a block and gives it back, whatever thread it runs on; at most
+// KEEP unused blocks stay (msg_release_cache frees them).
+struct PinnedPool {
+  struct Block {
+    void *p;
+    size_t n;
+    int dev;
+  };
+  static constexpr size_t KEEP = 16;
+  std::mutex mu;
+  std::vector<Block> free;
+  PinnedPool() { free.reserve(KEEP); }
+  void release() {
+    std::lock_guard<std::mutex> g(mu);
+    for (auto &b : free) (void)hipHostFree(b.p);
+    free.clear();
+  }
 };
-thread_local PinnedBuf g_pinned[16];
-
-int pinned_get(size_t bytes, void **p) {
-  int dev = 0;
-  HIPCHK(hipGetDevice(&dev));
-  PinnedBuf &b = g_pinned[dev & 15];
-  if (b.n < bytes) {
-    if (b.p) HIPCHK(hipHostFree(b.p));
-    b.p = nullptr;
-    b.n = 0;
+PinnedPool &pinned_pool() {
+  static PinnedPool *p = new PinnedPool();  // never destroyed: the runtime may be gone by then
+  return *p;
+}
+struct PinnedBuf {
+  PinnedPool::Block b{nullptr, 0, 0};
+  int get(size_t bytes) {
+    HIPCHK(hipGetDevice(&b.dev));
+    PinnedPool &pool = pinned_pool();
+    {
+      std::lock_guard<std::mutex> g(pool.mu);
+      for (size_t k = pool.free.size(); k-- > 0;)
+        if (pool.free[k].dev == b.dev && pool.free[k].n >= bytes) {
+          b = pool.free[k];
+          pool.free[k] = pool.free.back();
+          pool.free.pop_back();
+          return MSG_OK;
+        }
+    }
     bytes = std::max<size_t>(bytes, 4096);
     HIPCHK(hipHostMalloc(&b.p, bytes, hipHostMallocDefault));
     b.n = bytes;
+    return MSG_OK;
   }
-  *p = b.p;
-  return MSG_OK;
-}
+  ~PinnedBuf() {
+    if (!b.p) return;
+    PinnedPool &pool = pinned_pool();
+    {
+      std::lock_guard<std::mutex> g(pool.mu);
+      if (pool.free.size() < PinnedPool::KEEP) {
+        pool.free.push_back(b);
+        return;
+      }
+      auto least = std::min_element(pool.free.begin(), pool.free.end(),
+                                    [](const PinnedPool::Block &x, const PinnedPool::Block &y) { return x.n < y.n; });
+      if (least->n < b.n) std::swap(*least, b);
+    }
+    (void)hipHostFree(b.p);
+  }
+};
 
 // ------------------------------------------------------------------------------------------------
 // Kernel timing with HIP events on the stream each kernel is launched on (opt-in, per class mask).
@@ -1470,16 +1506,16 @@ int energy_impl(const void *R, const void *T, const void *phi, int n, int batch,
   CHK(launch_energy<S>((const S *)R, (const S *)T, (const S *)phi, (const S *)phi, (const S *)phi, n,
                        (const PairState *)stp, (double *)part, batch, s, data_term, 0, 0, false, yreg));
   // x-shift: the rows' NCC energies averaged over the rows (FELineShiftRegisEnergy::apply)
-  void *sums = nullptr;
-  CHK(pinned_get(sizeof(double) * 2 * batch, &sums));
+  PinnedBuf pinned;
+  CHK(pinned.get(sizeof(double) * 2 * batch));
+  double *sums = (double *)pinned.b.p;
   hipLaunchKernelGGL(k_energy_sums, dim3(2 * batch), dim3(256), 0, s, (const double *)part, nb, batch,
-                     data_term == msg::DT_XSHIFT ? 1.0 / n : 1.0, (double *)sums);
+                     data_term == msg::DT_XSHIFT ? 1.0 / n : 1.0, sums);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
-  const double *h = (const double *)sums;
   for (int p = 0; p < batch; ++p) {
-    if (e_data) e_data[p] = h[p];
-    if (e_reg) e_reg[p] = h[batch + p];
+    if (e_data) e_data[p] = sums[p];
+    if (e_reg) e_reg[p] = sums[batch + p];
   }
   return MSG_OK;
 }
@@ -2897,6 +2933,7 @@ int msg_profile_read(int cls, double *ms, long long *launches, double *bytes) {
 extern "C" {
 
 int msg_release_cache(void) {
+  pinned_pool().release();
   std::lock_guard<std::mutex> g(g_ctx_cache.mu);
   for (msg_ctx *c : g_ctx_cache.free) msg_ctx_destroy(c);
   g_ctx_cache.free.clear();

@@ -340,6 +340,37 @@ def test_f64_coarse_workgroups(gpu, n):
         assert np.array_equal(e, out[0][0][a:b]) and torch.equal(f, out[0][1][a:b])
 
 
+def test_energies_from_many_threads(gpu):
+    """The energies' results pass through pinned blocks that calls borrow and give back: threads that come and go,
+    with batches of different sizes and the blocks freed in between, get what one thread gets."""
+    import threading
+    g = torch.Generator(device="cuda").manual_seed(3)
+    work = []
+    for k, (n, pairs) in enumerate(((16, 1), (8, 700), (32, 3), (64, 2), (4, 3000), (128, 1))):
+        R, T = (torch.rand(pairs, n, n, device="cuda", generator=g) for _ in range(2))
+        phi = torch.randn(pairs, 2, n, n, device="cuda", generator=g) * (1.0 / n)
+        work.append((R, T, phi, gpu.energy(R, T, phi)))
+    torch.cuda.synchronize()
+    wrong = []
+
+    def run(k):
+        for r in range(10):
+            R, T, phi, want = work[(k + r) % len(work)]
+            got = gpu.energy(R, T, phi)
+            if not all(np.array_equal(a, b) for a, b in zip(got, want)):
+                wrong.append((k, r))
+            if k == 0 and r == 5:
+                gpu.release_cache()
+
+    for _ in range(2):
+        threads = [threading.Thread(target=run, args=(k,)) for k in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert not wrong
+
+
 def shortest(fn, calls=25):
     """The shortest of some calls, in seconds (every entry point waits for its result)."""
     import time
