@@ -627,17 +627,16 @@ int launch_prolong(const S *coarse, S *fine, int nc, int nfields, hipStream_t s)
 }
 
 // Warps of nimg n x n images (n a power of two); see k_warp.
-template <typename S, int RUN>
+template <typename S, int RUN, bool NEAR>
 int launch_warp_run(const S *img, const S *phi, S *out, int n, int nimg, int phi_shared, int mode, double ext,
-                    int nearest, hipStream_t s) {
+                    hipStream_t s) {
   const int nblk = cdiv(n * n, 256 * RUN);
   const size_t nn = (size_t)n * n;
   const int per = std::max(1, (1 << 23) / nblk);  // images a launch: a grid of at most 2^31 threads
   for (int i = 0; i < nimg; i += per) {
     const int m = std::min(per, nimg - i);
-    hipLaunchKernelGGL((msg::k_warp<S, RUN>), dim3((unsigned)nblk * m), dim3(256), 0, s, img + i * nn,
-                       phi + (phi_shared ? 0 : i * 2 * nn), out + i * nn, n, log2i(n), nblk, phi_shared, mode, ext,
-                       nearest);
+    hipLaunchKernelGGL((msg::k_warp<S, RUN, NEAR>), dim3((unsigned)nblk * m), dim3(256), 0, s, img + i * nn,
+                       phi + (phi_shared ? 0 : i * 2 * nn), out + i * nn, n, log2i(n), nblk, phi_shared, mode, ext);
     HIPCHK(hipGetLastError());
   }
   return MSG_OK;
@@ -645,9 +644,16 @@ int launch_warp_run(const S *img, const S *phi, S *out, int n, int nimg, int phi
 template <typename S>
 int launch_warp(const S *img, const S *phi, S *out, int n, int nimg, int phi_shared, int mode, double ext, int nearest,
                 hipStream_t s) {
-  if ((long)n * n * nimg >= msg::WARP_RUN_PIXELS)
-    return launch_warp_run<S, msg::WARP_RUN>(img, phi, out, n, nimg, phi_shared, mode, ext, nearest, s);
-  return launch_warp_run<S, 1>(img, phi, out, n, nimg, phi_shared, mode, ext, nearest, s);
+  const bool run = (long)n * n * nimg >= msg::WARP_RUN_PIXELS;
+  const auto launch = [&](auto r, auto near) {
+    return launch_warp_run<S, decltype(r)::value, decltype(near)::value>(img, phi, out, n, nimg, phi_shared, mode, ext, s);
+  };
+  using std::integral_constant;
+  if (nearest && mode == 0)
+    return run ? launch(integral_constant<int, msg::WARP_RUN>(), std::true_type())
+               : launch(integral_constant<int, 1>(), std::true_type());
+  return run ? launch(integral_constant<int, msg::WARP_RUN>(), std::false_type())
+             : launch(integral_constant<int, 1>(), std::false_type());
 }
 
 // Sampling positions k * (nc-1)/(n-1) of ResampleCopier (scalarArray.h:311-330): the step divided in

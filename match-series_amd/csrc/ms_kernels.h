@@ -1691,14 +1691,16 @@ __global__ void k_resample_rect(const S *__restrict__ src, int w, int h, S *__re
 // and 229 us. RUN = 4 pixels in a row, 256 apart, instead: 135 us, but 205 us where noisy (FP64 206 and 378 us), four
 // rows' neighbours at once being more than a compute unit's L1 holds. Few pixels have nothing to overlap:
 // 128^2 20.7 us with RUN = 1, 21.7 with 4; from WARP_RUN_PIXELS (512 workgroups of 4) on the latter is no slower:
-// 512^2 x 2 22.8 and 23.1 us, in FP64 up to 25.6 and 23.2.
+// 512^2 x 2 22.8 and 23.1 us, in FP64 up to 25.6 and 23.2. Positions rounded to nodes (NEAR) lie on one row, but on
+// the grid's last, and read that one alone (4 x 2048^2 in FP64, half the positions outside: 150 us with both rows, 132 so).
 constexpr int WARP_RUN = 4;
 constexpr long WARP_RUN_PIXELS = 1l << 19;
 
-template <typename S, int RUN>
+// NEAR: positions rounded to nodes (mode 0 only).
+template <typename S, int RUN, bool NEAR>
 __global__ void __launch_bounds__(256)
 k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out, int n, int logn, int nblk,
-       int phi_shared, int mode, double ext, int nearest) {
+       int phi_shared, int mode, double ext) {
   const int f = blockIdx.x / nblk, tile = blockIdx.x - f * nblk;
   const int cnt = n * n;
   const int logw = logn < 8 ? logn : 8;  // a tile's columns; its 256 RUN >> logw rows
@@ -1729,7 +1731,7 @@ k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out
     } else {
       if (dx < 0.0 || dx > hi || (mode == 0 && isnan(dx))) inside[k] = false;
       if (dy < 0.0 || dy > hi || (mode == 0 && isnan(dy))) inside[k] = false;
-      if (nearest && mode == 0) {
+      if (NEAR) {
         dx = floor(dx + 0.5);
         dy = floor(dy + 0.5);
       }
@@ -1740,8 +1742,12 @@ k_warp(const S *__restrict__ img, const S *__restrict__ phi, S *__restrict__ out
     const S *c = im + xL + (size_t)yL * n;
     v[k][0] = c[0];
     v[k][1] = c[1];
-    v[k][2] = c[n];
-    v[k][3] = c[n + 1];
+    if (!NEAR || Y[k] != 0) {
+      v[k][2] = c[n];
+      v[k][3] = c[n + 1];
+    } else {
+      v[k][2] = v[k][3] = 0;
+    }
   }
 #pragma unroll
   for (int k = 0; k < RUN; ++k) {
