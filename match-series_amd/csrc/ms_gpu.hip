@@ -2016,9 +2016,11 @@ int normalize_impl(void *img, int n, int nimg, double pct, int min_to_zero, hipS
     i1 = std::min(std::max(i1, 0), m1);
   }
   if (nn <= NORM_ONE) {
-    hipLaunchKernelGGL((msg::k_normalize_one<S>), dim3(nimg), dim3(msg::SEL1_THREADS), 0, s, (S *)img, nn, (unsigned)i0,
-                       (unsigned)i1, pct >= 0 ? 1 : 0, min_to_zero);
-    HIPCHK(hipGetLastError());
+    for (long k = 0; k < nimg; k += 1 << 20) {  // a grid of at most 2^30 threads
+      hipLaunchKernelGGL((msg::k_normalize_one<S>), dim3((unsigned)std::min(nimg - k, 1l << 20)), dim3(msg::SEL1_THREADS), 0, s,
+                         (S *)img + (size_t)k * nn, nn, (unsigned)i0, (unsigned)i1, pct >= 0 ? 1 : 0, min_to_zero);
+      HIPCHK(hipGetLastError());
+    }
     return MSG_OK;
   }
   if (nn <= NORM_SHORT && (long)nn * nimg <= NORM_SHORT_ALL)

@@ -60,6 +60,15 @@ def test_normalize_ranks(gpu, n, frames, code):
             assert np.array_equal(out[k], want, equal_nan=True), (k, pct, zero)
 
 
+def test_normalize_many_small_images(gpu):
+    """More images than one launch takes (2^20 workgroups): the ends of the launches and of the whole are what
+    they are alone."""
+    img = torch.randn((1 << 22) + 3, 2, 2, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    out = gpu.normalize(img.clone(), 0.15)
+    for k in (0, (1 << 20) - 1, 1 << 20, 1 << 21, (1 << 22) - 1, 1 << 22, (1 << 22) + 2):
+        assert torch.equal(out[k:k + 1], gpu.normalize(img[k:k + 1].clone(), 0.15))
+
+
 @pytest.mark.parametrize("frames", [1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 31, 32, 33, 63, 64, 65])
 @pytest.mark.parametrize("code", [0, 1])
 def test_series_stats_networks(gpu, frames, code):
