@@ -461,8 +461,9 @@ __device__ __forceinline__ float add_rounded(float a, float b) {
 // column to its left come by a lane shift and those from the row below stay in registers, so there is no LDS and no
 // barrier, node rows are loaded once per element row instead of twice, and of the elements only 1/64 (columns) and
 // 1/RUN (rows) are worked on twice, where the 32 x 8 tiles take 5 passes of a wave for 4 waves of nodes. Same values
-// as k_grad_f32's, bit for bit (a sum of zeros alone may differ in the zero's sign). Bound by vector arithmetic (312 instructions per element, the tile kernel 417
-// before its clip and offsets took FP32 forms): 8 pairs of 1024^2, 106 us -> 102 us in tiles and 83 us here.
+// as k_grad_f32's, bit for bit (a sum of zeros alone may differ in the zero's sign). Bound by vector arithmetic (312
+// instructions per element, the tile kernel 417 before its clip and offsets took FP32 forms): 8 pairs of 1024^2,
+// 106 us -> 102 us in tiles and 83 us here.
 // A run of 7 beat 4 and 5 (87, 86 us: more rows done twice) and 8 (87 us; 16: 100 us, too few waves at the end).
 // A wave's run is a chain of 8 elements at 1.6 us each, so small launches are faster in tiles: 512^2 6.9 us (runs
 // 12.0), 1024^2 16.4 (18.5), 2 x 1024^2 27.7 (25.1), 4 x 1024^2 49.3 (42.9): runs from 2^21 nodes on. And a run's 63

@@ -1687,8 +1687,8 @@ __global__ void k_resample_rect(const S *__restrict__ src, int w, int h, S *__re
 // together, displacements, then the 4 neighbours each, so a wave waits for two memory round trips in RUN pixels
 // and neighbouring rows meet in its cache lines. Pixels outside gather from clamped nodes and are replaced by a
 // select (no branches). 31 frames of 1024^2 in FP32, whole calls: 200 us with one pixel per thread and 64-bit index
-// divisions; 132 us so (the kernel 118 us, 4.4 TB/s), where the field is noisy (1.5 pixels) 205 and 137 us; FP64 226 and 197, noisy 261
-// and 229 us. RUN = 4 pixels in a row, 256 apart, instead: 135 us, but 205 us where noisy (FP64 206 and 378 us), four
+// divisions; 132 us so (the kernel 118 us, 4.4 TB/s), where the field is noisy (1.5 pixels) 205 and 137 us; FP64
+// 226 and 197, noisy 261 and 229 us. RUN = 4 pixels in a row, 256 apart, instead: 135 us, but 205 us where noisy (FP64 206 and 378 us), four
 // rows' neighbours at once being more than a compute unit's L1 holds. Few pixels have nothing to overlap:
 // 128^2 20.7 us with RUN = 1, 21.7 with 4; from WARP_RUN_PIXELS (512 workgroups of 4) on the latter is no slower:
 // 512^2 x 2 22.8 and 23.1 us, in FP64 up to 25.6 and 23.2. Positions rounded to nodes (NEAR) lie on one row, but on
